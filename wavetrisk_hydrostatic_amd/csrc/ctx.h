@@ -57,7 +57,9 @@ struct wtg_ctx {
   // member 1 once that member's cycles have converged (device [nmembers])
   const double* mg_mdone = nullptr;
   bool split_fused = true;  // FP64 split-explicit stages: trend and AXPY in one launch
-  int stage_version = 3;  // WTG_STAGE_KERNEL: 1 = tile loop, 2 = one thread per region cell, 3 = layer pairs
+  double* d_fix = nullptr;      // stage kernel's pentagon values [member][lozenge][corner][layer][2]
+  double* d_csum[2] = {};       // column sums of mass - temp of two stage states [member][cell]
+  int stage_version = 3;  // WTG_STAGE_KERNEL: 1 = tile loop, 2 = one thread per region cell, 3 = tile blocks
   bool topo_set = false;
   std::string err;
   // device geometry
@@ -203,7 +205,7 @@ struct WtgStageKeep {
   double* src;         // [L][3][NC] velocity source (-Qperp) on owned edges
   double *dm, *dt;     // [L][NC] scalar trends on owned cells and the pole masters
 };
-// one RK stage (or trend, trend_only = 1) of the FP64 layer-pair kernel
+// one RK stage (or trend, trend_only = 1) of the FP64 tile kernel
 // with optional kept quantities
 int wtg_launch_stage_keep(wtg_ctx* c, const wtg_ctx::Slot& y, const wtg_ctx::Slot& q, const wtg_ctx::Slot& out,
                           double h, int trend_only, const WtgStageKeep* keep);

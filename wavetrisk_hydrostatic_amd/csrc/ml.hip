@@ -9,7 +9,7 @@
 //   RK4                                             time_integr.f90:78-103
 //
 // One context per level (coarse to fine) holds the level's state slots.
-// The finest level's trend is the layer-pair stage kernel, which also keeps
+// The finest level's trend is the tile stage kernel, which also keeps
 // the fluxes, Bernoulli and Exner functions, velocity source and scalar
 // trends that the coarser levels restrict; on a full hierarchy every coarse
 // value is a restriction (sub-sampled Bernoulli and Exner functions,
@@ -1000,7 +1000,7 @@ int wtg_ml_create(const wtg_grid* const* grids, wtg_ctx* const* levels, int nlev
       if (levels[k] == c) return wtg_fail(nullptr, WTG_E_ARG, "level %d repeats a context", l);
   }
   if (nlevels > 1 && levels[nlevels - 1]->stage_version != 3)
-    return wtg_fail(nullptr, WTG_E_ARG, "the finest level must use the layer-pair stage kernel");
+    return wtg_fail(nullptr, WTG_E_ARG, "the finest level must use the default stage kernel");
   auto m = std::make_unique<wtg_ml>();
   m->nl = nlevels;
   m->L = levels[0]->params.nlayers;

@@ -64,8 +64,12 @@ struct StageArgs {
   int trend_only;              // 1: out = trend
   Geo g;
   double grav, rho0, p_top;
+  int kchunk;  // layers per block (tile kernel)
+  const double* csum_in;  // column sum of ym - yt (null: taken here)
+  double* csum_out;       // the same of the new state (null: not kept)
+  double* fix;            // pentagon values [member][lozenge][corner][layer][2]
   // optional copies of the intermediate quantities that the coarser levels
-  // of a hierarchy restrict (null: not kept); FP64 pair kernel only
+  // of a hierarchy restrict (null: not kept); FP64 tile kernel only
   double *k_hm, *k_ht;     // [L][3][NC] mass / temperature fluxes, region cells [-1, n]^2
   double *k_bern, *k_exn;  // [L][NC] Bernoulli, Exner on [0, n]^2
   double *k_src;           // [L][3][NC] velocity source (-Qperp) on owned edges
@@ -74,7 +78,7 @@ struct StageArgs {
   // velocity update adds theta1 g grad eta to the trend (eta [NC], per member)
   const double* eta;
   double th1;
-  // diffusion hooks (pair kernel, DIFF): scalar diffusive fluxes on the edges
+  // diffusion hooks (tile kernel, DIFF): scalar diffusive fluxes on the edges
   // of the region cells and velocity source on the owned edges, [L][3][NC]
   // (null: that hook is off)
   const double *phm, *pht, *phu;
@@ -94,6 +98,8 @@ __device__ __forceinline__ StageArgs member_args(const StageArgs& a0) {
   if (a.eta) a.eta += (int64_t)blockIdx.y * a0.NC;
   if (a.phm) a.phm += s3, a.pht += s3;
   if (a.phu) a.phu += s3;
+  if (a.csum_in) a.csum_in += (int64_t)blockIdx.y * a0.NC;
+  if (a.csum_out) a.csum_out += (int64_t)blockIdx.y * a0.NC;
   return a;
 }
 
@@ -402,38 +408,34 @@ __global__ __launch_bounds__(THREADS) void trisk_stage_kernel(StageArgs a_in) {
 // triangles next to the pentagon is recomputed with the pentagon's
 // circulation and mass, and two qe values per corner are overwritten.
 // `which` = 0..3 for the SW, SE, NW, NE corner; region cell (1,1), (T+1,1),
-// (1,T+1), (T+1,T+1).  u*, m, qe* are LDS planes of the 19 x 19 region.
-// The planes are FP64 or FP32 (F); the corrections are evaluated in FP64.
-template <class F>
-__device__ void pentagon_fixup(int which, const F* __restrict__ u0p, const F* __restrict__ u1p,
-                               const F* __restrict__ u2p, const F* __restrict__ mp, F* qe0, F* qe1, F* qe2,
-                               const Geo& g, int64_t NC, int64_t base, int S) {
-  auto r = [](int ri, int rj) { return rj * R + ri; };
+// (1,T+1), (T+1,T+1).  U(e, i, j) and M(i, j) give the region's velocities
+// and masses; out = the corner's two values of qe.
+template <class UF, class MF>
+__device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF& M, const Geo& g, int64_t NC,
+                                                int64_t base, int S, double out[2]) {
   auto gcell = [&](int ri, int rj) -> int64_t { return base + (int64_t)rj * S + ri; };
-  const F* up[3] = {u0p, u1p, u2p};
-  auto UPL = [&](int e, int i, int j) { return (double)up[e][r(i, j)] * g.len[(int64_t)e * NC + gcell(i, j)]; };
-  auto M = [&](int i, int j) { return (double)mp[r(i, j)]; };
+  auto P = [&](int e, int i, int j) { return U(e, i, j) * g.len[(int64_t)e * NC + gcell(i, j)]; };
   auto AR = [&](int p, int i, int j) { return g.area[(int64_t)(p - 1) * NC + gcell(i, j)]; };
   auto TRI = [&](int tt, int i, int j) { return g.tri[(int64_t)tt * NC + gcell(i, j)]; };
   auto COR = [&](int tt, int i, int j) { return g.cor[(int64_t)tt * NC + gcell(i, j)]; };
   if (which == 0) {  // IJMINUS
     const int i = 1, j = 1;
-    double cSW_L = UPL(2, i, j - 1) - UPL(0, i - 1, j) + UPL(0, i - 1, j - 1);
-    double cW_L = ((UPL(0, i - 1, j) + UPL(2, i, j) + UPL(1, i - 1, j)) / TRI(0, i - 1, j)) * TRI(0, i - 1, j);
-    double cS_U = (-(UPL(0, i, j) + UPL(1, i, j - 1) + UPL(2, i, j - 1)) / TRI(1, i, j - 1)) * TRI(1, i, j - 1);
+    double cSW_L = P(2, i, j - 1) - P(0, i - 1, j) + P(0, i - 1, j - 1);
+    double cW_L = ((P(0, i - 1, j) + P(2, i, j) + P(1, i - 1, j)) / TRI(0, i - 1, j)) * TRI(0, i - 1, j);
+    double cS_U = (-(P(0, i, j) + P(1, i, j - 1) + P(2, i, j - 1)) / TRI(1, i, j - 1)) * TRI(1, i, j - 1);
     double m1 = M(i - 1, j) * AR(6, i - 1, j) + M(i, j) * (AR(4, i, j) + AR(5, i, j)) + M(i, j - 1) * AR(3, i, j - 1);
     double m2 = M(i - 1, j) * AR(1, i - 1, j) + M(i, j) * AR(3, i, j) + M(i, j + 1) * AR(5, i, j + 1);
     double m3 = M(i, j - 1) * AR(2, i, j - 1) + M(i + 1, j) * AR(4, i + 1, j) + M(i, j) * AR(6, i, j);
     double pvWL = (COR(0, i - 1, j) + cW_L) / m1;
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m2;
     double pvSU = (COR(1, i, j - 1) + cS_U) / m3;
-    qe0[r(i - 1, j)] = (F)interp(pvWL, pvSWL);
-    qe2[r(i, j - 1)] = (F)interp(pvSU, pvSWL);
+    out[0] = interp(pvWL, pvSWL);
+    out[1] = interp(pvSU, pvSWL);
   } else if (which == 1) {  // IPLUSJMINUS
     const int i = T + 1, j = 1;
-    double cSW_L = -UPL(0, i, j) + UPL(0, i - 1, j - 1) + UPL(1, i - 1, j - 1);
-    double cL = ((UPL(0, i, j) + UPL(2, i + 1, j) + UPL(1, i, j)) / TRI(0, i, j)) * TRI(0, i, j);
-    double cSW_U = (-(UPL(0, i - 1, j) + UPL(1, i - 1, j - 1) + UPL(2, i - 1, j - 1)) / TRI(1, i - 1, j - 1)) *
+    double cSW_L = -P(0, i, j) + P(0, i - 1, j - 1) + P(1, i - 1, j - 1);
+    double cL = ((P(0, i, j) + P(2, i + 1, j) + P(1, i, j)) / TRI(0, i, j)) * TRI(0, i, j);
+    double cSW_U = (-(P(0, i - 1, j) + P(1, i - 1, j - 1) + P(2, i - 1, j - 1)) / TRI(1, i - 1, j - 1)) *
                    TRI(1, i - 1, j - 1);
     double m1 =
         M(i - 1, j - 1) * AR(1, i - 1, j - 1) + M(i, j - 1) * AR(3, i, j - 1) + M(i, j) * (AR(5, i, j) + AR(6, i, j));
@@ -442,13 +444,13 @@ __device__ void pentagon_fixup(int which, const F* __restrict__ u0p, const F* __
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m1;
     double pvL = (COR(0, i, j) + cL) / m2;
     double pvSWU = (COR(1, i - 1, j - 1) + cSW_U) / m3;
-    qe0[r(i, j)] = (F)interp(pvSWL, pvL);
-    qe1[r(i - 1, j - 1)] = (F)interp(pvSWL, pvSWU);
+    out[0] = interp(pvSWL, pvL);
+    out[1] = interp(pvSWL, pvSWU);
   } else if (which == 2) {  // IMINUSJPLUS
     const int i = 1, j = T + 1;
-    double cSW_U = UPL(2, i, j) - UPL(1, i - 1, j - 1) - UPL(2, i - 1, j - 1);
-    double cU = (-(UPL(1, i, j) + UPL(2, i, j) + UPL(0, i, j + 1)) / TRI(1, i, j)) * TRI(1, i, j);
-    double cSW_L = ((UPL(0, i - 1, j - 1) + UPL(2, i, j - 1) + UPL(1, i - 1, j - 1)) / TRI(0, i - 1, j - 1)) *
+    double cSW_U = P(2, i, j) - P(1, i - 1, j - 1) - P(2, i - 1, j - 1);
+    double cU = (-(P(1, i, j) + P(2, i, j) + P(0, i, j + 1)) / TRI(1, i, j)) * TRI(1, i, j);
+    double cSW_L = ((P(0, i - 1, j - 1) + P(2, i, j - 1) + P(1, i - 1, j - 1)) / TRI(0, i - 1, j - 1)) *
                    TRI(0, i - 1, j - 1);
     double m1 =
         M(i - 1, j - 1) * AR(2, i - 1, j - 1) + M(i, j) * (AR(3, i, j) + AR(4, i, j)) + M(i - 1, j) * AR(6, i - 1, j);
@@ -457,22 +459,38 @@ __device__ void pentagon_fixup(int which, const F* __restrict__ u0p, const F* __
     double pvSWU = (COR(1, i - 1, j - 1) + cSW_U) / m1;
     double pvU = (COR(1, i, j) + cU) / m2;
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m3;
-    qe2[r(i, j)] = (F)interp(pvSWU, pvU);
-    qe1[r(i - 1, j - 1)] = (F)interp(pvSWL, pvSWU);
+    out[0] = interp(pvSWU, pvU);
+    out[1] = interp(pvSWL, pvSWU);
   } else {  // IJPLUS
     const int i = T + 1, j = T + 1;
-    double cL = UPL(0, i, j) - UPL(0, i, j + 1) - UPL(2, i, j);
-    double cW_L = ((UPL(0, i - 1, j) + UPL(2, i, j) + UPL(1, i - 1, j)) / TRI(0, i - 1, j)) * TRI(0, i - 1, j);
-    double cS_U = (-(UPL(1, i, j - 1) + UPL(2, i, j - 1) + UPL(0, i, j)) / TRI(1, i, j - 1)) * TRI(1, i, j - 1);
+    double cL = P(0, i, j) - P(0, i, j + 1) - P(2, i, j);
+    double cW_L = ((P(0, i - 1, j) + P(2, i, j) + P(1, i - 1, j)) / TRI(0, i - 1, j)) * TRI(0, i - 1, j);
+    double cS_U = (-(P(1, i, j - 1) + P(2, i, j - 1) + P(0, i, j)) / TRI(1, i, j - 1)) * TRI(1, i, j - 1);
     double m1 = M(i + 1, j) * AR(3, i + 1, j) + M(i, j) * (AR(1, i, j) + AR(2, i, j)) + M(i, j + 1) * AR(6, i, j + 1);
     double m2 = M(i - 1, j) * AR(1, i - 1, j) + M(i, j) * AR(3, i, j) + M(i, j + 1) * AR(5, i, j + 1);
     double m3 = M(i, j - 1) * AR(2, i, j - 1) + M(i + 1, j) * AR(4, i + 1, j) + M(i, j) * AR(6, i, j);
     double pvL = (COR(0, i, j) + cL) / m1;
     double pvWL = (COR(0, i - 1, j) + cW_L) / m2;
     double pvSU = (COR(1, i, j - 1) + cS_U) / m3;
-    qe0[r(i, j)] = (F)interp(pvL, pvSU);
-    qe2[r(i, j)] = (F)interp(pvL, pvWL);
+    out[0] = interp(pvL, pvSU);
+    out[1] = interp(pvL, pvWL);
   }
+}
+
+// the same from and to LDS planes of the 19 x 19 region, FP64 or FP32 (F); the
+// corrections are evaluated in FP64
+template <class F>
+__device__ void pentagon_fixup(int which, const F* __restrict__ u0p, const F* __restrict__ u1p,
+                               const F* __restrict__ u2p, const F* __restrict__ mp, F* qe0, F* qe1, F* qe2,
+                               const Geo& g, int64_t NC, int64_t base, int S) {
+  const F* up[3] = {u0p, u1p, u2p};
+  double v[2];
+  pentagon_values(
+      which, [&](int e, int i, int j) { return (double)up[e][j * R + i]; },
+      [&](int i, int j) { return (double)mp[j * R + i]; }, g, NC, base, S, v);
+  const int at[4][2] = {{R, 1}, {R + T + 1, T}, {(T + 1) * R + 1, T * R}, {(T + 1) * R + T + 1, (T + 1) * R + T + 1}};
+  (which == 2 ? qe2 : qe0)[at[which][0]] = (F)v[0];
+  (which == 1 || which == 2 ? qe1 : qe2)[at[which][1]] = (F)v[1];
 }
 
 // Loads and stores at a uniform base pointer plus a 32-bit byte offset, so the
@@ -769,45 +787,242 @@ __global__ __launch_bounds__(THREADS2, 2) void trisk_stage_kernel2(StageArgs a_i
 }
 
 // ---------------------------------------------------------------------------
-// trisk_stage_pair_kernel: two layer groups per block.  768 threads = two
-// groups of 384; group 0 evaluates the even layers, group 1 the odd ones, in
-// lock step, so each barrier serves two layers and a compute unit holds 12
-// waves.  The launch-invariant geometry of the 19 x 19 region is staged once
-// in LDS and shared by both groups; the Qperp weights of the owned cell (its
-// own offsets 0-2 and those of E, NE, N for offsets 3-5) live in registers.
-// Each thread has two roles: region cell lt (lt < 361) for staging, PV,
-// fluxes and Bernoulli, and owned cell lt (lt < 256) for the trends, so only
-// four waves per group run the Qperp / gradient phase.
-// The hydrostatic column scan stays sequential per column: both groups
-// advance the bottom pressure and geopotential through every layer, taking
-// the other group's layer from its LDS planes, with the same operations in
-// the same order as a single sweep.
+// trisk_stage_tile_kernel: one RK stage of a 16 x 16 tile, one layer at a
+// time, in blocks of four waves of which a compute unit holds two (two waves
+// per SIMD with up to 256 registers each; six-wave blocks of 168 registers
+// fit only once, since every block starts on the same SIMD).
+// Thread lt owns tile node lt; the 105 halo cells of the 19 x 19 region are a
+// second cell of the threads of two of the waves.  Between the layers' three
+// barriers
+//   A  publishes the cells' PV, fluxes, edge products and Exner function,
+//   B  forms qe, Bernoulli and t/m from the neighbours' values of A,
+//   C  forms the trends of the owned nodes and stages the next layer (loaded
+//      since A).
+// A block spans the layers [k0, k0 + kchunk): the column scan takes the
+// layers below it first, with a single sweep's operations in the same order.
+// What bounds it at J8 L30: HBM latency and bandwidth together, 2.5 GB a
+// launch at 3.7 TB/s (a large copy reaches 4.7), and the registers: one
+// spilled value in the loop waits for the next layer's loads (677 -> 727 us).
+// Two independent blocks overlap each other's barriers; the earlier kernel
+// (two layers in lock step in one 768-thread block, the geometry in LDS)
+// took 1034 us, and 15.5 -> 13.7 us at J5 L1, 224 -> 156 us at J7 L20.  The
+// column sum of the stage before saves reading mass and temp twice (0.44 GB),
+// the split-explicit form no longer spills (2070 -> 720 us).
 // ---------------------------------------------------------------------------
 constexpr int GROUP = 384;
 constexpr int THREADS3 = 2 * GROUP;
 
-struct GeoS {  // launch-invariant geometry of the staged region
-  double len[3][RR], ped[3][RR], pedf[3][RR], area[6][RR], hinv[RR], cor[2][RR];
-};
-struct LayerS {  // one layer of one group; t holds t/m from phase 3 on
-  double m[RR], t[RR], u[3][RR];
+struct TileS {
+  double area[6][RR], hinv[RR];   // geometry that neighbours read
+  double m[RR], t[RR];            // staged layer
+  double p0[RR], p2[RR];          // u len of the RT and UP edges
   double pvL[RR], pvU[RR];
-  double qe[3][RR], hm[3][RR], ht[3][RR];
-  double bern[RR], exn[RR];
+  double kk[3][RR];               // (u len)(u pedlen)
+  double hm[3][RR], ht[3][RR];
+  double exn[RR], bern[RR], th[RR], qe[3][RR];
 };
+static_assert(2 * sizeof(TileS) <= 160 * 1024, "two blocks per compute unit");
 
-__device__ __forceinline__ void weights_lds(const GeoS& gs, int y, int offs, double w[5]) {
-  double acc0 = gs.area[offs][y];
-  double acc1 = acc0 + gs.area[(1 + offs) % 6][y];
-  double acc2 = acc1 + gs.area[(2 + offs) % 6][y];
-  double acc3 = acc2 + gs.area[(3 + offs) % 6][y];
-  double acc4 = acc3 + gs.area[(4 + offs) % 6][y];
-  double hi = gs.hinv[y];
+__device__ __forceinline__ void weights_lds(const TileS& s, int y, int offs, double w[5]) {
+  double acc0 = s.area[offs][y];
+  double acc1 = acc0 + s.area[(1 + offs) % 6][y];
+  double acc2 = acc1 + s.area[(2 + offs) % 6][y];
+  double acc3 = acc2 + s.area[(3 + offs) % 6][y];
+  double acc4 = acc3 + s.area[(4 + offs) % 6][y];
+  double hi = s.hinv[y];
   w[0] = 0.5 - acc0 * hi;
   w[1] = -(0.5 - acc1 * hi);
   w[2] = 0.5 - acc2 * hi;
   w[3] = -(0.5 - acc3 * hi);
   w[4] = 0.5 - acc4 * hi;
+}
+
+// a / d with r = 1 / d rounded to nearest: one remainder step makes the
+// product the correctly rounded quotient (Markstein, IBM J. Res. Dev. 34,
+// 1990) where nothing over- or underflows; an infinite a gives NaN
+__device__ __forceinline__ double div_by(double a, double d, double r) {
+  const double q = a * r;
+  return __builtin_fma(__builtin_fma(-q, d, a), r, q);
+}
+
+
+// Planes read and written through buffer descriptors: a uniform base, a
+// uniform 32-bit byte offset of the plane and the cell's 32-bit byte offset,
+// so that an address costs no vector register or instruction of its own.
+using Plane = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ Plane plane(const double* p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00027000);
+}
+__device__ __forceinline__ double ldp(Plane p, uint32_t xb, uint32_t off = 0) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(p, xb, off, 0));
+}
+__device__ __forceinline__ void stp(Plane p, uint32_t xb, double v, uint32_t off = 0) {
+  using V = decltype(__builtin_amdgcn_raw_buffer_load_b64(p, xb, off, 0));
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V, v), p, xb, off, 0);
+}
+
+// one region cell of a thread: its geometry, column state and layer values
+struct TileCell {
+  int x;         // region index
+  uint32_t xb;   // byte offset of the cell in a plane
+  double len[3], ped[3], pedf[3], cor[2];
+  double P, G;   // pressure and geopotential at the bottom of the layer
+  double m, t, u[3], nm, nt, nu[3];
+  double phi, pr, pvl, pvu;
+};
+
+__device__ __forceinline__ void tile_geometry(TileCell& c, const StageArgs& a) {
+  const uint32_t pb = (uint32_t)a.NC * 8u;
+  for (int e = 0; e < 3; ++e) {
+    c.len[e] = ldp(plane(a.g.len), c.xb, e * pb);
+    c.ped[e] = ldp(plane(a.g.ped), c.xb, e * pb);
+    c.pedf[e] = ldp(plane(a.g.pedf), c.xb, e * pb);
+  }
+  c.cor[0] = ldp(plane(a.g.cor), c.xb);
+  c.cor[1] = ldp(plane(a.g.cor), c.xb, pb);
+}
+
+// planes of the geometry that neighbours read, of one region cell
+__device__ __forceinline__ void tile_areas(double v[7], const StageArgs& a, uint32_t xb) {
+  for (int p = 0; p < 6; ++p) v[p] = ldp(plane(a.g.area), xb, p * (uint32_t)a.NC * 8u);
+  v[6] = ldp(plane(a.g.hinv), xb);
+}
+
+// column state at the bottom of layer k0 (cal_surf_press, set_surf_geopot)
+// from the column sum of mass - temp and the bottom height
+__device__ __forceinline__ void tile_column(TileCell& c, const StageArgs& a, double sum, double topo, int k0,
+                                            double rho, double rrho) {
+  constexpr int CH = 8;
+  const int64_t NC = a.NC;
+  c.P = a.grav * sum + a.p_top;
+  c.G = a.grav * topo;
+  for (int k = 0; k < k0; k += CH) {
+    double mo[CH], to[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int kk = min(k + j, k0 - 1);
+      mo[j] = ldo(a.ym + kk * NC, c.xb);
+      to[j] = ldo(a.yt + kk * NC, c.xb);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // all loads of the chunk before the first use
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+      if (k + j < k0) {
+        c.P = c.P - a.grav * (mo[j] - to[j]);
+        c.G = c.G + div_by(a.grav * mo[j], rho, rrho);
+      }
+  }
+}
+
+// a layer index that the compiler does not turn into per-thread running
+// pointers (two registers each): addresses stay a uniform base plus an offset
+__device__ __forceinline__ int uniform_layer(int k) {
+  asm volatile("" : "+s"(k));
+  return k;
+}
+
+__device__ __forceinline__ void tile_load(TileCell& c, const StageArgs& a, int k) {
+  const int64_t ks = (int64_t)k * a.NC;
+  const Plane pu = plane(a.yu + 3 * ks);
+  c.nm = ldp(plane(a.ym + ks), c.xb);
+  c.nt = ldp(plane(a.yt + ks), c.xb);
+  for (int e = 0; e < 3; ++e) c.nu[e] = ldp(pu, c.xb, e * (uint32_t)a.NC * 8u);
+}
+
+__device__ __forceinline__ void tile_stage(TileCell& c, TileS& s) {
+  c.m = c.nm;
+  c.t = c.nt;
+  for (int e = 0; e < 3; ++e) c.u[e] = c.nu[e];
+  s.m[c.x] = c.m;
+  s.t[c.x] = c.t;
+  s.p0[c.x] = c.u[0] * c.len[0];
+  s.p2[c.x] = c.u[2] * c.len[2];
+}
+
+// phase A of one cell; dpm, dpt: diffusive fluxes (DIFF)
+template <bool KEEP, bool DIFF>
+__device__ __forceinline__ void tile_fluxes(TileCell& c, TileS& s, const StageArgs& a, int64_t ke3, double rho,
+                                            double rrho, bool tri, const double* dpm, const double* dpt) {
+  const int x = c.x;
+  {
+    const double p_upper = c.P - a.grav * (c.m - c.t);
+    c.pr = interp(c.P, p_upper);
+    const double gpl = c.G;
+    c.G = gpl + div_by(a.grav * c.m, rho, rrho);
+    c.phi = interp(c.G, gpl);
+    c.P = p_upper;
+  }
+  if (!tri) return;
+  const double up0 = c.u[0] * c.len[0], up1 = c.u[1] * c.len[1], up2 = c.u[2] * c.len[2];
+  s.kk[0][x] = up0 * (c.u[0] * c.ped[0]);
+  s.kk[1][x] = up1 * (c.u[1] * c.ped[1]);
+  s.kk[2][x] = up2 * (c.u[2] * c.ped[2]);
+  const int xE = x + 1, xN = x + R, xNE = x + R + 1;
+  const double circL = up0 + s.p2[xE] + up1;
+  const double circU = -(up1 + up2 + s.p0[xN]);
+  const double mE = s.m[xE], mNE = s.m[xNE], mN = s.m[xN];
+  const double massL = c.m * s.area[0][x] + mE * s.area[2][xE] + mNE * s.area[4][xNE];
+  const double massU = c.m * s.area[1][x] + mNE * s.area[3][xNE] + mN * s.area[5][xN];
+  c.pvl = (c.cor[0] + circL) / massL;
+  c.pvu = (c.cor[1] + circU) / massU;
+  s.pvL[x] = c.pvl;
+  s.pvU[x] = c.pvu;
+  const double f0 = c.u[0] * c.pedf[0], f1 = c.u[1] * c.pedf[1], f2 = c.u[2] * c.pedf[2];
+  double hm[3], ht[3];
+  hm[0] = f0 * interp(c.m, mE);
+  hm[1] = f1 * interp(c.m, mNE);
+  hm[2] = f2 * interp(c.m, mN);
+  ht[0] = f0 * interp(c.t, s.t[xE]);
+  ht[1] = f1 * interp(c.t, s.t[xNE]);
+  ht[2] = f2 * interp(c.t, s.t[xN]);
+  for (int e = 0; e < 3; ++e) {
+    if (DIFF) {
+      hm[e] = hm[e] + dpm[e];
+      ht[e] = ht[e] + dpt[e];
+    }
+    s.hm[e][x] = hm[e];
+    s.ht[e][x] = ht[e];
+    if (KEEP) {
+      sto(a.k_hm + ke3 + e * a.NC, c.xb, hm[e]);
+      sto(a.k_ht + ke3 + e * a.NC, c.xb, ht[e]);
+    }
+  }
+  s.exn[x] = -c.phi;
+}
+
+// phase B of one cell's Bernoulli function
+template <bool KEEP>
+__device__ __forceinline__ double tile_bernoulli(const TileCell& c, TileS& s, const StageArgs& a, int64_t ks,
+                                                 double rho, double rrho) {
+  const int x = c.x;
+  const double ke =
+      (s.kk[2][x] + s.kk[1][x] + s.kk[0][x] + s.kk[2][x - R] + s.kk[1][x - R - 1] + s.kk[0][x - 1]) * s.hinv[x] / 4.0;
+  const double bern = ke + c.phi + div_by(c.pr, rho, rrho);
+  s.bern[x] = bern;
+  if (KEEP) {
+    sto(a.k_bern + ks, c.xb, bern);
+    sto(a.k_exn + ks, c.xb, -c.phi);
+  }
+  return bern;
+}
+
+// scalar trends and their update (C); bm, bt: base state; the new mass - temp
+template <bool KEEP>
+__device__ __forceinline__ double tile_scalars(const TileCell& c, const TileS& s, const StageArgs& a, int64_t ks,
+                                             double bm, double bt) {
+  const int x = c.x, xW = x - 1, xS = x - R, xSW = x - R - 1;
+  const double hi = s.hinv[x];
+  const double divm = (s.hm[0][x] - s.hm[0][xW] + s.hm[1][xSW] - s.hm[1][x] + s.hm[2][x] - s.hm[2][xS]) * hi;
+  const double divt = (s.ht[0][x] - s.ht[0][xW] + s.ht[1][xSW] - s.ht[1][x] + s.ht[2][x] - s.ht[2][xS]) * hi;
+  const double dmv = -divm, dtv = -divt;
+  const double vm = a.trend_only ? dmv : bm + a.h * dmv, vt = a.trend_only ? dtv : bt + a.h * dtv;
+  stp(plane(a.om + ks), c.xb, vm);
+  stp(plane(a.ot + ks), c.xb, vt);
+  if (KEEP) {
+    sto(a.k_dm + ks, c.xb, dmv);
+    sto(a.k_dt + ks, c.xb, dtv);
+  }
+  return vm - vt;
 }
 
 // KEEP: also store the stage's fluxes, Bernoulli / Exner functions, velocity
@@ -818,16 +1033,10 @@ __device__ __forceinline__ void weights_lds(const GeoS& gs, int y, int offs, dou
 // and the velocity source.  Separate instantiations, so that the plain step
 // carries none of them.
 template <bool KEEP, bool SPLIT, bool DIFF>
-__global__ __launch_bounds__(THREADS3) void trisk_stage_pair_kernel(StageArgs a_in) {
+__global__ __launch_bounds__(THREADS, 2) void trisk_stage_tile_kernel(StageArgs a_in) {
   const StageArgs a = member_args(a_in);
-  __shared__ GeoS gs;
-  __shared__ union {
-    LayerS ls[2];
-    double flat[2 * sizeof(LayerS) / sizeof(double)];
-  } lsu;
-  const int tid = threadIdx.x;
-  const int grp = __builtin_amdgcn_readfirstlane(tid / GROUP);  // uniform over each wave
-  const int lt = tid % GROUP;
+  __shared__ TileS s;
+  const int lt = threadIdx.x;
   const int64_t NC = a.NC;
   const int S = a.S;
   const Geo& g = a.g;
@@ -841,320 +1050,219 @@ __global__ __launch_bounds__(THREADS3) void trisk_stage_pair_kernel(StageArgs a_
   const int i0 = (rem % a.ntile) * T, j0 = (rem / a.ntile) * T;
   const int64_t base = (int64_t)lz * S * S + (int64_t)(j0 - 1 + H) * S + (i0 - 1 + H);
   auto gcell = [&](int ri, int rj) -> int64_t { return base + (int64_t)rj * S + ri; };
+  const int k0 = blockIdx.z * a.kchunk, k1 = min(k0 + a.kchunk, a.L);
 
   const bool cSW = (i0 == 0 && j0 == 0), cSE = (i0 + T == a.n && j0 == 0);
   const bool cNW = (i0 == 0 && j0 + T == a.n), cNE = (i0 + T == a.n && j0 + T == a.n);
+
+  // the owned node and, in two of the waves, a halo cell: first those with a
+  // triangle (68: the rows and columns at 0 and T + 1), then the rim at T + 2.
+  // The two blocks of a compute unit give the halo to different waves.
+  TileCell c, d;
+  c.x = (1 + lt / T) * R + 1 + lt % T;
+  const int hw = __builtin_amdgcn_readfirstlane(((lt >> 6) + ((b >> 7) & 2)) & 3);
+  const bool halo_wave = hw < 2;
+  const int hl = hw * 64 + (lt & 63);
+  const bool halo = halo_wave && hl < RR - T * T;
+  int hi_ = 0, hj = 0;
+  if (hl < NT) hi_ = hl, hj = 0;                                      // j = 0: i = 0 .. T + 1
+  else if (hl < 2 * NT) hi_ = hl - NT, hj = T + 1;                    // j = T + 1
+  else if (hl < 2 * NT + T) hi_ = 0, hj = hl - 2 * NT + 1;            // i = 0: j = 1 .. T
+  else if (hl < 2 * NT + 2 * T) hi_ = T + 1, hj = hl - 2 * NT - T + 1;  // i = T + 1
+  else if (hl < 2 * NT + 2 * T + R) hi_ = hl - 2 * NT - 2 * T, hj = T + 2;     // rim j = T + 2: i = 0 .. T + 2
+  else if (hl < RR - T * T) hi_ = T + 2, hj = hl - 2 * NT - 2 * T - R;         // rim i = T + 2: j = 0 .. T + 1
+  d.x = hj * R + hi_;
+  const bool dtri = halo && hl < 2 * NT + 2 * T;
+  const bool dp = dtri && hi_ >= 1 && hj >= 1;  // cell with a Bernoulli function
+  const bool pole = dp && ((lz == 0 && cSE && hi_ == T + 1 && hj == 1) || (lz == 5 && cNW && hi_ == 1 && hj == T + 1));
+  // qe of the halo cells at the pentagon corners, two values per corner,
+  // evaluated for all of the block's layers before the loop
+  const int which = hj <= 1 ? (hi_ <= 1 ? 0 : 1) : (hi_ <= 1 ? 2 : 3);
+  const bool mine = which == 0 ? cSW : which == 1 ? cSE : which == 2 ? cNW : cNE;
+  const bool fix0 = dtri && mine && ((which == 0 && d.x == R) || (which == 1 && d.x == R + T + 1) ||
+                                     (which == 3 && d.x == (T + 1) * R + T + 1));
+  const bool fix1 = dtri && mine && ((which == 1 && d.x == T) || (which == 2 && d.x == T * R));
+  const bool fix2 = dtri && mine && ((which == 0 && d.x == 1) || (which == 2 && d.x == (T + 1) * R + 1) ||
+                                     (which == 3 && d.x == (T + 1) * R + T + 1));
   const bool corner = cSW || cSE || cNW || cNE;
-
-  // region role
-  const bool active = lt < RR;
-  const int ri = lt % R, rj = lt / R;
-  const int x = lt;
-  const uint32_t xb = (uint32_t)(active ? gcell(ri, rj) : base) * 8u;  // byte offset of the cell in a plane
-  const bool tri_cell = active && ri <= T + 1 && rj <= T + 1;
-  const bool p_cell = active && ri >= 1 && rj >= 1 && ri <= T + 1 && rj <= T + 1;
-  const bool pole = (lz == 0 && cSE && ri == T + 1 && rj == 1) || (lz == 5 && cNW && ri == 1 && rj == T + 1);
-  // owned role
-  const bool own = lt < T * T;
-  const int oi = 1 + lt % T, oj = 1 + lt / T;
-  const int y = oj * R + oi;
-  const uint32_t ob = (uint32_t)gcell(oi, oj) * 8u;
-  // The loads inside the layer loop are unconditional, at clamped addresses
-  // (the values of idle threads and layers are dropped): with no branch
-  // around them the compiler's wait counts stay exact and a prefetch is not
-  // waited for before its use.
-  const int lo = lt % (T * T);
-  const uint32_t obl = (uint32_t)gcell(1 + lo % T, 1 + lo / T) * 8u;
-
-  // --- launch-invariant geometry into LDS (each group stages half) ----------
-  if (active) {
-    if (grp == 0) {
-      for (int e = 0; e < 3; ++e) {
-        gs.len[e][x] = ldo(g.len + e * NC, xb);
-        gs.ped[e][x] = ldo(g.ped + e * NC, xb);
-        gs.pedf[e][x] = ldo(g.pedf + e * NC, xb);
+  double* const fixes = a.fix + (int64_t)(blockIdx.y * 40 + lz * 4) * a.L * 2;  // [corner][layer][2]
+  if (corner) {
+    for (int i = lt; i < 4 * (k1 - k0); i += THREADS) {
+      const int wh = i & 3, k = k0 + (i >> 2);
+      if (wh == 0 ? cSW : wh == 1 ? cSE : wh == 2 ? cNW : cNE) {
+        const int64_t ks = (int64_t)k * NC;
+        double v[2];
+        pentagon_values(
+            wh, [&](int e, int i, int j) { return a.yu[3 * ks + e * NC + gcell(i, j)]; },
+            [&](int i, int j) { return a.ym[ks + gcell(i, j)]; }, g, NC, base, S, v);
+        fixes[((int64_t)wh * a.L + k) * 2] = v[0];
+        fixes[((int64_t)wh * a.L + k) * 2 + 1] = v[1];
       }
-    } else {
-      for (int p = 0; p < 6; ++p) gs.area[p][x] = ldo(g.area + p * NC, xb);
-      gs.hinv[x] = ldo(g.hinv, xb);
-      gs.cor[0][x] = ldo(g.cor, xb);
-      gs.cor[1][x] = ldo(g.cor + NC, xb);
     }
+    __threadfence_block();
   }
+  c.xb = (uint32_t)gcell(1 + lt % T, 1 + lt / T) * 8u;
+  d.xb = (uint32_t)gcell(hi_, hj) * 8u;
 
-  // column state (cal_surf_press, set_surf_geopot): P = pressure at the
-  // bottom of the next layer to scan, G = geopotential there.  The column
-  // sum of (mass - temp) is taken in layer order from LDS, where each group
-  // has stored (m - t) of every other layer (the layer planes are still free)
-  double P = 0, G = 0;
+  // --- launch-invariant geometry, first layer, column state ------------------
+  // (all loads before the first use)
+  const double rho = a.rho0 * 1.0, rrho = 1.0 / rho;
   {
-    constexpr int KMAX = (int)(sizeof(lsu.flat) / sizeof(double)) / RR;  // layers per round
-    double s = 0.0;
-    for (int k0 = 0; k0 < a.L; k0 += KMAX) {
-      const int kn = min(KMAX, a.L - k0);
-      if (active) {
-        for (int kk = grp; kk < kn; kk += 2) {
-          const int64_t ks = (int64_t)(k0 + kk) * NC;
-          lsu.flat[kk * RR + x] = ldo(a.ym + ks, xb) - ldo(a.yt + ks, xb);
-        }
-      }
-      __syncthreads();
-      if (p_cell)
-        for (int kk = 0; kk < kn; ++kk) s = s + lsu.flat[kk * RR + x];
-      __syncthreads();
+    double av[7], dv[7], csum = 0.0, dsum = 0.0, dt = 0.0;
+    const double* const sums = a.csum_in ? a.csum_in : g.topo;  // a load in either case
+    tile_load(c, a, k0);
+    tile_geometry(c, a);
+    tile_areas(av, a, c.xb);
+    const double ct = ldo(g.topo, c.xb);
+    csum = ldo(sums, c.xb);
+    if (halo_wave) {
+      tile_load(d, a, k0);
+      tile_geometry(d, a);
+      tile_areas(dv, a, d.xb);
+      dt = ldo(g.topo, d.xb);
+      dsum = ldo(sums, d.xb);
     }
-    if (p_cell) {
-      P = a.grav * s + a.p_top;
-      G = a.grav * ldo(g.topo, xb);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int p = 0; p < 6; ++p) s.area[p][c.x] = av[p];
+    s.hinv[c.x] = av[6];
+    tile_stage(c, s);
+    if (halo) {
+      for (int p = 0; p < 6; ++p) s.area[p][d.x] = dv[p];
+      s.hinv[d.x] = dv[6];
+      tile_stage(d, s);
     }
+    if (!a.csum_in) {
+      csum = column_sum(a.ym, a.yt, a.L, NC, c.xb);
+      if (halo_wave) dsum = column_sum(a.ym, a.yt, a.L, NC, d.xb);
+    }
+    tile_column(c, a, csum, ct, k0, rho, rrho);
+    if (halo_wave) tile_column(d, a, dsum, dt, k0, rho, rrho);
   }
-
-  LayerS& sl = lsu.ls[grp];
-  const LayerS& so = lsu.ls[1 - grp];
-  // the group's first layer, staged here; later layers are staged at the end
-  // of the previous iteration from registers loaded one iteration ahead
-  double m, t, u0, u1, u2;
-  {
-    const int64_t ks = (int64_t)min(grp, a.L - 1) * NC, ke3 = 3 * ks;
-    m = ldo(a.ym + ks, xb);
-    t = ldo(a.yt + ks, xb);
-    u0 = ldo(a.yu + ke3, xb);
-    u1 = ldo(a.yu + ke3 + NC, xb);
-    u2 = ldo(a.yu + ke3 + 2 * NC, xb);
+  double rl[3];  // reciprocals of the owned edges' lengths
+  for (int e = 0; e < 3; ++e) rl[e] = 1.0 / c.len[e];
+  double ge[3] = {0.0, 0.0, 0.0};
+  if (SPLIT) {  // theta1 grad_eta_e: g (eta(E) - eta) / len, g (eta - eta(NE)) / len, g (eta(N) - eta) / len
+    const double e0 = ldo(a.eta, c.xb);
+    ge[0] = a.th1 * (a.grav * (ldo(a.eta, c.xb + 8u) - e0) / c.len[0]);
+    ge[1] = a.th1 * (a.grav * (e0 - ldo(a.eta, c.xb + 8u * (uint32_t)(S + 1))) / c.len[1]);
+    ge[2] = a.th1 * (a.grav * (ldo(a.eta, c.xb + 8u * (uint32_t)S) - e0) / c.len[2]);
   }
-  if (active && grp < a.L) {
-    sl.m[x] = m;
-    sl.t[x] = t;
-    sl.u[0][x] = u0;
-    sl.u[1][x] = u1;
-    sl.u[2][x] = u2;
-  }
-  __builtin_amdgcn_s_waitcnt(0);  // nothing outstanding enters the layer loop
-
-  // Qperp weights of the neighbours' offsets 3-5 stay in registers; the
-  // cell's own offsets 0-2 are rebuilt from LDS in each layer
+  __syncthreads();
+  // Qperp weights of the E, NE, N neighbours (offsets 3-5); the node's own
+  // (0-2) are rebuilt from LDS in each layer
   double w[6][5];
-  if (own) {
-    weights_lds(gs, y + 1, 3, w[3]);
-    weights_lds(gs, y + R + 1, 4, w[4]);
-    weights_lds(gs, y + R, 5, w[5]);
-  }
+  weights_lds(s, c.x + 1, 3, w[3]);
+  weights_lds(s, c.x + R + 1, 4, w[4]);
+  weights_lds(s, c.x + R, 5, w[5]);
 
-  const int niter = (a.L + 1) / 2;
-  for (int it = 0; it < niter; ++it) {
-    const int k = 2 * it + grp;
-    const bool lay = k < a.L;                 // uniform over the group
-    const bool pair = 2 * it + 1 < a.L;       // both layers of the pair exist
-    const int64_t ks = (int64_t)k * NC, ke3 = 3 * ks;
-    __syncthreads();
-    // --- 1. prefetch the group's next layer (its loads overlap phases 2-4) ----
-    double nm, nt, nu0, nu1, nu2;
-    {
-      const int64_t ks2 = (int64_t)min(k + 2, a.L - 1) * NC, ke32 = 3 * ks2;
-      nm = ldo(a.ym + ks2, xb);
-      nt = ldo(a.yt + ks2, xb);
-      nu0 = ldo(a.yu + ke32, xb);
-      nu1 = ldo(a.yu + ke32 + NC, xb);
-      nu2 = ldo(a.yu + ke32 + 2 * NC, xb);
+  double sum = 0.0;  // column sum of the new mass - temp
+  for (int k = k0; k < k1; ++k) {
+    const int ku = uniform_layer(k);
+    const int64_t ks = (int64_t)ku * NC, ke3 = 3 * ks;
+    const int y = c.x;
+    // --- A. column scan, PV, fluxes, edge products.  Loads return in order:
+    //        those that A and B use are issued before the next layer's ---------
+    double fix[2] = {0.0, 0.0};
+    if (corner && halo_wave && mine) {
+      fix[0] = fixes[((int64_t)which * a.L + ku) * 2];
+      fix[1] = fixes[((int64_t)which * a.L + ku) * 2 + 1];
     }
-    // the layer's diffusion hooks (clamped layer, unconditional like the prefetch)
-    double dpm[3] = {0.0, 0.0, 0.0}, dpt[3] = {0.0, 0.0, 0.0}, dpu[3] = {0.0, 0.0, 0.0};
+    double cpm[3], cpt[3], cpu[3], hpm[3], hpt[3];
     if (DIFF) {
-      const int64_t kd3 = 3 * (int64_t)min(k, a.L - 1) * NC;
       for (int e = 0; e < 3; ++e) {
-        if (a.phm) {
-          dpm[e] = ldo(a.phm + kd3 + e * NC, xb);
-          dpt[e] = ldo(a.pht + kd3 + e * NC, xb);
+        cpm[e] = a.phm ? ldo(a.phm + ke3 + e * NC, c.xb) : 0.0;
+        cpt[e] = a.phm ? ldo(a.pht + ke3 + e * NC, c.xb) : 0.0;
+        if (halo_wave) {
+          hpm[e] = a.phm ? ldo(a.phm + ke3 + e * NC, d.xb) : 0.0;
+          hpt[e] = a.phm ? ldo(a.pht + ke3 + e * NC, d.xb) : 0.0;
         }
-        if (a.phu) dpu[e] = ldo(a.phu + kd3 + e * NC, obl);
+        cpu[e] = a.phu ? ldo(a.phu + ke3 + e * NC, c.xb) : 0.0;
       }
     }
+    const int kn = min(ku + 1, a.L - 1);
+    tile_load(c, a, kn);
+    if (halo_wave) tile_load(d, a, kn);
+    tile_fluxes<KEEP, DIFF>(c, s, a, ke3, rho, rrho, true, cpm, cpt);
+    if (halo_wave) tile_fluxes<KEEP, DIFF>(d, s, a, ke3, rho, rrho, dtri, hpm, hpt);
+    __syncthreads();
 
-    // --- 2. column scan; PV, fluxes; kinetic energy, Bernoulli, Exner ---------
-    if (lay) {
-      if (p_cell) {
-        // layer 2it is group 0's; group 1 scans it from group 0's planes first
-        double pr, phi_k;
-        if (grp == 1) {
-          const double mo = so.m[x], to = so.t[x];
-          P = P - a.grav * (mo - to);
-          G = G + a.grav * mo / (a.rho0 * 1.0);
-        }
-        {
-          double p_upper = P - a.grav * (m - t);
-          pr = interp(P, p_upper);
-          double gpl = G;
-          G = gpl + a.grav * m / (a.rho0 * 1.0);
-          phi_k = interp(G, gpl);
-          P = p_upper;
-        }
-        if (grp == 0 && pair) {
-          const double mo = so.m[x], to = so.t[x];
-          P = P - a.grav * (mo - to);
-          G = G + a.grav * mo / (a.rho0 * 1.0);
-        }
-        const int xW = x - 1, xS = x - R, xSW = x - R - 1;
-        double uS = sl.u[2][xS], uSW = sl.u[1][xSW], uW = sl.u[0][xW];
-        double ke = ((u2 * gs.len[2][x]) * (u2 * gs.ped[2][x]) + (u1 * gs.len[1][x]) * (u1 * gs.ped[1][x]) +
-                     (u0 * gs.len[0][x]) * (u0 * gs.ped[0][x]) + (uS * gs.len[2][xS]) * (uS * gs.ped[2][xS]) +
-                     (uSW * gs.len[1][xSW]) * (uSW * gs.ped[1][xSW]) + (uW * gs.len[0][xW]) * (uW * gs.ped[0][xW])) *
-                    gs.hinv[x] / 4.0;
-        sl.bern[x] = ke + phi_k + pr / (a.rho0 * 1.0);
-        sl.exn[x] = -phi_k;
-        if (KEEP) {
-          sto(a.k_bern + ks, xb, sl.bern[x]);
-          sto(a.k_exn + ks, xb, sl.exn[x]);
-        }
+    // --- B. base state of the update (q = y for a trend), consumed in C; qe on
+    //        edges, Bernoulli function, potential temperature ------------------
+    const uint32_t pb = (uint32_t)NC * 8u;
+    const Plane qu3 = plane(a.qu + ke3);
+    const double bm = ldp(plane(a.qm + ks), c.xb), bt = ldp(plane(a.qt + ks), c.xb);
+    const double bu[3] = {ldp(qu3, c.xb), ldp(qu3, c.xb, pb), ldp(qu3, c.xb, 2 * pb)};
+    const double qe[3] = {interp(s.pvU[y - R], c.pvl), interp(c.pvu, c.pvl), interp(c.pvu, s.pvL[y - 1])};
+    for (int e = 0; e < 3; ++e) s.qe[e][y] = qe[e];
+    const double th0 = c.t / c.m;
+    s.th[y] = th0;
+    const double b0 = tile_bernoulli<KEEP>(c, s, a, ks, rho, rrho), x0 = -c.phi;
+    if (halo_wave) {
+      if (dtri) {
+        if (hj >= 1) s.qe[0][d.x] = fix0 ? fix[0] : interp(s.pvU[d.x - R], d.pvl);
+        s.qe[1][d.x] = fix1 ? fix[1] : interp(d.pvu, d.pvl);
+        if (hi_ >= 1) s.qe[2][d.x] = fix2 ? (which == 2 ? fix[0] : fix[1]) : interp(d.pvu, s.pvL[d.x - 1]);
       }
-      if (tri_cell) {
-        const int xE = x + 1, xN = x + R, xNE = x + R + 1;
-        double upRT = u0 * gs.len[0][x], upDG = u1 * gs.len[1][x], upUP = u2 * gs.len[2][x];
-        double circL = upRT + sl.u[2][xE] * gs.len[2][xE] + upDG;
-        double circU = -(upDG + upUP + sl.u[0][xN] * gs.len[0][xN]);
-        double mE = sl.m[xE], mNE = sl.m[xNE], mN = sl.m[xN];
-        double massL = m * gs.area[0][x] + mE * gs.area[2][xE] + mNE * gs.area[4][xNE];
-        double massU = m * gs.area[1][x] + mNE * gs.area[3][xNE] + mN * gs.area[5][xN];
-        sl.pvL[x] = (gs.cor[0][x] + circL) / massL;
-        sl.pvU[x] = (gs.cor[1][x] + circU) / massU;
-        const double f0 = gs.pedf[0][x], f1 = gs.pedf[1][x], f2 = gs.pedf[2][x];
-        sl.hm[0][x] = u0 * f0 * interp(m, mE) + dpm[0];
-        sl.hm[1][x] = u1 * f1 * interp(m, mNE) + dpm[1];
-        sl.hm[2][x] = u2 * f2 * interp(m, mN) + dpm[2];
-        sl.ht[0][x] = u0 * f0 * interp(t, sl.t[xE]) + dpt[0];
-        sl.ht[1][x] = u1 * f1 * interp(t, sl.t[xNE]) + dpt[1];
-        sl.ht[2][x] = u2 * f2 * interp(t, sl.t[xN]) + dpt[2];
-        if (KEEP) {
-          for (int e = 0; e < 3; ++e) {
-            sto(a.k_hm + ke3 + e * NC, xb, sl.hm[e][x]);
-            sto(a.k_ht + ke3 + e * NC, xb, sl.ht[e][x]);
-          }
-        }
+      if (dp) {
+        s.th[d.x] = d.t / d.m;
+        tile_bernoulli<KEEP>(d, s, a, ks, rho, rrho);
       }
     }
     __syncthreads();
 
-    // --- 3. base state of the update (q = y for a trend), consumed in phase 4;
-    //        qe on edges; potential temperature t/m in place ------------------
-    double bm, bt, bu0, bu1, bu2;
+    // --- C. trends of owned nodes and edges, pole master; RK update -----------
+    const double dmt = tile_scalars<KEEP>(c, s, a, ks, bm, bt);
+    if (!SPLIT && !KEEP) sum = sum + dmt;
+    if (halo_wave && pole) {
+      const double pmt = tile_scalars<KEEP>(d, s, a, ks, ldo(a.qm + ks, d.xb), ldo(a.qt + ks, d.xb));
+      if (!SPLIT && !KEEP && a.csum_out) sto(a.csum_out, d.xb, (k == k0 ? 0.0 : ldo(a.csum_out, d.xb)) + pmt);
+    }
     {
-      const int64_t ksb = (int64_t)min(k, a.L - 1) * NC, ke3b = 3 * ksb;
-      bm = ldo(a.qm + ksb, obl);
-      bt = ldo(a.qt + ksb, obl);
-      bu0 = ldo(a.qu + ke3b, obl);
-      bu1 = ldo(a.qu + ke3b + NC, obl);
-      bu2 = ldo(a.qu + ke3b + 2 * NC, obl);
-    }
-    if (lay && active) {
-      if (tri_cell) {
-        if (rj >= 1) sl.qe[0][x] = interp(sl.pvU[x - R], sl.pvL[x]);
-        sl.qe[1][x] = interp(sl.pvU[x], sl.pvL[x]);
-        if (ri >= 1) sl.qe[2][x] = interp(sl.pvU[x], sl.pvL[x - 1]);
-      }
-      sl.t[x] = t / m;
-    }
-    __syncthreads();
-
-    if (corner) {
-      const bool mine[4] = {cSW, cSE, cNW, cNE};
-      if (lay && lt < 4 && mine[lt])
-        pentagon_fixup(lt, sl.u[0], sl.u[1], sl.u[2], sl.m, sl.qe[0], sl.qe[1], sl.qe[2], g, NC, base, S);
-      __syncthreads();
-    }
-
-    // --- 4. trends of owned nodes and edges, pole master; RK update -----------
-    if (lay && own) {
       const int xW = y - 1, xS = y - R, xSW = y - R - 1, xE = y + 1, xN = y + R, xNE = y + R + 1;
       const int xNW = y + R - 1, xSE = y - R + 1;
-      const double hi = gs.hinv[y];
-      double divm = (sl.hm[0][y] - sl.hm[0][xW] + sl.hm[1][xSW] - sl.hm[1][y] + sl.hm[2][y] - sl.hm[2][xS]) * hi;
-      double divt = (sl.ht[0][y] - sl.ht[0][xW] + sl.ht[1][xSW] - sl.ht[1][y] + sl.ht[2][y] - sl.ht[2][xS]) * hi;
-      double dmv = -divm, dtv = -divt;
-      sto(a.om + ks, ob, a.trend_only ? dmv : bm + a.h * dmv);
-      sto(a.ot + ks, ob, a.trend_only ? dtv : bt + a.h * dtv);
-      if (KEEP) {
-        sto(a.k_dm + ks, ob, dmv);
-        sto(a.k_dt + ks, ob, dtv);
-      }
       double qp[3];
-      weights_lds(gs, y, 0, w[0]);
-      weights_lds(gs, y, 1, w[1]);
-      weights_lds(gs, y, 2, w[2]);
-#define HM(e, xx) sl.hm[e][xx]
-#define QE(e, xx) sl.qe[e][xx]
-      double qr = QE(0, y);
-      qp[0] = HM(1, y) * interp(QE(1, y), qr) * w[0][0] + HM(2, y) * interp(QE(2, y), qr) * w[0][1] +
+      weights_lds(s, c.x, 0, w[0]);
+      weights_lds(s, c.x, 1, w[1]);
+      weights_lds(s, c.x, 2, w[2]);
+#define HM(e, xx) s.hm[e][xx]
+#define QE(e, xx) s.qe[e][xx]
+      const double qr = qe[0], qd = qe[1], qu = qe[2];
+      qp[0] = HM(1, y) * interp(qd, qr) * w[0][0] + HM(2, y) * interp(qu, qr) * w[0][1] +
               HM(0, xW) * interp(QE(0, xW), qr) * w[0][2] + HM(1, xSW) * interp(QE(1, xSW), qr) * w[0][3] +
               HM(2, xS) * interp(QE(2, xS), qr) * w[0][4] + HM(1, xS) * interp(QE(1, xS), qr) * w[3][0] +
               HM(2, xSE) * interp(QE(2, xSE), qr) * w[3][1] + HM(0, xE) * interp(QE(0, xE), qr) * w[3][2] +
               HM(1, xE) * interp(QE(1, xE), qr) * w[3][3] + HM(2, xE) * interp(QE(2, xE), qr) * w[3][4];
-      double qd = QE(1, y);
-      qp[1] = HM(2, y) * interp(QE(2, y), qd) * w[1][0] + HM(0, xW) * interp(QE(0, xW), qd) * w[1][1] +
+      qp[1] = HM(2, y) * interp(qu, qd) * w[1][0] + HM(0, xW) * interp(QE(0, xW), qd) * w[1][1] +
               HM(1, xSW) * interp(QE(1, xSW), qd) * w[1][2] + HM(2, xS) * interp(QE(2, xS), qd) * w[1][3] +
-              HM(0, y) * interp(QE(0, y), qd) * w[1][4] + HM(2, xE) * interp(QE(2, xE), qd) * w[4][0] +
+              HM(0, y) * interp(qr, qd) * w[1][4] + HM(2, xE) * interp(QE(2, xE), qd) * w[4][0] +
               HM(0, xNE) * interp(QE(0, xNE), qd) * w[4][1] + HM(1, xNE) * interp(QE(1, xNE), qd) * w[4][2] +
               HM(2, xNE) * interp(QE(2, xNE), qd) * w[4][3] + HM(0, xN) * interp(QE(0, xN), qd) * w[4][4];
-      double qu = QE(2, y);
       qp[2] = HM(0, xW) * interp(QE(0, xW), qu) * w[2][0] + HM(1, xSW) * interp(QE(1, xSW), qu) * w[2][1] +
-              HM(2, xS) * interp(QE(2, xS), qu) * w[2][2] + HM(0, y) * interp(QE(0, y), qu) * w[2][3] +
-              HM(1, y) * interp(QE(1, y), qu) * w[2][4] + HM(0, xN) * interp(QE(0, xN), qu) * w[5][0] +
+              HM(2, xS) * interp(QE(2, xS), qu) * w[2][2] + HM(0, y) * interp(qr, qu) * w[2][3] +
+              HM(1, y) * interp(qd, qu) * w[2][4] + HM(0, xN) * interp(QE(0, xN), qu) * w[5][0] +
               HM(1, xN) * interp(QE(1, xN), qu) * w[5][1] + HM(2, xN) * interp(QE(2, xN), qu) * w[5][2] +
               HM(0, xNW) * interp(QE(0, xNW), qu) * w[5][3] + HM(1, xW) * interp(QE(1, xW), qu) * w[5][4];
 #undef HM
 #undef QE
-      const double th0 = sl.t[y];
-      double the[3] = {interp(th0, sl.t[xE]), interp(th0, sl.t[xNE]), interp(th0, sl.t[xN])};
-      const double b0 = sl.bern[y], x0 = sl.exn[y];
-      const double ll[3] = {gs.len[0][y], gs.len[1][y], gs.len[2][y]};
-      double gB[3] = {(sl.bern[xE] - b0) / ll[0], (b0 - sl.bern[xNE]) / ll[1], (sl.bern[xN] - b0) / ll[2]};
-      double gX[3] = {(sl.exn[xE] - x0) / ll[0], (x0 - sl.exn[xNE]) / ll[1], (sl.exn[xN] - x0) / ll[2]};
-      const double bu[3] = {bu0, bu1, bu2};
-      double ge[3] = {0.0, 0.0, 0.0};
-      if (SPLIT) {  // grad_eta_e: g (eta(E) - eta) / len, g (eta - eta(NE)) / len, g (eta(N) - eta) / len
-        const double e0 = ldo(a.eta, ob);
-        ge[0] = a.grav * (ldo(a.eta, ob + 8u) - e0) / ll[0];
-        ge[1] = a.grav * (e0 - ldo(a.eta, ob + 8u * (uint32_t)(S + 1))) / ll[1];
-        ge[2] = a.grav * (ldo(a.eta, ob + 8u * (uint32_t)S) - e0) / ll[2];
-      }
+      const double the[3] = {interp(th0, s.th[xE]), interp(th0, s.th[xNE]), interp(th0, s.th[xN])};
+      const double dB[3] = {s.bern[xE] - b0, b0 - s.bern[xNE], s.bern[xN] - b0};
+      const double dX[3] = {s.exn[xE] - x0, x0 - s.exn[xNE], s.exn[xN] - x0};
+      const Plane ou3 = plane(a.ou + ke3);
       for (int e = 0; e < 3; ++e) {
-        double src = -qp[e] + dpu[e] * ll[e];
-        double du = src / ll[e] - gB[e] - the[e] * gX[e];
-        sto(a.ou + ke3 + e * NC, ob, a.trend_only ? du : bu[e] + a.h * (SPLIT ? du + a.th1 * ge[e] : du));
-        if (KEEP) sto(a.k_src + ke3 + e * NC, ob, src);
+        const double l = c.len[e];
+        double src = -qp[e];
+        if (DIFF) src = src + cpu[e] * l;
+        const double du = div_by(src, l, rl[e]) - div_by(dB[e], l, rl[e]) - the[e] * div_by(dX[e], l, rl[e]);
+        stp(ou3, c.xb, a.trend_only ? du : bu[e] + a.h * (SPLIT ? du + ge[e] : du), e * pb);
+        if (KEEP) sto(a.k_src + ke3 + e * NC, c.xb, src);
       }
     }
-    if (!(lay && own)) {
-      // threads that store nothing still wait for their base-state loads
-      // here, so no later phase inherits an unknown wait on them
-      asm volatile("" ::"v"(bm), "v"(bt), "v"(bu0), "v"(bu1), "v"(bu2));
-    }
-    if (lay && pole) {
-      const double hi = gs.hinv[x];
-      const int xW = x - 1, xS = x - R, xSW = x - R - 1;
-      double divm = (sl.hm[0][x] - sl.hm[0][xW] + sl.hm[1][xSW] - sl.hm[1][x] + sl.hm[2][x] - sl.hm[2][xS]) * hi;
-      double divt = (sl.ht[0][x] - sl.ht[0][xW] + sl.ht[1][xSW] - sl.ht[1][x] + sl.ht[2][x] - sl.ht[2][xS]) * hi;
-      double dmv = -divm, dtv = -divt;
-      sto(a.om + ks, xb, a.trend_only ? dmv : ldo(a.qm + ks, xb) + a.h * dmv);
-      sto(a.ot + ks, xb, a.trend_only ? dtv : ldo(a.qt + ks, xb) + a.h * dtv);
-      if (KEEP) {
-        sto(a.k_dm + ks, xb, dmv);
-        sto(a.k_dt + ks, xb, dtv);
-      }
-    }
+    // --- the next layer's planes, which C does not read ------------------------
+    tile_stage(c, s);
+    if (halo) tile_stage(d, s);
     __syncthreads();
-    // --- 5. stage the group's next layer --------------------------------------
-    if (active && k + 2 < a.L) {
-      sl.m[x] = nm;
-      sl.t[x] = nt;
-      sl.u[0][x] = nu0;
-      sl.u[1][x] = nu1;
-      sl.u[2][x] = nu2;
-    }
-    m = nm;
-    t = nt;
-    u0 = nu0;
-    u1 = nu1;
-    u2 = nu2;
   }
+  if (!SPLIT && !KEEP && a.csum_out) sto(a.csum_out, c.xb, sum);
 }
 
 // halo := owner (nodes: mass and temp; edges: velocity with sign), all
@@ -1167,7 +1275,7 @@ constexpr int GF_KC = 8;
 template <class F>
 __global__ void ghost_fill_kernel(int L, int64_t NC, const int64_t* __restrict__ nd, int nn,
                                   const int64_t* __restrict__ ed, const int8_t* __restrict__ es, int ne, F* m, F* t,
-                                  F* u) {
+                                  F* u, double* cs = nullptr, int ncs = 0) {
   const int64_t E = (int64_t)nn + ne;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= E * ((L + GF_KC - 1) / GF_KC)) return;
@@ -1188,6 +1296,8 @@ __global__ void ghost_fill_kernel(int L, int64_t NC, const int64_t* __restrict__
         m[(int64_t)(k0 + i) * NC + dst] = vm[i];
         t[(int64_t)(k0 + i) * NC + dst] = vt[i];
       }
+    if (cs && k0 == 0)  // the members' column sums
+      for (int i = 0; i < ncs; ++i) cs[(int64_t)i * NC + dst] = cs[(int64_t)i * NC + src];
   } else {
     const int64_t j = e - nn;
     const int64_t dst = ed[2 * j], src = ed[2 * j + 1];  // plane indices e*NC + cell
@@ -1247,7 +1357,8 @@ __global__ void copy_frozen_kernel(int L, int64_t NC, const int64_t* __restrict_
 // ---------------------------------------------------------------------------
 // FP32-bulk stage kernel (precision mode WTG_PRECISION_FP32_BULK)
 // ---------------------------------------------------------------------------
-// The same tile, layer pairing and phases as trisk_stage_pair_kernel, with
+// The same tile and stencils as trisk_stage_tile_kernel in 768-thread blocks of
+// two layers in lock step (two groups of 384 threads), with
 // the bulk of the stencils in FP32: the velocity, mass and temperature planes
 // of the flux stencils, circulation, potential vorticity, qe, mass and
 // temperature fluxes, kinetic energy, divergence and the Qperp sum.  FP64
@@ -2029,13 +2140,14 @@ __global__ void geo_f32_kernel(int64_t NC, const double* __restrict__ len, const
 // dilation of mass / temp to the free surface eta; porosity 1, mean state 0
 __global__ void baro_correction_kernel(int nmaster, const int64_t* __restrict__ ncl, int L, int64_t NC, double rho0,
                                        const double* __restrict__ eta, const double* __restrict__ topo, double* m,
-                                       double* t) {
+                                       double* t, double* csum) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nmaster) return;
   const int64_t c = ncl[2 * i + 1];
   double h = 0.0;  // total_height (cal_height: rho_dz / porous_density)
   for (int k = 0; k < L; ++k) h = h + (0.0 + m[(int64_t)k * NC + c]) / (rho0 * 1.0);
   const double e = eta[c] / 1.0, b = topo[c];
+  double s = 0.0;  // column sum of the new mass - temp, for the stage kernel
   for (int k = 0; k < L; ++k) {
     const int64_t x = (int64_t)k * NC + c;
     double rho_dz = 0.0 + m[x];
@@ -2043,8 +2155,11 @@ __global__ void baro_correction_kernel(int nmaster, const int64_t* __restrict__ 
     const double mm = (e - b) / h * rho_dz - 0.0;
     m[x] = mm;
     rho_dz = 0.0 + mm;
-    t[x] = rho_dz * theta - 0.0;
+    const double tt = rho_dz * theta - 0.0;
+    t[x] = tt;
+    s = s + (mm - tt);
   }
+  if (csum) csum[c] = s;
 }
 
 // g grad(eta) on edge e of cell c (grad_eta, step1 itype 3, ops.f90:217-220)
@@ -2130,18 +2245,20 @@ int check_slot(wtg_ctx* c, int slot) {
 }
 
 template <class F>
-int launch_ghost_fill(wtg_ctx* c, F* m, F* t, F* u) {
+int launch_ghost_fill(wtg_ctx* c, F* m, F* t, F* u, double* csum = nullptr) {
   const int L = c->params.nlayers * c->nmembers;
   int64_t total = (int64_t)(c->nn + c->ne) * ((L + GF_KC - 1) / GF_KC);
   if (total == 0) return 0;
   int threads = 256;
   int64_t blocks = (total + threads - 1) / threads;
   hipLaunchKernelGGL(ghost_fill_kernel<F>, dim3((unsigned)blocks), dim3(threads), 0, c->stream, L, c->info.ncells,
-                     c->d_nd, c->nn, c->d_ed, c->d_es, c->ne, m, t, u);
+                     c->d_nd, c->nn, c->d_ed, c->d_es, c->ne, m, t, u, csum, csum ? c->nmembers : 0);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
-int launch_ghost_fill(wtg_ctx* c, const wtg_ctx::Slot& s) { return launch_ghost_fill(c, s.m, s.t, s.u); }
+int launch_ghost_fill(wtg_ctx* c, const wtg_ctx::Slot& s, double* csum = nullptr) {
+  return launch_ghost_fill(c, s.m, s.t, s.u, csum);
+}
 
 int launch_copy_frozen(wtg_ctx* c, const wtg_ctx::Slot& from, const wtg_ctx::Slot& to) {
   const int L = c->params.nlayers * c->nmembers;
@@ -2155,18 +2272,44 @@ int launch_copy_frozen(wtg_ctx* c, const wtg_ctx::Slot& from, const wtg_ctx::Slo
   return 0;
 }
 
+// Chunks of layers per tile: as many as keep every block resident at once (512
+// blocks, two per compute unit), so that small grids fill the chip; a chunk
+// scans the columns below it, which costs more than it gives once the tiles
+// alone fill the chip.  Stage launch without / with chunks: J6 L7 (160 tiles, 3
+// chunks) 42 -> 28 us, J6 L20 86 -> 49 us, J5 L20 (40 tiles, 10 chunks) 85 ->
+// 30 us; J6 L20 in twice as many chunks 67 us.
+constexpr unsigned RESIDENT_BLOCKS = 512;
+int stage_chunks(unsigned blocks, int L) {
+  return std::max(1, std::min(L, (int)(RESIDENT_BLOCKS / blocks)));
+}
+
+unsigned stage_blocks(const wtg_ctx* c) {
+  const unsigned nt = (unsigned)(c->info.n / T);
+  return 10 * nt * nt * (unsigned)c->nmembers;
+}
+
+// whether a stage can leave the column sums of its new state: one block holds
+// all of a tile's layers
+bool stage_keeps_csum(const wtg_ctx* c) {
+  return c->stage_version == 3 && stage_chunks(stage_blocks(c), c->params.nlayers) == 1;
+}
+
 int launch_stage(wtg_ctx* c, const wtg_ctx::Slot& y, const wtg_ctx::Slot& q, const wtg_ctx::Slot& out, double h,
-                 int trend_only, const WtgStageKeep* keep = nullptr, const double* split_eta = nullptr) {
+                 int trend_only, const WtgStageKeep* keep = nullptr, const double* split_eta = nullptr,
+                 const double* csum_in = nullptr, double* csum_out = nullptr) {
   StageArgs a{};
+  a.csum_in = csum_in;
+  a.csum_out = csum_out;
+  a.fix = c->d_fix;
   if (split_eta) {
     if (c->stage_version != 3 || keep || trend_only)
-      return fail(c, WTG_E_STATE, "the fused split-explicit stage needs the layer-pair kernel");
+      return fail(c, WTG_E_STATE, "the fused split-explicit stage needs the default stage kernel");
     a.eta = split_eta;
     a.th1 = c->fs_theta1;
   }
   if (c->dif_on) {
     if (c->stage_version != 3 || keep)
-      return fail(c, WTG_E_STATE, "diffusion needs the layer-pair stage kernel on a single level");
+      return fail(c, WTG_E_STATE, "diffusion needs the default stage kernel on a single level");
     if (int rc = wtg_diffusion_prepass(c, y.m, y.t, y.u)) return rc;
     a.phm = c->dif_phm;
     a.pht = c->dif_pht;
@@ -2174,7 +2317,7 @@ int launch_stage(wtg_ctx* c, const wtg_ctx::Slot& y, const wtg_ctx::Slot& q, con
   }
   if (keep) {
     if (c->stage_version != 3 || c->nmembers != 1)
-      return fail(c, WTG_E_STATE, "kept stage quantities need the layer-pair kernel on a single-member context");
+      return fail(c, WTG_E_STATE, "kept stage quantities need the default stage kernel on a single-member context");
     a.k_hm = keep->hm;
     a.k_ht = keep->ht;
     a.k_bern = keep->bern;
@@ -2207,20 +2350,23 @@ int launch_stage(wtg_ctx* c, const wtg_ctx::Slot& y, const wtg_ctx::Slot& q, con
   a.p_top = c->params.p_top;
   unsigned blocks = (unsigned)(10 * a.ntile * a.ntile);
   const dim3 grid(blocks, (unsigned)c->nmembers);
+  const int nz = stage_chunks(blocks * (unsigned)c->nmembers, a.L);
+  a.kchunk = (a.L + nz - 1) / nz;
+  const dim3 tgrid(blocks, (unsigned)c->nmembers, (unsigned)((a.L + a.kchunk - 1) / a.kchunk));
   if (c->stage_version == 1)
     hipLaunchKernelGGL(trisk_stage_kernel, grid, dim3(THREADS), 0, c->stream, a);
   else if (c->stage_version == 2)
     hipLaunchKernelGGL(trisk_stage_kernel2, grid, dim3(THREADS2), 0, c->stream, a);
   else if (keep)
-    hipLaunchKernelGGL((trisk_stage_pair_kernel<true, false, false>), grid, dim3(THREADS3), 0, c->stream, a);
+    hipLaunchKernelGGL((trisk_stage_tile_kernel<true, false, false>), tgrid, dim3(THREADS), 0, c->stream, a);
   else if (split_eta && c->dif_on)
-    hipLaunchKernelGGL((trisk_stage_pair_kernel<false, true, true>), grid, dim3(THREADS3), 0, c->stream, a);
+    hipLaunchKernelGGL((trisk_stage_tile_kernel<false, true, true>), tgrid, dim3(THREADS), 0, c->stream, a);
   else if (split_eta)
-    hipLaunchKernelGGL((trisk_stage_pair_kernel<false, true, false>), grid, dim3(THREADS3), 0, c->stream, a);
+    hipLaunchKernelGGL((trisk_stage_tile_kernel<false, true, false>), tgrid, dim3(THREADS), 0, c->stream, a);
   else if (c->dif_on)
-    hipLaunchKernelGGL((trisk_stage_pair_kernel<false, false, true>), grid, dim3(THREADS3), 0, c->stream, a);
+    hipLaunchKernelGGL((trisk_stage_tile_kernel<false, false, true>), tgrid, dim3(THREADS), 0, c->stream, a);
   else
-    hipLaunchKernelGGL((trisk_stage_pair_kernel<false, false, false>), grid, dim3(THREADS3), 0, c->stream, a);
+    hipLaunchKernelGGL((trisk_stage_tile_kernel<false, false, false>), tgrid, dim3(THREADS), 0, c->stream, a);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -2403,14 +2549,18 @@ int rk4_steps(wtg_ctx* c, int slot, double dt, int nsteps, hipEvent_t* ev) {
   const auto& w2 = c->slots[c->nslots + 1];
   const double coef[4] = {dt / 4.0, dt / 3.0, dt / 2.0, dt};
   int launch = 0;
+  // a stage leaves the column sums of its new state to the next one
+  const bool carry = stage_keeps_csum(c);
   for (int s = 0; s < nsteps; ++s) {
     const wtg_ctx::Slot* ys[4] = {&sol, &w1, &w2, &w1};
     const wtg_ctx::Slot* os[4] = {&w1, &w2, &w1, &sol};
     for (int st = 0; st < 4; ++st, ++launch) {
+      const double* cin = carry && launch > 0 ? c->d_csum[launch % 2] : nullptr;
+      double* cout = carry ? c->d_csum[(launch + 1) % 2] : nullptr;
       if (ev) HIPCHK(c, hipEventRecord(ev[2 * launch], c->stream));
-      if (int rc = launch_stage(c, *ys[st], sol, *os[st], coef[st], 0)) return rc;
+      if (int rc = launch_stage(c, *ys[st], sol, *os[st], coef[st], 0, nullptr, nullptr, cin, cout)) return rc;
       if (ev) HIPCHK(c, hipEventRecord(ev[2 * launch + 1], c->stream));
-      if (int rc = launch_ghost_fill(c, *os[st])) return rc;
+      if (int rc = launch_ghost_fill(c, *os[st], cout)) return rc;
     }
   }
   return 0;
@@ -2467,10 +2617,10 @@ int rk4_graph_impl(wtg_ctx* c, int slot, double dt, int nsteps) {
 // RK4_split (time_integr.f90:360-382): four RK_split stages (444-462) and
 // free_surface_update (464-478); the free surface solved by BiCGSTAB, the
 // reference's SRJ on a single level
-int baro_correction(wtg_ctx* c, const wtg_ctx::Slot& s) {
+int baro_correction(wtg_ctx* c, const wtg_ctx::Slot& s, double* csum = nullptr) {
   const int n = c->nmaster;
   hipLaunchKernelGGL(baro_correction_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, n, c->d_ncl,
-                     c->params.nlayers, c->info.ncells, c->params.ref_density, c->fs[FS_ETA], c->d_topo, s.m, s.t);
+                     c->params.nlayers, c->info.ncells, c->params.ref_density, c->fs[FS_ETA], c->d_topo, s.m, s.t, csum);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -2551,7 +2701,7 @@ int wtg_ghost_fill_layers(wtg_ctx* c, int L, double* m, double* t, double* u) {
   const int threads = 256;
   const int64_t blocks = (total + threads - 1) / threads;
   hipLaunchKernelGGL(ghost_fill_kernel<double>, dim3((unsigned)blocks), dim3(threads), 0, c->stream, L, c->info.ncells,
-                     c->d_nd, nn, c->d_ed, c->d_es, ne, m, t, u);
+                     c->d_nd, nn, c->d_ed, c->d_es, ne, m, t, u, (double*)nullptr, 0);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -2600,7 +2750,7 @@ int wtg_split_steps(wtg_ctx* c, int slot, int nsteps, wtg_fs_solver solve, void*
   // FP32-bulk: the trend stencils run in FP32 into the first FP32 stage
   // buffer; the stage states, the AXPYs and the free surface stay FP64
   const bool f32 = c->precision == WTG_PRECISION_FP32_BULK;
-  // FP64 with the layer-pair kernel: the stage's update is the split AXPY
+  // FP64 with the default kernel: the stage's update is the split AXPY
   const bool fused = !f32 && c->stage_version == 3 && c->split_fused;
   if (f32) {
     if (int rc = f32_ready(c)) return rc;
@@ -2641,18 +2791,19 @@ int wtg_split_steps(wtg_ctx* c, int slot, int nsteps, wtg_fs_solver solve, void*
                              c->stream));
     for (int st = 0; st < nstages; ++st) {
       const auto &in = c->slots[ins[st]], &tr = c->slots[trs[st]], &out = c->slots[outs[st]];
-      for (wtg_ctx* v : V)
-        if (int rc = baro_correction(v, v->slots[ins[st]])) return view_err(v, rc);
-      if (int rc = launch_ghost_fill(c, in)) return rc;
+      double* const csum = c->d_csum[0];
+      for (size_t i = 0; i < V.size(); ++i)
+        if (int rc = baro_correction(V[i], V[i]->slots[ins[st]], csum + (int64_t)i * NC)) return view_err(V[i], rc);
+      if (int rc = launch_ghost_fill(c, in, csum)) return rc;
       if (fused && ins[st] != outs[st]) {  // trend and u_star / scalar_star in one launch
-        if (int rc = launch_stage(c, in, sol, out, coef[st], 0, nullptr, c->fs[FS_ETA])) return rc;
+        if (int rc = launch_stage(c, in, sol, out, coef[st], 0, nullptr, c->fs[FS_ETA], csum)) return rc;
         if (int rc = launch_ghost_fill(c, out)) return rc;
         continue;
       }
       if (f32) {
         if (int rc = launch_stage_mixed<false, float>(c, in, nullptr, ftr.m, ftr.t, ftr.u, 1.0)) return rc;
       } else {
-        if (int rc = launch_stage(c, in, in, tr, 0.0, 1)) return rc;
+        if (int rc = launch_stage(c, in, in, tr, 0.0, 1, nullptr, nullptr, csum)) return rc;
       }
       for (wtg_ctx* v : V) {
         const auto &vs = v->slots[slot], &vt = v->slots[trs[st]], &vo = v->slots[outs[st]];
@@ -2951,7 +3102,10 @@ int wtg_create_ensemble(const wtg_grid* grid, const wtg_params* params, int nmem
     wtg_destroy(c.release());
     return rc;
   }
-  if ((rc = dalloc<double>(cp, &c->d_topo, (size_t)nmembers * NC))) {
+  if ((rc = dalloc<double>(cp, &c->d_topo, (size_t)nmembers * NC)) ||
+      (rc = dalloc<double>(cp, &c->d_csum[0], (size_t)nmembers * NC)) ||
+      (rc = dalloc<double>(cp, &c->d_csum[1], (size_t)nmembers * NC)) ||
+      (rc = dalloc<double>(cp, &c->d_fix, (size_t)nmembers * 80 * params->nlayers))) {
     g_create_error = c->err;
     wtg_destroy(c.release());
     return rc;
@@ -3084,7 +3238,7 @@ int wtg_ghost_fill_split_timed(wtg_ctx* c, int slot, int nshards, int reps, doub
       hipEventRecord(e0, c->stream);
       for (int k = 0; k < reps; ++k)
         hipLaunchKernelGGL(ghost_fill_kernel<double>, dim3(blocks), dim3(256), 0, c->stream, L, NC, dn, nn, de, dsg,
-                           ne, s.m, s.t, s.u);
+                           ne, s.m, s.t, s.u, (double*)nullptr, 0);
       hipEventRecord(e1, c->stream);
       if (hipGetLastError() != hipSuccess || hipEventSynchronize(e1) != hipSuccess)
         rc = fail(c, WTG_E_DEVICE, "split ghost fill failed");
@@ -3235,7 +3389,7 @@ int wtg_set_diffusion(wtg_ctx* c, const wtg_diffusion* d) {
   if (on && c->precision != WTG_PRECISION_FP64)
     return fail(c, WTG_E_STATE, "diffusion is FP64 only (the context is in the FP32-bulk precision)");
   if (on && c->stage_version != 3)
-    return fail(c, WTG_E_STATE, "diffusion needs the layer-pair stage kernel (WTG_STAGE_KERNEL unset)");
+    return fail(c, WTG_E_STATE, "diffusion needs the default stage kernel (WTG_STAGE_KERNEL unset)");
   c->dif = v;
   c->dif_on = on;
   if (on)
