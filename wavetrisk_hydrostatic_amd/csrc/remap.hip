@@ -12,7 +12,7 @@
 // reconciliation, remap.f90:737-948).
 //
 // One thread per column (owned node or pole master; grid y = ensemble
-// member): the old interface heights z_old(k) = z_s + sum of mass / rho0 and
+// member), or per field of it (grid z; remapPPR is a kernel of its own): the old interface heights z_old(k) = z_s + sum of mass / rho0 and
 // the target ones z_new(k) = a_vert(k) eta + b_vert(k) z_s, the buoyancy
 // t / m remapped and the new mass rho0 dz, then each of the node's three
 // edges: the column of interface heights averaged with the neighbour's, the
@@ -20,11 +20,12 @@
 // copy taken before the launch, so no column sees another's update.  The
 // column arrays are private (up to WTG_REMAP_MAX_LAYERS layers); FP64 in the
 // reference's evaluation order without FMA contraction, so results equal the
-// oracle bit for bit.  The kernel is HBM-bound on a single pass over the
-// state (about 96 bytes read and written per node-layer).
+// oracle bit for bit.  remap_kernel is bound by the
+// traffic of its private arrays (scratch memory).
 #include <hip/hip_runtime.h>
 
 #include "ctx.h"
+#include "exact_div.h"
 
 namespace {
 
@@ -444,6 +445,28 @@ __device__ bool solve4(const double A[4][4], double v[4], double eps) {
   return true;
 }
 
+// the first unknown of solve4, its repeated divisors through their reciprocals
+__device__ __forceinline__ bool solve4_first(const double A[4][4], double v[4], double eps) {
+  const double adet = A[0][0] * A[1][1] - A[0][1] * A[1][0];
+  if (!(fabs(adet) > eps)) return false;
+  const double ra = 1.0 / adet;
+  const double i00 = A[1][1], i01 = -A[0][1], i10 = -A[1][0], i11 = A[0][0];
+  const double L00 = 0.0 + (A[2][0] * i00 + A[2][1] * i10), L10 = 0.0 + (A[3][0] * i00 + A[3][1] * i10);
+  const double L01 = 0.0 + (A[2][0] * i01 + A[2][1] * i11), L11 = 0.0 + (A[3][0] * i01 + A[3][1] * i11);
+  const double U00 = 0.0 + (i00 * A[0][2] + i01 * A[1][2]), U01 = 0.0 + (i00 * A[0][3] + i01 * A[1][3]);
+  const double sc = -ra;  // -1 / adet
+  const double p00 = L00 * A[0][2] + L01 * A[1][2], p10 = L10 * A[0][2] + L11 * A[1][2];
+  const double p01 = L00 * A[0][3] + L01 * A[1][3], p11 = L10 * A[0][3] + L11 * A[1][3];
+  // mul_2x2's branches for a scale of +1 and -1 give the same numbers
+  const double S00 = A[2][2] + sc * p00, S10 = A[3][2] + sc * p10, S01 = A[2][3] + sc * p01, S11 = A[3][3] + sc * p11;
+  const double sdet = S00 * S11 - S01 * S10, rs = 1.0 / sdet;
+  const double v2 = v[2] - div_by(L00 * v[0] + L01 * v[1], adet, ra), v3 = v[3] - div_by(L10 * v[0] + L11 * v[1], adet, ra);
+  const double t0 = div_by(i00 * v[0] + i01 * v[1], adet, ra);
+  const double t2 = div_by(S11 * v2 + -S01 * v3, sdet, rs), t3 = div_by(-S10 * v2 + S00 * v3, sdet, rs);
+  v[0] = t0 - div_by(U00 * t2 + U01 * t3, adet, ra);
+  return true;
+}
+
 #define PX(i) zo[(i) - 1]
 #define PXN(i) zn[(i) - 1]
 #define PF(i) vo[(i) - 1]
@@ -702,42 +725,32 @@ __device__ void coordinates(const RemapArgs& a, const double* topo, const double
   for (int k = 0; k <= a.L; ++k) zn[k] = a.a[k] * eta + a.b[k] * zs;
 }
 
-__global__ __launch_bounds__(RT) void remap_kernel(RemapArgs a) {
-  const int64_t nown = (int64_t)10 * a.n * a.n;
-  const int64_t tid = (int64_t)blockIdx.x * RT + threadIdx.x;
-  if (tid >= nown + 2) return;
-  const int64_t NC = a.NC, s1 = (int64_t)blockIdx.y * a.L * NC;
-  const double* topo = a.topo + (int64_t)blockIdx.y * NC;
+// the fields [f0, f1) of a node in private arrays: field 0 the buoyancy (with
+// the new mass), fields 1..3 the velocities of its RT, DG, UP edges
+__device__ void remap_fields(const RemapArgs& a, int64_t mb, int64_t c, int f0, int f1) {
+  const int64_t NC = a.NC, s1 = mb * a.L * NC;
+  const double* topo = a.topo + mb * NC;
   const double* mold = a.mold + s1;
   double *m = a.m + s1, *t = a.t + s1, *u = a.u + 3 * s1;
-  int64_t c;
-  bool pole = false;
-  if (tid < nown) {
-    const int lz = (int)(tid / ((int64_t)a.n * a.n)), r = (int)(tid % ((int64_t)a.n * a.n));
-    c = (int64_t)lz * a.S * a.S + (int64_t)(r / a.n + H) * a.S + (r % a.n + H);
-  } else {
-    c = tid == nown ? a.spole : a.npole;
-    pole = true;
-  }
   double zo[RMAX + 1], zn[RMAX + 1], zeo[RMAX + 1], zen[RMAX + 1], vo[RMAX], vn[RMAX];
   Work w;
   const int L = a.L;
   coordinates(a, topo, mold, c, zn, zo);
-  // buoyancy, then the new mass and mass-weighted buoyancy
-  for (int k = 0; k < L; ++k) {
-    const int64_t x = (int64_t)k * NC + c;
-    vo[k] = (0.0 + t[x]) / (0.0 + m[x]);
+  if (f0 == 0) {  // buoyancy, then the new mass and mass-weighted buoyancy
+    for (int k = 0; k < L; ++k) {
+      const int64_t x = (int64_t)k * NC + c;
+      vo[k] = (0.0 + t[x]) / (0.0 + mold[x]);
+    }
+    remap_col(a.scheme, L, vn, zn, vo, zo, w);
+    for (int k = 0; k < L; ++k) {
+      const int64_t x = (int64_t)k * NC + c;
+      const double rho_dz = (a.rho0 * 1.0) * (zn[k + 1] - zn[k]);
+      m[x] = rho_dz - 0.0;
+      t[x] = rho_dz * vn[k] - 0.0;
+    }
   }
-  remap_col(a.scheme, L, vn, zn, vo, zo, w);
-  for (int k = 0; k < L; ++k) {
-    const int64_t x = (int64_t)k * NC + c;
-    const double rho_dz = (a.rho0 * 1.0) * (zn[k + 1] - zn[k]);
-    m[x] = rho_dz - 0.0;
-    t[x] = rho_dz * vn[k] - 0.0;
-  }
-  if (pole) return;  // velocities are not remapped at the poles
   const int64_t nb[3] = {c + 1, c + a.S + 1, c + a.S};
-  for (int e = 0; e < 3; ++e) {
+  for (int e = max(f0, 1) - 1; e < f1 - 1; ++e) {
     coordinates(a, topo, mold, nb[e], zen, zeo);
     for (int k = 0; k <= L; ++k) {
       zen[k] = 0.5 * (zn[k] + zen[k]);
@@ -746,6 +759,342 @@ __global__ __launch_bounds__(RT) void remap_kernel(RemapArgs a) {
     for (int k = 0; k < L; ++k) vo[k] = u[((int64_t)k * 3 + e) * NC + c];
     remap_col(a.scheme, L, vn, zen, vo, zeo, w);
     for (int k = 0; k < L; ++k) u[((int64_t)k * 3 + e) * NC + c] = vn[k];
+  }
+}
+
+// the cell of column `tid`: owned nodes, then the south and north pole masters
+__device__ __forceinline__ int64_t column_cell(const RemapArgs& a, int64_t tid) {
+  const int64_t nown = (int64_t)10 * a.n * a.n;
+  if (tid >= nown) return tid == nown ? a.spole : a.npole;
+  const int lz = (int)(tid / ((int64_t)a.n * a.n)), r = (int)(tid % ((int64_t)a.n * a.n));
+  return (int64_t)lz * a.S * a.S + (int64_t)(r / a.n + H) * a.S + (r % a.n + H);
+}
+
+// grid z = 1: a thread takes the node's four fields; 4: one of them
+__global__ __launch_bounds__(RT) void remap_kernel(RemapArgs a) {
+  const int64_t nown = (int64_t)10 * a.n * a.n;
+  const int64_t tid = (int64_t)blockIdx.x * RT + threadIdx.x;
+  const int f0 = blockIdx.z, f1 = gridDim.z == 1 ? 4 : f0 + 1;
+  if (tid >= (f0 == 0 ? nown + 2 : nown)) return;
+  remap_fields(a, blockIdx.y, column_cell(a, tid), f0, tid >= nown ? 1 : f1);  // no velocities at the poles
+}
+
+// ---------------------------------------------------------------------------
+// remapPPR as one sweep of the column, for four layers and more: a lane holds a
+// column of one field and slides the four cells that an edge value needs along
+// in registers; each old cell's parabola is integrated over the new cells that
+// it overlaps as soon as it is formed.  A first sweep takes the surface height
+// and the spacings' sum and extremes (whether the column is uniform) and parks
+// the field's values in LDS, since the new ones are stored over them.  Same
+// operations in the same order as remap_ppr, divisions by a repeated divisor
+// through its reciprocal; a column whose old or new interfaces do not increase
+// (or are not numbers) goes to remap_ppr itself.
+// Bound by FP64 operations (about 600 an old cell and field, the 4 x 4 fits
+// first).  J8 L30: the whole call 6.03 -> 1.70 ms.
+// ---------------------------------------------------------------------------
+struct PprEdge {  // a fit's right-hand side and spacings: cells j, j + 1, ...
+  double h[4], f[4];
+};
+
+// edge value between the second and third cell: the cubic through four means
+__device__ __forceinline__ double ppr_interior(const PprEdge& q, bool uni, double dmin) {
+  const double* f = q.f;
+  if (uni) return (-(1.0 * f[0]) + 7.0 * f[1] + 7.0 * f[2] - 1.0 * f[3]) / 12.0;
+  const double* h = q.h;
+  const double xhat = 0.5 * fmax(h[1], dmin) + 0.5 * fmax(h[2], dmin), rx = 1.0 / xhat;
+  const double s[5] = {div_by(-(h[0] + h[1]), xhat, rx), div_by(-h[1], xhat, rx), 0.0, div_by(h[2], xhat, rx),
+                       div_by(h[2] + h[3], xhat, rx)};
+  constexpr double third = 1.0 / 3.0;
+  double iv[5][4];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    iv[k][0] = s[k];
+    iv[k][1] = pw2(s[k]) / 2.0;
+    iv[k][2] = div_by(pw3(s[k]), 3.0, third);
+    iv[k][3] = pw4(s[k]) / 4.0;
+  }
+  double A[4][4], v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) A[r][p] = iv[r + 1][p] - iv[r][p];
+    v[r] = div_by(h[r] * f[r], xhat, rx);
+  }
+  return solve4_first(A, v, 1.0e-14 * dmin) ? v[0] : f[1] * 0.5 + f[2] * 0.5;
+}
+
+// the loose end fit's three edge values (end_fit) of cells 0..2 of q
+__device__ __forceinline__ void ppr_end(bool low, const PprEdge& q, double dmin, double e[3]) {
+  const double h0 = q.h[0], h1 = q.h[1], h2 = q.h[2];
+  const double xhat = fmax(h1, dmin) * 0.5;
+  const double s[4] = {-(h0 + h1 * 0.5) / xhat, -1.0, 1.0, (h2 + h1 * 0.5) / xhat};
+  double A[3][3], v[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    A[r][0] = s[r + 1] / 1.0 - s[r] / 1.0;
+    A[r][1] = pw2(s[r + 1]) / 2.0 - pw2(s[r]) / 2.0;
+    A[r][2] = pw3(s[r + 1]) / 3.0 - pw3(s[r]) / 3.0;
+    v[r] = q.h[r] * q.f[r] / xhat;
+  }
+  if (solve3(A, v, 1.0e-14 * dmin)) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const double x = low ? s[k] : s[k + 1];
+      e[k] = 1.0 * v[0] + (x * 1.0) * v[1] + (pw2(x) * 1.0) * v[2];
+    }
+  } else {
+    e[0] = low ? q.f[0] * 1.0 : q.f[0] * 0.5 + q.f[1] * 0.5;
+    e[1] = low ? q.f[0] * 0.5 + q.f[1] * 0.5 : q.f[1] * 0.5 + q.f[2] * 0.5;
+    e[2] = low ? q.f[1] * 0.5 + q.f[2] * 0.5 : q.f[2] * 1.0;
+  }
+}
+
+__global__ __launch_bounds__(RT, 2) void remap_ppr_kernel(RemapArgs a, int ncb) {
+  extern __shared__ double lds[];  // a, b [L + 1] each, then the old values [L][64]
+  const int L = a.L, lane = threadIdx.x;
+  double *av = lds, *bv = lds + L + 1, *fo = lds + 2 * (L + 1) + lane;
+  for (int i = lane; i <= L; i += RT) {
+    av[i] = a.a[i];
+    bv[i] = a.b[i];
+  }
+  __syncthreads();
+  // consecutive blocks lie on different XCDs: an XCD takes a run of column
+  // blocks, the four fields of one after another
+  const int per = ncb / 8, id = blockIdx.x;
+  const int field = (id / 8) % 4, cb = (id % 8) * per + id / 32;
+  const int64_t nown = (int64_t)10 * a.n * a.n, tid = (int64_t)cb * RT + lane;
+  if (tid >= (field == 0 ? nown + 2 : nown)) return;
+  const int64_t NC = a.NC, mb = blockIdx.y, s1 = mb * L * NC;
+  const int64_t c = column_cell(a, tid);
+  const int64_t nb = field == 0 ? c : field == 1 ? c + 1 : field == 2 ? c + a.S + 1 : c + a.S;
+  const bool edge = field > 0;
+  const double *mc = a.mold + s1 + c, *mn = a.mold + s1 + nb;
+  double* const v = edge ? a.u + 3 * s1 + (field - 1) * NC + c : a.t + s1 + c;
+  const int64_t vs = edge ? 3 * NC : NC;
+  const double rho = a.rho0 * 1.0, rrho = 1.0 / rho;
+  const double zs0 = a.topo[mb * NC + c], zs1 = a.topo[mb * NC + nb];
+
+  // first sweep
+  double z0 = zs0, z1 = zs1;
+  const double xlo = edge ? 0.5 * (z0 + z1) : z0;
+  double x = xlo, sum = 0.0, hmin = INFINITY, hmax = -INFINITY, first = 0.0;
+  constexpr int CH = 5;
+  for (int k0 = 0; k0 < L; k0 += CH) {
+    double m0[CH], m1[CH], f[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = min(k0 + j, L - 1);
+      m0[j] = mc[k * NC];
+      m1[j] = mn[k * NC];
+      f[j] = v[k * vs];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int k = k0 + j;
+      if (k < L) {
+        z0 = z0 + div_by(0.0 + m0[j], rho, rrho);
+        z1 = z1 + div_by(0.0 + m1[j], rho, rrho);
+        const double xn = edge ? 0.5 * (z0 + z1) : z0, h = xn - x;
+        x = xn;
+        if (k == 0) first = h;
+        sum = k == 0 ? h : sum + h;
+        hmin = fmin(hmin, h);
+        hmax = fmax(hmax, h);
+        fo[k * RT] = edge ? f[j] : (0.0 + f[j]) / (0.0 + m0[j]);
+      }
+    }
+  }
+  const double eta0 = z0, eta1 = z1, xhi = x;
+  auto target = [&](int k) {
+    const double p = av[k] * eta0 + bv[k] * zs0;
+    return edge ? 0.5 * (p + (av[k] * eta1 + bv[k] * zs1)) : p;
+  };
+  bool rising = hmin > 0.0 && hmax < INFINITY && sum < INFINITY;
+  double xn0 = target(0);
+  {
+    double p = xn0;
+    for (int k = 1; k <= L; ++k) {
+      const double q = target(k);
+      rising = rising && q > p;
+      p = q;
+    }
+  }
+  if (!rising) {
+    remap_fields(a, mb, c, field, field + 1);
+    return;
+  }
+  // rmap1d: evenly spaced to 1e-14 keeps one spacing (the rounded distance from
+  // the mean is largest at the smallest or the largest spacing)
+  const double same = (xhi - xlo) / L, xtol = same * 1.0e-14;
+  const bool uni = !(fabs(hmin - same) > xtol) && !(fabs(hmax - same) > xtol);
+  const double dmin = 1.0e-14 * (uni ? first : sum / L);
+
+  // second sweep: h, f of cells i - 1 .. i + 2, x(i), x(i + 1)
+  z0 = zs0;
+  z1 = zs1;
+  double pm0 = mc[0], pm1 = mn[0];
+  double xt = xlo;  // interface below the next cell to enter
+  int kin = 0;
+  auto enter = [&]() {  // spacing of cell kin + 1; the next one's masses are loaded ahead
+    z0 = z0 + div_by(0.0 + pm0, rho, rrho);
+    z1 = z1 + div_by(0.0 + pm1, rho, rrho);
+    const double xn = edge ? 0.5 * (z0 + z1) : z0, h = xn - xt;
+    xt = xn;
+    kin = min(kin + 1, L - 1);
+    pm0 = mc[kin * NC];
+    pm1 = mn[kin * NC];
+    return h;
+  };
+  PprEdge q;
+  double xa = xlo, xb, xc, xd;  // x(i) .. x(i + 3)
+  q.h[0] = 0.0;
+  q.f[0] = 0.0;
+  q.h[1] = enter();
+  xb = xt;
+  q.h[2] = enter();
+  xc = xt;
+  q.h[3] = enter();
+  xd = xt;
+  q.f[1] = fo[0];
+  q.f[2] = fo[RT];
+  q.f[3] = fo[2 * RT];
+  double e[3];
+  {
+    const double hu = uni ? q.h[1] : 0.0;
+    const PprEdge b = {{uni ? hu : q.h[1], uni ? hu : q.h[2], uni ? hu : q.h[3], 0.0}, {q.f[1], q.f[2], q.f[3], 0.0}};
+    ppr_end(true, b, dmin, e);
+  }
+  double el_ = e[0], elow = e[1], ehigh = 0.0;
+  double acc = 0.0, xn1 = target(1), fmn = 0.0, fmx = 0.0, dmn = 0.0, dmx = 0.0;
+  int k = 0, kmin = 0, kmax = 0;  // new cell k + 1
+  double so = 0.0, eo = 0.0, sn = 0.0, en = 0.0;
+  auto finish = [&]() {  // new cell k + 1
+    const double dz = xn1 - xn0, fnew = acc / fmax(dz, xtol);
+    if (k == 0) {
+      fmn = fmx = fnew;
+      dmn = dmx = dz;
+    } else if (fnew > fmx) {
+      kmax = k;
+      fmx = fnew;
+      dmx = dz;
+    } else if (fnew < fmn) {
+      kmin = k;
+      fmn = fnew;
+      dmn = dz;
+    }
+    const double b = dz * fnew, tt = sn + b;
+    en = fabs(sn) >= fabs(b) ? en + ((sn - tt) + b) : en + ((b - tt) + sn);
+    sn = tt;
+    if (edge) {
+      v[k * vs] = fnew;
+    } else {
+      const double rho_dz = rho * dz;
+      a.m[s1 + k * NC + c] = rho_dz - 0.0;
+      v[k * vs] = rho_dz * fnew - 0.0;
+    }
+    acc = 0.0;
+    ++k;
+    xn0 = xn1;
+    xn1 = target(min(k + 1, L));
+  };
+  for (int i = 1; i <= L; ++i) {
+    const double f0 = q.f[1], h0 = q.h[1];
+    const double fl = i > 1 ? q.f[0] : f0, fr = i < L ? q.f[2] : f0;
+    const double hl = i > 1 ? q.h[0] : h0, hr = i < L ? q.h[2] : h0;
+    // the cell's upper edge
+    double er;
+    if (i == 1) {
+      er = elow;
+    } else if (i <= L - 2) {
+      er = ppr_interior(q, uni, dmin);
+    } else if (i == L - 1) {
+      const PprEdge b = {{uni ? first : q.h[0], uni ? first : q.h[1], uni ? first : q.h[2], 0.0},
+                         {q.f[0], q.f[1], q.f[2], 0.0}};
+      ppr_end(false, b, dmin, e);
+      er = e[1];
+      ehigh = e[2];
+    } else {
+      er = ehigh;
+    }
+    double el = el_;
+    el_ = er;
+    // plsv / plsc: the limited centred slope
+    double d0 = 0.0;
+    const double dm = f0 - fl, dp = fr - f0;
+    if (dm * dp > 0.0) {
+      double sl, sr;
+      if (uni) {
+        sl = (fl + f0) * 0.5;
+        sr = (f0 + fr) * 0.5;
+      } else {
+        sl = (h0 * fl + hl * f0) / (hl + h0);
+        sr = (hr * f0 + h0 * fr) / (h0 + hr);
+      }
+      d0 = 0.5 * (sr - sl);
+      d0 = fmin(fmin(fabs(dm), fabs(dp)) / fmax(fabs(d0), 1.0e-14), 1.0) * d0;
+    }
+    double u0, u1, u2, l0, l1, l2;
+    parabola(f0, el, er, u0, u1, u2);
+    if ((fr - f0) * (f0 - fl) < 0.0) {
+      l0 = f0; l1 = 0.0; l2 = 0.0;
+    } else {
+      if ((fl - el) * (el - f0) <= 0.0) el = f0 - d0;
+      if ((fr - er) * (er - f0) <= 0.0) er = f0 + d0;
+      parabola(f0, el, er, l0, l1, l2);
+      if (fabs(l2) > fabs(l1) * 0.5) {
+        const double turn = -0.5 * l1 / l2;
+        if (turn >= -1.0 && turn <= 0.0) {
+          er = 3.0 * f0 - 2.0 * el;
+          parabola(f0, el, er, l0, l1, l2);
+        } else if (turn > 0.0 && turn <= 1.0) {
+          el = 3.0 * f0 - 2.0 * er;
+          parabola(f0, el, er, l0, l1, l2);
+        }
+      }
+    }
+    const double c0 = 0.0 * u0 + 1.0 * l0, c1 = 0.0 * u1 + 1.0 * l1, c2 = 0.0 * u2 + 1.0 * l2;
+    {  // compensated sum of the old column's content
+      const double b = h0 * f0, tt = so + b;
+      eo = fabs(so) >= fabs(b) ? eo + ((so - tt) + b) : eo + ((b - tt) + so);
+      so = tt;
+    }
+    // imap1d: the cell's share of the new cells that it overlaps
+    const double mid = xb * 0.5 + xa * 0.5, half = xb * 0.5 - xa * 0.5, hx = fmax(half, xtol), rh = 1.0 / hx;
+    constexpr double third = 1.0 / 3.0;
+    while (k < L && xb > xn0) {
+      if (xa < xn1) {
+        const double lo = fmax(xa, xn0), hi = fmin(xb, xn1);
+        const double sl = div_by(lo - mid, hx, rh), sh = div_by(hi - mid, hx, rh);
+        const double w0 = sh - sl, w1 = pw2(sh) / 2.0 - pw2(sl) / 2.0;
+        const double w2 = div_by(pw3(sh), 3.0, third) - div_by(pw3(sl), 3.0, third);
+        double in = w0 * c0 + w1 * c1 + w2 * c2;
+        in = in * half;
+        acc = acc + in;
+      }
+      if (!(xb >= xn1)) break;
+      finish();
+    }
+    // slide
+    xa = xb; xb = xc; xc = xd;
+    q.h[0] = q.h[1]; q.h[1] = q.h[2]; q.h[2] = q.h[3];
+    q.f[0] = q.f[1]; q.f[1] = q.f[2]; q.f[2] = q.f[3];
+    if (i + 3 <= L) {
+      q.h[3] = enter();
+      q.f[3] = fo[(i + 2) * RT];
+      xd = xt;
+    }
+  }
+  while (k < L) finish();  // new cells that reach above the old column
+  // the difference of the contents goes to the smallest (deficit) or largest
+  // (excess) new cell
+  const double err = (so + eo) - (sn + en);
+  if (err > 0.0) {
+    const double fnew = fmn + err / dmn;
+    v[kmin * vs] = edge ? fnew : (rho * dmn) * fnew - 0.0;
+  } else if (err < 0.0) {
+    const double fnew = fmx + err / dmx;
+    v[kmax * vs] = edge ? fnew : (rho * dmx) * fnew - 0.0;
   }
 }
 
@@ -780,7 +1129,18 @@ extern "C" int wtg_remap(wtg_ctx* c, int slot, int scheme, const double* a_vert,
   RemapArgs a{c->info.n, c->info.S, L, scheme, NC, c->info.south_pole, c->info.north_pole, c->d_remap_ab,
               c->d_remap_ab + RMAX + 1, c->d_topo, mold, s.m, s.t, s.u, c->params.ref_density};
   const int64_t cols = (int64_t)10 * c->info.n * c->info.n + 2;
-  hipLaunchKernelGGL(remap_kernel, dim3((unsigned)((cols + RT - 1) / RT), (unsigned)M), dim3(RT), 0, c->stream, a);
+  const int ncb = (int)((cols + RT - 1) / RT);
+  if (scheme == WTG_REMAP_PPR && L >= 4) {  // below four layers the edge values are two-point means
+    const int padded = (ncb + 7) / 8 * 8;
+    const size_t lds = (2 * (size_t)(L + 1) + (size_t)L * RT) * sizeof(double);
+    hipLaunchKernelGGL(remap_ppr_kernel, dim3((unsigned)(4 * padded), (unsigned)M), dim3(RT), lds, c->stream, a, padded);
+  } else {
+    // a thread for each field where whole nodes leave compute units without
+    // waves (J5 L6, remap1: 149 -> 78 us a call); at J7 L20 both shapes take
+    // 1.75 ms, remap0 loses 5 % to the node's coordinates formed four times
+    const unsigned split = (int64_t)ncb * M <= 2048 ? 4 : 1;
+    hipLaunchKernelGGL(remap_kernel, dim3((unsigned)ncb, (unsigned)M, split), dim3(RT), 0, c->stream, a);
+  }
   WTG_HIPCHK(c, hipGetLastError());
   if (int rc = wtg_ghost_fill_layers(c, L * M, s.m, s.t, s.u)) return rc;
   WTG_HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "ctx.h"
+#include "exact_div.h"
 
 namespace {
 
@@ -836,15 +837,6 @@ __device__ __forceinline__ void weights_lds(const TileS& s, int y, int offs, dou
   w[3] = -(0.5 - acc3 * hi);
   w[4] = 0.5 - acc4 * hi;
 }
-
-// a / d with r = 1 / d rounded to nearest: one remainder step makes the
-// product the correctly rounded quotient (Markstein, IBM J. Res. Dev. 34,
-// 1990) where nothing over- or underflows; an infinite a gives NaN
-__device__ __forceinline__ double div_by(double a, double d, double r) {
-  const double q = a * r;
-  return __builtin_fma(__builtin_fma(-q, d, a), r, q);
-}
-
 
 // Planes read and written through buffer descriptors: a uniform base, a
 // uniform 32-bit byte offset of the plane and the cell's 32-bit byte offset,
