@@ -151,6 +151,7 @@ struct wtg_ctx {
   wtg_vdiff vd{};
   bool vd_set = false;
   double *vd_kt = nullptr, *vd_kv = nullptr, *vd_tke = nullptr, *vd_force = nullptr;
+  unsigned long long* vd_left = nullptr;  // systems that the register kernels leave, a word per block
 };
 
 extern thread_local std::string g_create_error;

@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include "ctx.h"
+#include "exact_div.h"
 
 namespace {
 
@@ -36,6 +37,7 @@ struct VdArgs {
   const double* force;                          // [members][6][NC]
   double *m, *t, *u;                            // the state slot
   double *kt, *kv, *tke;                        // [members][L + 1][NC], [members][L][NC]
+  unsigned long long* left;                     // lanes that a register kernel leaves, a word per block
 };
 
 // LAPACK dgtsv with one right-hand side on rows 1..n of 1-based arrays.  The
@@ -253,14 +255,10 @@ struct TkeRows {
   }
 };
 
-// turbulent_diffusion of every owned node and pole master
-__global__ __launch_bounds__(VT) void vd_turbulent_kernel(VdArgs a) {
-  const int64_t tid = (int64_t)blockIdx.x * VT + threadIdx.x;
-  if (tid >= (int64_t)10 * a.n * a.n + 2) return;
-  bool pole;
-  const int64_t c = column(a, tid, pole);
+// turbulent_diffusion of one column in private arrays
+__device__ __forceinline__ void turbulent_column(const VdArgs& a, int64_t mb, int64_t c) {
   const int L = a.L;
-  const int64_t NC = a.NC, mb = blockIdx.y;
+  const int64_t NC = a.NC;
   const double* m = a.m + mb * L * NC;
   const double* t = a.t + mb * L * NC;
   const double* u = a.u + mb * 3 * L * NC;
@@ -340,6 +338,209 @@ __global__ __launch_bounds__(VT) void vd_turbulent_kernel(VdArgs a) {
   for (int l = 1; l <= L; ++l) tke[(int64_t)(l - 1) * NC + c] = fmax(w.e[l], p.e_min);
 }
 
+// turbulent_diffusion of every owned node and pole master: the analytic
+// profiles, and the TKE closure for any number of layers
+__global__ __launch_bounds__(VT) void vd_turbulent_kernel(VdArgs a) {
+  const int64_t tid = (int64_t)blockIdx.x * VT + threadIdx.x;
+  if (tid >= (int64_t)10 * a.n * a.n + 2) return;
+  bool pole;
+  turbulent_column(a, blockIdx.y, column(a, tid, pole));
+}
+
+// the columns that vd_tke_kernel left (a thread looks at a block's word)
+__global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) {
+  const int id = blockIdx.x * VT + threadIdx.x;
+  if (id >= nblocks) return;
+  for (unsigned long long w = a.left[(int64_t)blockIdx.y * nblocks + id]; w; w &= w - 1) {
+    bool pole;
+    turbulent_column(a, blockIdx.y, column(a, (int64_t)id * VT + __builtin_ctzll(w), pole));
+  }
+}
+
+// The TKE closure for at most LM layers (and istep > 1, whose coefficients are
+// known before the rows), the column in registers: the loops over levels are
+// unrolled and run in four sweeps,
+//   down  the length from the surface,
+//   up    the length from the bottom, the rows and their elimination,
+//   down  the back substitution and the new length from the surface,
+//   up    the new length from the bottom and the coefficients,
+// with dUdZ^2, N^2, one length or pivot and the right-hand side per level kept
+// between them.  Same operations as turbulent_column, to which a system that
+// dgtsv would pivot is left (vd_tke_left_kernel).  Bound by the latency of its divisions and square roots at
+// one or two waves per SIMD.  J8 L30: TKE_FIGURES
+template <int LM>
+__global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
+  const int64_t tid = (int64_t)blockIdx.x * VT + threadIdx.x;
+  const bool live = tid < (int64_t)10 * a.n * a.n + 2;
+  bool pole;
+  const int64_t c = column(a, live ? tid : 0, pole);
+  const int L = a.L;
+  const int64_t NC = a.NC, mb = blockIdx.y;
+  const double* m = a.m + mb * L * NC + c;
+  const double* t = a.t + mb * L * NC + c;
+  const double* u = a.u + mb * 3 * L * NC;
+  double* kt = a.kt + mb * (L + 1) * NC + c;
+  double* kv = a.kv + mb * (L + 1) * NC + c;
+  double* tke = a.tke + mb * L * NC + c;
+  const double tau = a.force[(mb * 6 + 2) * NC + c];
+  const wtg_vdiff& p = a.p;
+  const double rho = a.rho0 * 1.0, rrho = 1.0 / rho, dt = a.dt;
+  const int64_t W = c - 1, SW = c - a.S - 1, Sx = c - a.S;
+  // dUdZ^2 and N^2 at the interfaces 1 .. L - 1
+  double dU2[LM], Nsq[LM], A[LM + 1], X[LM];
+  {
+    const double l0 = a.len[c], l1 = a.len[NC + c], l2 = a.len[2 * NC + c], p0 = a.ped[c], p1 = a.ped[NC + c];
+    const double p2 = a.ped[2 * NC + c], lS = a.len[2 * NC + Sx], pS = a.ped[2 * NC + Sx], lSW = a.len[NC + SW];
+    const double pSW = a.ped[NC + SW], lW = a.len[W], pW = a.ped[W], hi = a.hinv[c];
+    double umag = 0.0, dzp = 0.0, bp = 0.0;
+    constexpr int CH = 4;
+#pragma unroll
+    for (int k0 = 0; k0 < LM; k0 += CH) {
+      if (k0 < L) {
+        double v[CH][6], mm[CH], tt[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+          const int64_t k = min(k0 + j, L - 1);
+          const double* uk = u + 3 * k * NC;
+          v[j][0] = uk[c];
+          v[j][1] = uk[NC + c];
+          v[j][2] = uk[2 * NC + c];
+          v[j][3] = uk[2 * NC + Sx];
+          v[j][4] = uk[NC + SW];
+          v[j][5] = uk[W];
+          mm[j] = m[k * NC];
+          tt[j] = t[k * NC];
+        }
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+          const int k = k0 + j;
+          const double dz = div_by(0.0 + mm[j], rho, rrho);
+          const double pRT = v[j][0] * l0, pDG = v[j][1] * l1, pUP = v[j][2] * l2;
+          const double dRT = v[j][0] * p0, dDG = v[j][1] * p1, dUP = v[j][2] * p2;
+          const double pUPS = v[j][3] * lS, pDGSW = v[j][4] * lSW, pRTW = v[j][5] * lW;
+          const double dRTW = v[j][5] * pW, dDGSW = v[j][4] * pSW, dUPS = v[j][3] * pS;
+          const double ke =
+              (pUP * dUP + pDG * dDG + pRT * dRT + pUPS * dUPS + pDGSW * dDGSW + pRTW * dRTW) * hi / 4.0;
+          const double um = sqrt(2.0 * ke), b = tt[j] / (0.0 + mm[j]);
+          if (k >= 1) {
+            const double dzm = 0.5 * (dzp + dz), rz = 1.0 / dzm, q = div_by(um - umag, dzm, rz);
+            dU2[k - 1] = q * q;
+            Nsq[k - 1] = div_by(a.grav * (b - bp), dzm, rz);
+          }
+          umag = um;
+          dzp = dz;
+          bp = b;
+        }
+      }
+    }
+  }
+#define DZ(k) div_by(0.0 + m[(int64_t)((k) - 1) * NC], rho, rrho)
+#define E_OLD(l) fmax(tke[(int64_t)((l) - 1) * NC], p.e_min)
+#define FIRST(e, nsq) sqrt(2.0 * (e) / fmax(nsq, p.Neps_sq))
+  // interface l has dU2[l - 1], Nsq[l - 1]; the ends take their neighbours' N^2
+  const double up_top = fmax(p.l_0, p.kappa_VK * p.C_l / (a.rho0 * a.grav) * tau);
+  {
+    double prev = up_top;
+#pragma unroll
+    for (int l = LM - 1; l >= 1; --l)
+      if (l < L) {
+        prev = fmin(FIRST(E_OLD(l), Nsq[l - 1]), prev + DZ(l + 1));
+        A[l] = prev;
+      }
+  }
+  bool fast = true;
+  double di = 0.0, xi = 0.0, ui = 0.0;
+  {
+    double dn = p.l_0, dzc = DZ(1), Kvp = 0.0, Kvc = kv[NC];
+#pragma unroll
+    for (int l = 1; l < LM; ++l)
+      if (l < L) {
+        const double KT = kt[(int64_t)l * NC], KV = Kvc, Kvn = kv[(int64_t)(l + 1) * NC];
+        const double e = E_OLD(l), dzn = DZ(l + 1), N2 = Nsq[l - 1], U2 = dU2[l - 1];
+        dn = fmin(FIRST(e, N2), dn + dzc);
+        const double leps = fmax(p.l_min, sqrt(A[l] * dn));
+        const double turb = e == 0.0 ? 0.0 : p.C_eps * sqrt(e) / leps;
+        double S1 = KV * U2 - KT * N2, S2;
+        if (p.patankar && S1 <= 0.0) {
+          S1 = KV * U2;
+          S2 = -turb - KT * N2 / e;
+        } else {
+          S2 = -turb;
+        }
+        const double dzl = 0.5 * (dzc + dzn);
+        const double up = l <= L - 2 ? -(dt * p.C_e * (0.5 * (KV + Kvn)) / (dzl * dzn)) : 0.0;
+        const double lo = l >= 2 ? -(dt * p.C_e * (0.5 * (KV + Kvp)) / (dzl * dzc)) : 0.0;
+        const double dg = 1.0 - (up + lo) - dt * S2, r = e + dt * S1;
+        if (l == 1) {
+          di = dg;
+          xi = r;
+        } else {
+          fast = fast && fabs(di) >= fabs(lo) && di != 0.0;
+          const double fact = lo / di;
+          di = dg - fact * ui;
+          xi = r - fact * xi;
+        }
+        ui = up;
+        A[l] = di;
+        X[l] = xi;
+        Kvp = KV;
+        Kvc = Kvn;
+        dzc = dzn;
+      }
+    fast = fast && di != 0.0;
+  }
+  const unsigned long long left = __ballot(!fast && live);
+  if (threadIdx.x == 0) a.left[mb * gridDim.x + blockIdx.x] = left;
+  if (!fast || !live) return;
+  const double e_top = fmax(p.C_srf * tau / a.rho0, p.e_min_srf);
+  {
+    double x1 = 0.0, x2 = 0.0, prev = up_top, dzn = DZ(L), Kvn = 0.0;
+#pragma unroll
+    for (int l = LM - 1; l >= 1; --l)
+      if (l < L) {
+        const double dzc = DZ(l), KV = kv[(int64_t)l * NC];
+        double x;
+        if (l == L - 1) {
+          x = X[l] / A[l];
+        } else {  // the super-diagonal again, as the rows have it
+          const double up = -(dt * p.C_e * (0.5 * (KV + Kvn)) / (0.5 * (dzc + dzn) * dzn));
+          x = (X[l] - up * x1 - 0.0 * x2) / A[l];
+        }
+        x2 = l == L - 1 ? 0.0 : x1;
+        x1 = x;
+        const double e = p.patankar ? x : fmax(x, p.e_min);
+        X[l] = e;
+        prev = fmin(FIRST(e, Nsq[l - 1]), prev + dzn);
+        A[l] = prev;
+        dzn = dzc;
+        Kvn = KV;
+      }
+    A[0] = fmin(FIRST(p.e_0, Nsq[0]), prev + dzn);
+  }
+  {  // update_Kv_Kt
+    auto store = [&](int l, double e, double n2, double u2, double up, double dn) {
+      const double Ri = n2 / (u2 + p.eps_s), v = kv_tke(p, e, fmax(p.l_min, fmin(up, dn)));
+      kv[(int64_t)l * NC] = v;
+      kt[(int64_t)l * NC] = kt_tke(p, v, n2, Ri);
+      if (l >= 1) tke[(int64_t)(l - 1) * NC] = fmax(e, p.e_min);
+    };
+    double dn = p.l_0, n2 = Nsq[0];
+    store(0, p.e_0, n2, 0.0, A[0], dn);
+#pragma unroll
+    for (int l = 1; l < LM; ++l)
+      if (l < L) {
+        n2 = Nsq[l - 1];
+        dn = fmin(FIRST(X[l], n2), dn + DZ(l));
+        store(l, X[l], n2, dU2[l - 1], A[l], dn);
+      }
+    dn = fmin(FIRST(e_top, n2), dn + DZ(L));
+    store(L, e_top, n2, 0.0, up_top, dn);
+  }
+#undef DZ
+#undef E_OLD
+#undef FIRST
+}
+
 __device__ __forceinline__ double irradiance(const wtg_vdiff& p, double depth) {
   return p.Q_sr * (0.58 * exp(-depth / 0.35) + (1.0 - 0.58) * exp(-depth / 23.0));
 }
@@ -411,6 +612,51 @@ struct Rows {
   }
 };
 
+// One system of a column in private arrays: the buoyancy (e = -1) or the
+// velocity of the RT, DG or UP edge (0..2)
+__device__ void solve_column(const VdArgs& a, int64_t mb, int64_t c, int e, double eta, SolveWork& w) {
+  const int L = a.L;
+  const int64_t NC = a.NC;
+  const double* m = a.m + mb * L * NC;
+  double* t = a.t + mb * L * NC;
+  double* u = a.u + mb * 3 * L * NC;
+  const double* f = a.force + mb * 6 * NC;
+  const double zs = a.topo[mb * NC + c];
+  const bool edge = e >= 0;
+  const int64_t nb = e == 0 ? c + 1 : e == 1 ? c + a.S + 1 : e == 2 ? c + a.S : c;
+  Rows rows{a, m, t, u, (edge ? a.kv : a.kt) + mb * (L + 1) * NC, f, c, nb, e, eta, a.dt};
+  solve_rows(L, rows, zs, w);
+  for (int k = 1; k <= L; ++k) {
+    const int64_t x = (int64_t)(k - 1) * NC + c;
+    if (edge)
+      u[((int64_t)(k - 1) * 3 + e) * NC + c] = w.X[k];
+    else
+      t[x] = (0.0 + m[x]) * w.X[k];
+  }
+}
+
+// One system of a column in private arrays: the buoyancy (e = -1) or the
+// velocity of the RT, DG or UP edge (0..2)
+__device__ void solve_column(const VdArgs& a, int64_t mb, int64_t c, int e, double eta) {
+  const int L = a.L;
+  const int64_t NC = a.NC;
+  const double* m = a.m + mb * L * NC;
+  double* t = a.t + mb * L * NC;
+  double* u = a.u + mb * 3 * L * NC;
+  const bool edge = e >= 0;
+  const int64_t nb = e == 0 ? c + 1 : e == 1 ? c + a.S + 1 : e == 2 ? c + a.S : c;
+  SolveWork w;
+  Rows rows{a, m, t, u, (edge ? a.kv : a.kt) + mb * (L + 1) * NC, a.force + mb * 6 * NC, c, nb, e, eta, a.dt};
+  solve_rows(L, rows, a.topo[mb * NC + c], w);
+  for (int k = 1; k <= L; ++k) {
+    const int64_t x = (int64_t)(k - 1) * NC + c;
+    if (edge)
+      u[((int64_t)(k - 1) * 3 + e) * NC + c] = w.X[k];
+    else
+      t[x] = (0.0 + m[x]) * w.X[k];
+  }
+}
+
 // backwards_euler_temp of every owned node and pole master, then
 // backwards_euler_velo of the owned nodes' edges
 __global__ __launch_bounds__(VT) void vd_solve_kernel(VdArgs a) {
@@ -439,6 +685,137 @@ __global__ __launch_bounds__(VT) void vd_solve_kernel(VdArgs a) {
     Rows ru{a, m, t, u, a.kv + mb * (L + 1) * NC, f, c, nb[e], e, eta, a.dt};
     solve_rows(L, ru, zs, w);
     for (int k = 1; k <= L; ++k) u[((int64_t)(k - 1) * 3 + e) * NC + c] = w.X[k];
+  }
+}
+
+// The same for at most LM layers, a lane one system: the elimination's
+// diagonal, super-diagonal and right-hand side stay in registers (the loops
+// over layers are unrolled), so that the state's own bytes are what moves.
+// Rows without a solar flux; a system that dgtsv would pivot, one with a solar
+// flux and a column with a thickness that is not positive are left to
+// vd_solve_left_kernel (a call from here would cost the arrays their registers).
+// Bound by memory latency at two waves per SIMD (three arrays of 32 doubles are
+// 192 registers).  J8 L30: SOLVE_FIGURES; with the arrays in LDS (three waves
+// per compute unit) 1.6 ms.
+template <int LM>
+__global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArgs a, int ncb) {
+  const int L = a.L;
+  // consecutive blocks lie on different XCDs: an XCD takes a run of column
+  // blocks, the four systems of one after another
+  const int per = ncb / 8, id = blockIdx.x, e = (id / 8) % 4 - 1, cb = (id % 8) * per + id / 32;
+  const bool edge = e >= 0;
+  const int64_t nown = (int64_t)10 * a.n * a.n, tid = (int64_t)cb * VT + threadIdx.x;
+  const bool live = tid < (edge ? nown : nown + 2);  // the poles carry no edges of their own
+  bool pole;
+  const int64_t c = column(a, live ? tid : 0, pole);
+  const int64_t NC = a.NC, mb = blockIdx.y;
+  const double* m = a.m + mb * L * NC;
+  const double* f = a.force + mb * 6 * NC + c;
+  const double* K = (edge ? a.kv : a.kt) + mb * (L + 1) * NC + c;
+  const int64_t nb = e == 0 ? c + 1 : e == 1 ? c + a.S + 1 : e == 2 ? c + a.S : c;
+  double* const v = edge ? a.u + (mb * 3 * L + e) * NC + c : a.t + mb * L * NC + c;
+  const int64_t vs = edge ? 3 * NC : NC;
+  const double rho = a.rho0 * 1.0, rrho = 1.0 / rho, dt = a.dt;
+  const wtg_vdiff& p = a.p;
+  // thickness, coefficient at the upper interface and value of every layer;
+  // they become the elimination's super-diagonal, diagonal and right-hand side
+  double U[LM], D[LM], X[LM];
+  double least = INFINITY;
+  constexpr int CH = 4;
+#pragma unroll
+  for (int k0 = 0; k0 < LM; k0 += CH) {
+    if (k0 < L) {
+      double m0[CH], m1[CH];
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        const int64_t k = min(k0 + j, L - 1);
+        m0[j] = m[k * NC + c];
+        m1[j] = m[k * NC + nb];
+        D[k0 + j] = K[(k + 1) * NC];
+        X[k0 + j] = v[k * vs];
+      }
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        const double z = div_by(0.0 + m0[j], rho, rrho);
+        U[k0 + j] = edge ? 0.5 * (z + div_by(0.0 + m1[j], rho, rrho)) : z;
+        least = U[k0 + j] > 0.0 ? least : -1.0;
+        if (!edge) X[k0 + j] = X[k0 + j] / (0.0 + m0[j]);
+      }
+    }
+  }
+  bool fast = least > 0.0 && (edge || p.Q_sr == 0.0);
+  if (fast) {
+    const double bot = edge ? 0.0 : f[0], top = edge ? f[(3 + e) * NC] : f[NC];
+    double di = 0.0, xi = 0.0, ui = 0.0, Kp = 0.0, dzp = 0.0;
+#pragma unroll
+    for (int k = 0; k < LM; ++k) {
+      if (k < L) {
+        const bool last = k == L - 1;
+        const double dz = U[k], dzn = k + 1 < LM && !last ? U[k + 1 < LM ? k + 1 : k] : 0.0, Kc = D[k];
+        const double lo = k > 0 ? -(dt * Kp / (0.5 * (dzp + dz) * dz)) : 0.0;
+        const double up = last ? 0.0 : -(dt * Kc / (0.5 * (dz + dzn) * dz));
+        double dg = 1.0 - (up + lo), r = X[k];
+        if (edge) {
+          if (k == 0) dg = dg + dt * p.bottom_friction / dz;
+          if (last) r = r + dt * top / dz;
+        } else {
+          if (k == 0) r = r + dt * (-bot + 0.0) / dz;
+          if (last) {
+            // the reference's top row takes the row below's super-diagonal entry
+            dg = 1.0 - (-(dt * Kp / (0.5 * (dzp + dz) * dzp)));
+            r = X[k] + dt * (top + p.Q_sr / (a.rho0 * p.c_p)) / dz;
+          }
+        }
+        if (k == 0) {
+          di = dg;
+          xi = r;
+        } else {
+          fast = fast && fabs(di) >= fabs(lo) && di != 0.0;
+          const double fact = lo / di;
+          di = dg - fact * ui;
+          xi = r - fact * xi;
+        }
+        ui = up;
+        D[k] = di;
+        X[k] = xi;
+        U[k] = up;
+        Kp = Kc;
+        dzp = dz;
+      }
+    }
+    fast = fast && di != 0.0;
+    if (fast) {
+      double x1 = 0.0, x2 = 0.0;
+#pragma unroll
+      for (int k = LM - 1; k >= 0; --k) {
+        if (k < L) {
+          const double x = k == L - 1 ? X[k] / D[k] : (X[k] - U[k] * x1 - 0.0 * x2) / D[k];
+          x2 = k == L - 1 ? 0.0 : x1;
+          x1 = x;
+          X[k] = x;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < LM; ++k)
+        if (k < L && live) v[k * vs] = edge ? X[k] : (0.0 + m[k * NC + c]) * X[k];
+    }
+  }
+  const unsigned long long left = __ballot(!fast && live);
+  if (threadIdx.x == 0) a.left[mb * gridDim.x + id] = left;
+}
+
+// the systems that vd_solve_reg_kernel left (a thread looks at a block's word)
+__global__ __launch_bounds__(VT) void vd_solve_left_kernel(VdArgs a, int ncb) {
+  const int id = blockIdx.x * VT + threadIdx.x;
+  if (id >= 4 * ncb) return;
+  const int64_t mb = blockIdx.y, NC = a.NC;
+  const int per = ncb / 8, e = (id / 8) % 4 - 1, cb = (id % 8) * per + id / 32;
+  for (unsigned long long w = a.left[mb * 4 * ncb + id]; w; w &= w - 1) {
+    bool pole;
+    const int64_t c = column(a, (int64_t)cb * VT + __builtin_ctzll(w), pole);
+    const double zs = a.topo[mb * NC + c];
+    const double eta = e >= 0 ? 0.0 : a.eta ? a.eta[mb * NC + c] : free_surface(a, a.m + mb * a.L * NC, zs, c);
+    solve_column(a, mb, c, e, eta);
   }
 }
 
@@ -485,6 +862,8 @@ extern "C" int wtg_set_vdiff(wtg_ctx* c, const wtg_vdiff* p) {
     if (int rc = wtg_dalloc<double>(c, &c->vd_kv, (size_t)M * (L + 1) * NC)) return rc;
     if (int rc = wtg_dalloc<double>(c, &c->vd_tke, (size_t)M * L * NC)) return rc;
     if (int rc = wtg_dalloc<double>(c, &c->vd_force, (size_t)M * 6 * NC)) return rc;
+    const size_t nblk = ((size_t)10 * c->info.n * c->info.n + 2 + VT - 1) / VT;
+    if (int rc = wtg_dalloc<unsigned long long>(c, &c->vd_left, (size_t)M * 4 * ((nblk + 7) / 8 * 8))) return rc;
     WTG_HIPCHK(c, hipMemsetAsync(c->vd_kt, 0, (size_t)M * (L + 1) * NC * sizeof(double), c->stream));
     WTG_HIPCHK(c, hipMemsetAsync(c->vd_kv, 0, (size_t)M * (L + 1) * NC * sizeof(double), c->stream));
     WTG_HIPCHK(c, hipMemsetAsync(c->vd_tke, 0, (size_t)M * L * NC * sizeof(double), c->stream));
@@ -554,12 +933,39 @@ extern "C" int wtg_vertical_diffusion(wtg_ctx* c, int slot, double dt, int istep
   if (int rc = wtg_ghost_fill_layers(c, L * M, s.m, s.t, s.u)) return rc;
   VdArgs a{c->info.n, c->info.S, L, istep, c->info.ncells, c->info.south_pole, c->info.north_pole, dt,
            c->params.ref_density, c->params.grav, c->vd, c->d_len, c->d_ped, c->d_hinv, c->d_topo, eta, c->vd_force,
-           s.m, s.t, s.u, c->vd_kt, c->vd_kv, c->vd_tke};
+           s.m, s.t, s.u, c->vd_kt, c->vd_kv, c->vd_tke, c->vd_left};
   const int64_t cols = (int64_t)10 * c->info.n * c->info.n + 2;
   const dim3 grid((unsigned)((cols + VT - 1) / VT), (unsigned)M);
-  hipLaunchKernelGGL(vd_turbulent_kernel, grid, dim3(VT), 0, c->stream, a);
+  // the register kernels hold up to 32 layers; above, the private arrays
+  const int nblk = (int)grid.x, ncb = (nblk + 7) / 8 * 8;
+  const dim3 systems((unsigned)(4 * ncb), (unsigned)M);
+  if (!c->vd.tke_closure || istep == 1 || L > 32) {
+    hipLaunchKernelGGL(vd_turbulent_kernel, grid, dim3(VT), 0, c->stream, a);
+  } else {
+    if (L <= 16)
+      hipLaunchKernelGGL(vd_tke_kernel<16>, grid, dim3(VT), 0, c->stream, a);
+    else if (L <= 24)
+      hipLaunchKernelGGL(vd_tke_kernel<24>, grid, dim3(VT), 0, c->stream, a);
+    else
+      hipLaunchKernelGGL(vd_tke_kernel<32>, grid, dim3(VT), 0, c->stream, a);
+    WTG_HIPCHK(c, hipGetLastError());
+    hipLaunchKernelGGL(vd_tke_left_kernel, dim3((unsigned)((nblk + VT - 1) / VT), (unsigned)M), dim3(VT), 0, c->stream,
+                       a, nblk);
+  }
   WTG_HIPCHK(c, hipGetLastError());
-  hipLaunchKernelGGL(vd_solve_kernel, grid, dim3(VT), 0, c->stream, a);
+  if (L > 32) {
+    hipLaunchKernelGGL(vd_solve_kernel, grid, dim3(VT), 0, c->stream, a);
+  } else {
+    if (L <= 16)
+      hipLaunchKernelGGL(vd_solve_reg_kernel<16>, systems, dim3(VT), 0, c->stream, a, ncb);
+    else if (L <= 24)
+      hipLaunchKernelGGL(vd_solve_reg_kernel<24>, systems, dim3(VT), 0, c->stream, a, ncb);
+    else
+      hipLaunchKernelGGL(vd_solve_reg_kernel<32>, systems, dim3(VT), 0, c->stream, a, ncb);
+    WTG_HIPCHK(c, hipGetLastError());
+    hipLaunchKernelGGL(vd_solve_left_kernel, dim3((unsigned)((4 * ncb + VT - 1) / VT), (unsigned)M), dim3(VT), 0,
+                       c->stream, a, ncb);
+  }
   WTG_HIPCHK(c, hipGetLastError());
   if (int rc = wtg_ghost_fill_layers(c, L * M, s.m, s.t, s.u)) return rc;
   WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
