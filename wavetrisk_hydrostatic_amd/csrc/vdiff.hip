@@ -12,11 +12,11 @@
 // so it must finish before any velocity changes.  The second steps the
 // buoyancy of the same columns and the velocities of each owned node's RT,
 // DG and UP edges (with the node's Kv and the layer thicknesses averaged with
-// the edge's other node).  Column arrays are private (up to
-// WTG_REMAP_MAX_LAYERS layers); FP64 in the reference's evaluation order
-// without FMA contraction.  The analytic profiles call exp, whose last bit may
-// differ from the host library's; everything else equals the oracle bit for
-// bit.  Both kernels are HBM-bound single passes over the column state.
+// the edge's other node).  Up to 32 layers a column stays in registers (unrolled
+// loops, sizes 16, 24, 32); above, and where dgtsv would pivot, its arrays are
+// private (up to WTG_REMAP_MAX_LAYERS layers).  FP64 in the reference's
+// evaluation order without FMA contraction.  The analytic profiles call exp, whose last bit may
+// differ from the host library's; everything else equals the oracle bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "ctx.h"
@@ -26,7 +26,7 @@ namespace {
 
 constexpr int H = wtg::HALO;
 constexpr int VMAX = WTG_REMAP_MAX_LAYERS;
-constexpr int VT = 64;  // threads per block: the private column arrays are large
+constexpr int VT = 64;  // threads per block: one wave, since the column arrays are large
 
 struct VdArgs {
   int n, S, L, istep;
@@ -367,7 +367,8 @@ __global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) 
 // with dUdZ^2, N^2, one length or pivot and the right-hand side per level kept
 // between them.  Same operations as turbulent_column, to which a system that
 // dgtsv would pivot is left (vd_tke_left_kernel).  Bound by the latency of its divisions and square roots at
-// one or two waves per SIMD.  J8 L30: TKE_FIGURES
+// one or two waves per SIMD.  J8 L30: 1.79 -> 0.88 ms
+// (one wave per SIMD); the whole call 3.48 -> 1.85 ms, at J7 L20 0.69 -> 0.30 ms.
 template <int LM>
 __global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
   const int64_t tid = (int64_t)blockIdx.x * VT + threadIdx.x;
@@ -695,7 +696,7 @@ __global__ __launch_bounds__(VT) void vd_solve_kernel(VdArgs a) {
 // flux and a column with a thickness that is not positive are left to
 // vd_solve_left_kernel (a call from here would cost the arrays their registers).
 // Bound by memory latency at two waves per SIMD (three arrays of 32 doubles are
-// 192 registers).  J8 L30: SOLVE_FIGURES; with the arrays in LDS (three waves
+// 192 // 192 registers).  J8 L30: 1.63 -> 0.70 ms; with the arrays in LDS (three waves
 // per compute unit) 1.6 ms.
 template <int LM>
 __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArgs a, int ncb) {
