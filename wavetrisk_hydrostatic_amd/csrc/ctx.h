@@ -109,6 +109,13 @@ struct wtg_ctx {
   // launch); larger ones use a final one-block kernel, because the last
   // block's device-scope fence costs L2 write-backs that grow with the grid
   int lastblock_max = 64;
+  // BiCGSTAB in one launch (small levels): owner of every cell, the blocks'
+  // partial sums, and per member whether a wait ran out with its host copy
+  bool bicg_one = true;
+  bool red_masters = false;  // the reduction cells are the masters, in order
+  int* d_src = nullptr;
+  double* d_bpart = nullptr;
+  unsigned *d_sync = nullptr, *h_sync = nullptr;
   double* d_scal = nullptr;      // device scalars of the solvers
   double* h_scal = nullptr;      // pinned host copy (hipHostMalloc)
   int part_blocks = 0;

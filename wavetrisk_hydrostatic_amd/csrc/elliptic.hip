@@ -20,6 +20,7 @@
 #include <utility>
 
 #include "ctx.h"
+#include "exact_div.h"
 #include "mg_ops.h"
 #include "mlp.h"
 
@@ -589,6 +590,223 @@ __global__ __launch_bounds__(FS_NT) void fs_bicg_res_kernel(
   if (count) dot_last_block(nbred, 2, part, SC_T0, SC_T3, 0, scal, OP_ERR_BETA, 1, count, sh);
 }
 
+// ---------------------------------------------------------------------------
+// fs_bicg_solve_kernel: a whole BiCGSTAB solve in one launch, for levels whose
+// masters fit into BICG_BLOCKS resident blocks.  A thread holds one master's
+// residual, direction and operator coefficients and its six neighbours' residual
+// and direction in registers; the neighbours' new values come from memory
+// after each of an iteration's three reductions, which are barriers over the
+// member's blocks at the same time.  Residual and Ap are stored and read at
+// device scope (past the XCDs' L2s), so no cache is written back or
+// invalidated; a block's partial sums go out after its values, and every block
+// then adds all partials in fs_dot_final_kernel's order.  The same operations
+// as the launches of `bicgstab`: same iterates, residuals and counts.
+// A wait is bounded (2 s): if it ends, every block leaves with u untouched and
+// the solve is repeated by the launches.
+// Bound by the three device-wide round trips of an iteration.  An iteration by
+// launches (five, replayed from a graph) -> in here: J4 31.1 -> 9.3 us, J5 37.0
+// -> 11.1, J6 (161 blocks) 31.1 -> 12.6; the grids of J7 and finer do not fit.
+// ---------------------------------------------------------------------------
+constexpr int BICG_BLOCKS = 256;  // at most one block of a solve per compute unit, so that all are resident
+constexpr unsigned long long BICG_WAIT = 200000000ull;  // ticks of the 100 MHz wall clock
+
+__device__ __forceinline__ double load_out(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_out(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A slot of `part` that holds no sum yet; the sums' NaNs are the plain one
+constexpr unsigned long long BICG_EMPTY = 0x7ff4b1c657ab0001ull;
+
+// sums of acc[0], acc[1] over the member's blocks, after every block's earlier
+// store_out; false if the wait ran out.  Three sets of slots in turn: a block
+// that leaves a reduction knows that all have read the one before, and empties
+// its slot of that one, which the reduction after the next uses.
+__device__ __forceinline__ bool reduce_out(double s0, double s1, double (*sh)[FS_NT], double* part, unsigned& epoch,
+                                           int* ok, double out[2]) {
+  const int nb = gridDim.x, tid = threadIdx.x;
+  auto slot = [&](unsigned e, int b) { return part + ((e % 3) * BICG_BLOCKS + b) * 2; };
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have left
+  double acc[RED_MAX] = {s0, s1, 0.0};
+  block_tree(acc, sh);
+  if (tid < 2) {
+    const double v = sh[tid][0];
+    store_out(slot(epoch, blockIdx.x) + tid, v == v ? v : __longlong_as_double(0x7ff8000000000000ll));
+  }
+  acc[0] = acc[1] = 0.0;
+  if (tid < nb) {  // nb <= BICG_BLOCKS = FS_NT: one block's sums a thread
+    const double* q = slot(epoch, tid);
+    const unsigned long long t0 = wall_clock64();
+    double v0, v1;
+    while (true) {
+      v0 = load_out(q), v1 = load_out(q + 1);
+      if (__double_as_longlong(v0) != (long long)BICG_EMPTY && __double_as_longlong(v1) != (long long)BICG_EMPTY) break;
+      if (wall_clock64() - t0 > BICG_WAIT) {
+        *ok = 0;
+        break;
+      }
+    }
+    acc[0] = acc[0] + v0, acc[1] = acc[1] + v1;
+  }
+  __syncthreads();  // sh is free again
+  block_tree(acc, sh);
+  __syncthreads();
+  out[0] = sh[0][0], out[1] = sh[1][0];
+  const bool good = *ok;
+  __syncthreads();
+  if (tid < 2) store_out(slot(epoch + 2, blockIdx.x) + tid, __longlong_as_double((long long)BICG_EMPTY));
+  ++epoch;
+  return good;
+}
+
+struct BicgArgs {
+  const double* mdone;
+  int n;               // masters
+  const int64_t* ncl;
+  const int* src;      // owner of every cell (itself where it has none)
+  FsGeo g;
+  const double *u, *f, *eo;
+  double grav, coef, tol;
+  int zero_u, maxit;
+  double *res, *Ap;    // the published vectors
+  double* out;         // the solution's masters
+  const double* rw;    // reduction weight of every master
+  double *scal, *part;
+  unsigned* sync;      // [member]: a wait ran out
+  int64_t ms;
+};
+
+__global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
+  __shared__ double sh[RED_MAX][FS_NT];
+  __shared__ int ok;
+  if (threadIdx.x == 0) ok = 1;
+  FsGeo g = a.g;
+  g.topo = mem(g.topo, a.ms);
+  const double *u = mem(a.u, a.ms), *f = mem(a.f, a.ms), *eo = mem(a.eo, a.ms);
+  double *const res = mem(a.res, a.ms), *const Apv = mem(a.Ap, a.ms), *const out = mem(a.out, a.ms);
+  double* const scal = mem(a.scal, SC_NSCAL);
+  double* const part = mem(a.part, (int64_t)6 * BICG_BLOCKS);
+  const int t = blockIdx.x * FS_NT + threadIdx.x;
+  const bool live = t < a.n;
+  const int64_t c = a.ncl[2 * (live ? t : 0) + 1];
+  if (mdone_of(a.mdone)) {  // converged member: only the zero guess is set
+    if (live) out[c] = a.zero_u ? 0.0 : u[c];
+    if (t == 0) {
+      scal[SC_DONE] = 1.0;
+      scal[SC_ITER] = 0.0;
+    }
+    return;
+  }
+  int64_t x7[7];
+  cells7(g, c, x7);
+  int nb[7];
+  for (int k = 1; k < 7; ++k) nb[k] = a.src[x7[k]];
+  // the six fluxes' mean squared wave speed, length and dual length (ell_flux)
+  double I[6], len[6], rl[6], ped[6];
+  {
+    const int at[6] = {0, 4, 5, 0, 0, 6}, to[6] = {1, 0, 0, 2, 3, 0}, ed[6] = {0, 0, 1, 1, 2, 2};
+    double cs[7];
+    for (int k = 0; k < 7; ++k) cs[k] = a.grav * (fabs(g.topo[x7[k]]) * 1.0 + eo[x7[k]]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      I[k] = interp(cs[at[k]], cs[to[k]]);
+      len[k] = g.lenf[ed[k] * g.NC + x7[at[k]]];
+      ped[k] = g.pedf[ed[k] * g.NC + x7[at[k]]];
+      rl[k] = 1.0 / len[k];
+    }
+  }
+  const double hinv = g.hinv[c], w = live ? a.rw[t] : 0.0;
+  auto flux = [&](int k, double d) { return div_by(I[k] * d, len[k], rl[k]) * ped[k]; };
+  auto apply = [&](const double q[7]) {
+    const double dv = (flux(0, q[1] - q[0]) - flux(1, q[0] - q[4]) + flux(2, q[5] - q[0]) - flux(3, q[0] - q[2]) +
+                       flux(4, q[3] - q[0]) - flux(5, q[0] - q[6])) *
+                      hinv;
+    return a.coef * dv - q[0];
+  };
+  unsigned epoch = 0;
+  double sum[2];
+  auto sums = [&](double s0, double s1) {
+    return reduce_out(live ? w * s0 : 0.0, live ? w * s1 : 0.0, sh, part, epoch, &ok, sum);
+  };
+  // res = f - L u; nrm_f = l2(f); rho = dp(res0, res)
+  const double fc = f[c];
+  double uc = 0.0, r;
+  if (a.zero_u) {
+    r = fc - 0.0;
+  } else {
+    double q[7];
+    for (int k = 0; k < 7; ++k) q[k] = u[x7[k]];
+    uc = q[0];
+    r = fc - apply(q);
+  }
+  if (live) store_out(res + c, r);
+  bool good = sums(fc * fc, r * r);
+  const double nf = sqrt(sum[0]), nrmf = nf == 0.0 ? 1.0 : nf, res0 = r;
+  double rho = sum[1], p7[7], r7[7], A7[7], err = 0.0;
+  auto gather = [&](const double* v, double own, double q[7]) {
+    q[0] = own;
+    for (int k = 1; k < 7; ++k) q[k] = load_out(v + nb[k]);
+  };
+  gather(res, r, r7);
+  for (int k = 0; k < 7; ++k) p7[k] = r7[k];
+  double Ap = apply(p7);
+  int iter = 1;
+  bool done = false;
+  for (; good && iter <= a.maxit; ++iter) {
+    if (live) store_out(Apv + c, Ap);
+    good = sums(Ap * res0, 0.0);
+    const double alph = rho / sum[0], ma = -1.0 * alph;
+    gather(Apv, Ap, A7);
+    double s7[7];
+    for (int k = 0; k < 7; ++k) s7[k] = 1.0 * r7[k] + ma * A7[k];
+    const double sc = s7[0], As = apply(s7);
+    good = good && sums(As * sc, As * As);
+    const double omga = sum[0] / sum[1], mo = -1.0 * omga;
+    const double corr = (1.0 * alph) * p7[0] + (1.0 * omga) * sc;
+    uc = 1.0 * uc + 1.0 * corr;
+    r = 1.0 * sc + mo * As;
+    if (live) store_out(res + c, r);
+    good = good && sums(r * r, res0 * r);
+    err = sqrt(sum[0]) / nrmf;
+    if (err <= a.tol) {
+      done = true;
+      break;
+    }
+    const double rho_old = rho;
+    rho = sum[1];
+    const double b = (alph / omga) * (rho / rho_old), bb = 1.0 * b;
+    gather(res, r, r7);
+    for (int k = 0; k < 7; ++k) {
+      const double cr = 1.0 * p7[k] + mo * A7[k];
+      p7[k] = 1.0 * r7[k] + bb * cr;
+    }
+    Ap = apply(p7);
+  }
+  if (!good) {
+    if (threadIdx.x == 0) mem(a.sync, 1)[0] = 1u;
+    return;
+  }
+  if (live) out[c] = uc;
+  if (t == 0) {
+    scal[SC_NRMF] = nrmf;
+    scal[SC_ERR] = err;
+    scal[SC_ITER] = (double)(done ? iter : a.maxit);
+    scal[SC_DONE] = done ? 1.0 : 0.0;
+  }
+}
+
+// u = the solution of fs_bicg_solve_kernel, masters and halo copies; its
+// slots empty for the next launch
+__global__ void fs_bicg_out_kernel(int n, const int64_t* __restrict__ ncl, const double* __restrict__ out,
+                                   double* __restrict__ u, double* __restrict__ part, int64_t ms) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 6 * BICG_BLOCKS) mem(part, (int64_t)6 * BICG_BLOCKS)[t] = __longlong_as_double((long long)BICG_EMPTY);
+  if (t >= n) return;
+  mem(u, ms)[ncl[2 * t]] = mem(out, ms)[ncl[2 * t + 1]];
+}
+
 // ===========================================================================
 // Multi-level scalar wavelet transform (one level) and the multigrid solvers
 // ===========================================================================
@@ -795,7 +1013,22 @@ int fs_ready(wtg_ctx* c) {
   WTG_HIPCHK(c, hipMemsetAsync(c->d_count, 0, M * sizeof(unsigned), c->stream));
   if (int rc = wtg_dalloc<double>(c, &c->d_scal, (size_t)SC_NSCAL * M)) return rc;
   WTG_HIPCHK(c, hipMemsetAsync(c->d_scal, 0, SC_NSCAL * M * sizeof(double), c->stream));
-  WTG_HIPCHK(c, hipHostMalloc((void**)&c->h_scal, SC_NSCAL * M * sizeof(double), hipHostMallocDefault));
+  // (the failed waits of fs_bicg_solve_kernel come back behind the scalars)
+  WTG_HIPCHK(c, hipHostMalloc((void**)&c->h_scal, SC_NSCAL * M * sizeof(double) + M * sizeof(unsigned),
+                              hipHostMallocDefault));
+  c->h_sync = reinterpret_cast<unsigned*>(c->h_scal + SC_NSCAL * M);
+  std::vector<int> src;
+  if (c->red_masters && nblk(c->nmaster) <= BICG_BLOCKS) {
+    src.resize(c->info.ncells);
+    for (int64_t x = 0; x < c->info.ncells; ++x) src[x] = (int)(c->node_src[x] >= 0 ? c->node_src[x] : x);
+    if (int rc = wtg_dalloc<int>(c, &c->d_src, src.size())) return rc;
+    if (int rc = wtg_dalloc<unsigned>(c, &c->d_sync, M)) return rc;
+    const std::vector<unsigned long long> empty(6 * BICG_BLOCKS * M, BICG_EMPTY);
+    if (int rc = wtg_dalloc<double>(c, &c->d_bpart, empty.size())) return rc;
+    WTG_HIPCHK(c, hipMemcpy(c->d_bpart, empty.data(), empty.size() * sizeof(double), hipMemcpyHostToDevice));
+    WTG_HIPCHK(c, hipMemcpyAsync(c->d_src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    WTG_HIPCHK(c, hipMemsetAsync(c->d_sync, 0, M * sizeof(unsigned), c->stream));
+  }
   WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -925,11 +1158,69 @@ int read_scalar(wtg_ctx* c, int i, double* out) {
 // masters in place and its halo copies refreshed after the loop.
 constexpr int BICG_CHUNK = 8;
 
+// whether a solve on this level is one launch of fs_bicg_solve_kernel: one
+// block per 256 masters of every member, all resident at once with room for a
+// second such solve on another stream (a compute unit holds two blocks).  It is
+// the faster one wherever it fits; a context that replays graphs has asked for
+// the launches.
+bool bicg_one_launch(const wtg_ctx* c, int maxit) {
+  return c->bicg_one && c->d_src && !c->fs_graph && maxit > 0 &&
+         (int64_t)nblk(c->nmaster) * c->nmembers <= BICG_BLOCKS;
+}
+
+int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int* iters, double* err_out,
+                        bool zero_u, bool sync_end, bool* solved) {
+  double** W = c->fs + FS_W0;
+  const int M = c->nmembers;
+  const int64_t ms = c->info.ncells;
+  BicgArgs a{c->mg_mdone, c->nmaster, c->d_ncl, c->d_src, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav,
+             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[3], c->d_rw, c->d_scal, c->d_bpart, c->d_sync, ms};
+  hipLaunchKernelGGL(fs_bicg_solve_kernel, dim3(nblk(c->nmaster), M), dim3(FS_NT), 0, c->stream, a);
+  WTG_HIPCHK(c, hipGetLastError());
+  WTG_HIPCHK(c, hipMemcpyAsync(c->h_scal, c->d_scal, (size_t)SC_NSCAL * M * sizeof(double), hipMemcpyDeviceToHost,
+                               c->stream));
+  WTG_HIPCHK(c, hipMemcpyAsync(c->h_sync, c->d_sync, M * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
+  WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
+  bool failed = false;
+  for (int m = 0; m < M; ++m) failed = failed || c->h_sync[m];
+  if (failed) {  // u is as it was; leave the slots empty and the flags down
+    hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(nblk(6 * BICG_BLOCKS), M), dim3(FS_NT), 0, c->stream, 0, c->d_ncl,
+                       W[3], u, c->d_bpart, ms);
+    WTG_HIPCHK(c, hipGetLastError());
+    WTG_HIPCHK(c, hipMemsetAsync(c->d_sync, 0, M * sizeof(unsigned), c->stream));
+    return 0;
+  }
+  hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(std::max(nblk(c->nncl), nblk(6 * BICG_BLOCKS)), M), dim3(FS_NT), 0,
+                     c->stream, c->nncl, c->d_ncl, W[3], u, c->d_bpart, ms);
+  WTG_HIPCHK(c, hipGetLastError());
+  if (sync_end) WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
+  // ensembles: the most iterations and the largest residual of the members
+  bool done = true;
+  int itmax = 0;
+  double emax = 0.0;
+  for (int m = 0; m < M; ++m) {
+    const double* s = c->h_scal + m * SC_NSCAL;
+    done = done && s[SC_DONE] != 0.0;
+    itmax = std::max(itmax, (int)s[SC_ITER]);
+    emax = std::max(emax, s[SC_ERR]);
+  }
+  *iters = done ? itmax : maxit + 1;
+  *err_out = emax;
+  *solved = true;
+  return 0;
+}
+
 // zero_u: start from u = 0 (u is overwritten); sync_end: wait for the
 // final ghost copy of u before returning (callers that stay on the stream
 // need not)
 int bicgstab(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int* iters, double* err_out,
              bool zero_u = false, bool sync_end = true) {
+  if (bicg_one_launch(c, maxit)) {
+    bool solved = false;
+    RC(bicgstab_one_launch(c, u, f, tol, maxit, iters, err_out, zero_u, sync_end, &solved));
+    if (solved) return 0;
+    c->bicg_one = false;  // its blocks did not run together; u is as it was
+  }
   double** W = c->fs + FS_W0;
   double *res = W[0], *res0 = W[1], *p = W[2], *s = W[3], *Ap = W[4], *As = W[5], *p_alt = W[6];
   RC(launch_dots_g(c, false, OP_NRMF, 1, f, f, SC_T0));  // nrm_f = l2(f)

@@ -3068,6 +3068,8 @@ int wtg_create_ensemble(const wtg_grid* grid, const wtg_params* params, int nmem
   }
   c->nncl = (int)(ncl.size() / 2);
   c->nred = (int)rcell.size();
+  c->red_masters = c->nred == c->nmaster;
+  for (int q = 0; q < c->nred && c->red_masters; ++q) c->red_masters = rcell[q] == ncl[2 * q];
   c->nn = (int)(nd.size() / 2);
   c->ne = (int)(ed.size() / 2);
   c->nfn = (int)fn.size();
