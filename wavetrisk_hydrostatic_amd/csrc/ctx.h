@@ -109,13 +109,17 @@ struct wtg_ctx {
   // launch); larger ones use a final one-block kernel, because the last
   // block's device-scope fence costs L2 write-backs that grow with the grid
   int lastblock_max = 64;
-  // BiCGSTAB in one launch (small levels): owner of every cell, the blocks'
-  // partial sums, and per member whether a wait ran out with its host copy
+  // BiCGSTAB in one launch (small levels): owner of every cell and the
+  // blocks' partial sums
   bool bicg_one = true;
   bool red_masters = false;  // the reduction cells are the masters, in order
   int* d_src = nullptr;
   double* d_bpart = nullptr;
-  unsigned *d_sync = nullptr, *h_sync = nullptr;
+  // several Jacobi sweeps in one launch: 0 not built, 1 built, -1 not for this
+  // grid; its tiles, and the most masters of a tile with 0.. rings around it
+  int sw_state = 0, sw_tiles = 0, sw_rows[6] = {};
+  int *d_swcnt = nullptr, *d_swcell = nullptr, *d_swhalo = nullptr;
+  unsigned* d_swnb = nullptr;
   double* d_scal = nullptr;      // device scalars of the solvers
   double* h_scal = nullptr;      // pinned host copy (hipHostMalloc)
   int part_blocks = 0;

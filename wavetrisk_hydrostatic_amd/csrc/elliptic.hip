@@ -37,6 +37,7 @@ enum Scal {
   SC_ITER,  // iterations completed by the gated loop
   SC_TOL,   // its tolerance
   SC_MR,    // minimal-residual step of the learned correction
+  SC_FAIL,  // a wait of fs_bicg_solve_kernel ran out
   SC_NSCAL
 };
 
@@ -504,6 +505,35 @@ __device__ __forceinline__ void cells7(const FsGeo& g, int64_t c, int64_t x7[7])
   x7[6] = c - g.S;
 }
 
+// the operator at one cell, held in registers: of the six fluxes the mean
+// squared wave speed, length and dual length; ell_apply_at's operations
+struct EllCoef {
+  double I[6], len[6], rl[6], ped[6], hinv, coef;
+  __device__ __forceinline__ void load(const FsGeo& g, const double* __restrict__ eo, double grav, double coef_,
+                                       const int64_t x7[7]) {
+    const int at[6] = {0, 4, 5, 0, 0, 6}, to[6] = {1, 0, 0, 2, 3, 0}, ed[6] = {0, 0, 1, 1, 2, 2};
+    double cs[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) cs[k] = grav * (fabs(g.topo[x7[k]]) * 1.0 + eo[x7[k]]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      I[k] = interp(cs[at[k]], cs[to[k]]);
+      len[k] = g.lenf[ed[k] * g.NC + x7[at[k]]];
+      ped[k] = g.pedf[ed[k] * g.NC + x7[at[k]]];
+      rl[k] = 1.0 / len[k];
+    }
+    hinv = g.hinv[x7[0]];
+    coef = coef_;
+  }
+  __device__ __forceinline__ double flux(int k, double d) const { return div_by(I[k] * d, len[k], rl[k]) * ped[k]; }
+  __device__ __forceinline__ double apply(const double q[7]) const {
+    const double dv = (flux(0, q[1] - q[0]) - flux(1, q[0] - q[4]) + flux(2, q[5] - q[0]) - flux(3, q[0] - q[2]) +
+                       flux(4, q[3] - q[0]) - flux(5, q[0] - q[6])) *
+                      hinv;
+    return coef * dv - q[0];
+  }
+};
+
 // s = res - alph Ap and As = L s in one pass (s is evaluated at the stencil's
 // seven cells; res and Ap are ghost filled, so halo values equal the owners')
 __global__ void fs_bicg_s_apply_kernel(const double* __restrict__ gate, int n, const int64_t* __restrict__ ncl,
@@ -674,7 +704,6 @@ struct BicgArgs {
   double* out;         // the solution's masters
   const double* rw;    // reduction weight of every master
   double *scal, *part;
-  unsigned* sync;      // [member]: a wait ran out
   int64_t ms;
 };
 
@@ -703,28 +732,10 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
   cells7(g, c, x7);
   int nb[7];
   for (int k = 1; k < 7; ++k) nb[k] = a.src[x7[k]];
-  // the six fluxes' mean squared wave speed, length and dual length (ell_flux)
-  double I[6], len[6], rl[6], ped[6];
-  {
-    const int at[6] = {0, 4, 5, 0, 0, 6}, to[6] = {1, 0, 0, 2, 3, 0}, ed[6] = {0, 0, 1, 1, 2, 2};
-    double cs[7];
-    for (int k = 0; k < 7; ++k) cs[k] = a.grav * (fabs(g.topo[x7[k]]) * 1.0 + eo[x7[k]]);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      I[k] = interp(cs[at[k]], cs[to[k]]);
-      len[k] = g.lenf[ed[k] * g.NC + x7[at[k]]];
-      ped[k] = g.pedf[ed[k] * g.NC + x7[at[k]]];
-      rl[k] = 1.0 / len[k];
-    }
-  }
-  const double hinv = g.hinv[c], w = live ? a.rw[t] : 0.0;
-  auto flux = [&](int k, double d) { return div_by(I[k] * d, len[k], rl[k]) * ped[k]; };
-  auto apply = [&](const double q[7]) {
-    const double dv = (flux(0, q[1] - q[0]) - flux(1, q[0] - q[4]) + flux(2, q[5] - q[0]) - flux(3, q[0] - q[2]) +
-                       flux(4, q[3] - q[0]) - flux(5, q[0] - q[6])) *
-                      hinv;
-    return a.coef * dv - q[0];
-  };
+  EllCoef ell;
+  ell.load(g, eo, a.grav, a.coef, x7);
+  const double w = live ? a.rw[t] : 0.0;
+  auto apply = [&](const double q[7]) { return ell.apply(q); };
   unsigned epoch = 0;
   double sum[2];
   auto sums = [&](double s0, double s1) {
@@ -785,7 +796,7 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
     Ap = apply(p7);
   }
   if (!good) {
-    if (threadIdx.x == 0) mem(a.sync, 1)[0] = 1u;
+    if (threadIdx.x == 0) scal[SC_FAIL] = 1.0;
     return;
   }
   if (live) out[c] = uc;
@@ -800,11 +811,139 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
 // u = the solution of fs_bicg_solve_kernel, masters and halo copies; its
 // slots empty for the next launch
 __global__ void fs_bicg_out_kernel(int n, const int64_t* __restrict__ ncl, const double* __restrict__ out,
-                                   double* __restrict__ u, double* __restrict__ part, int64_t ms) {
+                                   double* __restrict__ u, double* __restrict__ part, double* __restrict__ scal,
+                                   int64_t ms) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t == 0) mem(scal, SC_NSCAL)[SC_FAIL] = 0.0;
   if (t < 6 * BICG_BLOCKS) mem(part, (int64_t)6 * BICG_BLOCKS)[t] = __longlong_as_double((long long)BICG_EMPTY);
   if (t >= n) return;
   mem(u, ms)[ncl[2 * t]] = mem(out, ms)[ncl[2 * t + 1]];
+}
+
+// ---------------------------------------------------------------------------
+// fs_sweeps_kernel: several Jacobi sweeps, and the residual after them, in one
+// launch without a word between its blocks.  A block owns a tile of 16 x 16
+// masters and carries as many rings of masters around it as the sweeps need,
+// each ring good for one sweep less; a thread holds one master's operator in
+// registers for all of them and the values go through LDS.  Rings are masters
+// found over the grid's seams too and evaluated with their own stencil, so
+// every value has the operations of fs_jacobi_kernel, to the last bit.
+// Bound by the loads of the operator (15 doubles a master) and the rings' share
+// of them: 1.6 times the tile's masters for two rings, 2.6 times for five.
+// A V-cycle's smoothing (2 sweeps down and up, 4 after) as single sweeps -> in
+// here: cycles on levels J5-J7 249 -> 176 us, J5-J8 513 -> 302 us, of which the
+// coarse solve takes about 110.  Four sweeps with the residual take 20 us at J7
+// (11 each before).  The tiles of an XCD in a row instead of dealt out: 3 to
+// 6 % of a cycle.
+// ---------------------------------------------------------------------------
+constexpr int SW_RINGS = 5;     // most rings of a launch
+constexpr int SW_ROWS = 768;    // most masters of a block and its rings
+constexpr int SW_SMALL = 512;   // blocks of up to this many run two to a compute unit
+enum { SW_HALO0 = SW_RINGS + 1, SW_HALO1, SW_NCNT };
+
+struct SwPlan {
+  const int* cnt;       // [tile][SW_NCNT]: masters within 0.. rings; the tile's halo copies
+  const int* cell;      // [tile][SW_ROWS]
+  const unsigned* nb;   // [tile][3][SW_ROWS]: rows of the six neighbours, two a word (SW_ROWS: none)
+  const int* halo;      // (halo cell, row)
+};
+
+template <class F>
+struct SwArgs {
+  const double* mdone;
+  SwPlan plan;
+  FsGeo g;
+  const F *u, *add, *f;  // the sweeps start from u (null: 0), or u + add
+  const double* eo;
+  double grav, coef, dt2, th12, w;
+  int n, rings;          // sweeps; rings they and the residual need
+  F *out, *res;          // res null: no residual
+  int64_t ms;
+};
+
+template <class F, int NT>
+__global__ __launch_bounds__(NT, NT > SW_SMALL ? 3 : 4) void fs_sweeps_kernel(SwArgs<F> a) {
+  __shared__ double v[2][NT + 1];
+  // an eighth of the tiles, neighbours mostly, to each XCD's L2
+  const int per = gridDim.x / 8, b = blockIdx.x, tile = b < 8 * per ? b % 8 * per + b / 8 : b;
+  const int t = threadIdx.x, nt = blockDim.x;
+  const int* cnt = a.plan.cnt + tile * SW_NCNT;
+  const int own = cnt[0], rows = cnt[a.rings];
+  F *const out = mem(a.out, a.ms), *const res = a.res ? mem(a.res, a.ms) : nullptr;
+  const bool live = t < rows;
+  const int64_t c = live ? a.plan.cell[(int64_t)tile * SW_ROWS + t] : 0;
+  double* q = v[0];
+  const bool done = mdone_of(a.mdone);  // converged member: u stays, no residual
+  double r = 0.0;
+  if (live && a.u) {
+    const F* const u = mem(a.u, a.ms);
+    r = a.add && !done ? (double)(F)(1.0 * u[c] + 1.0 * mem(a.add, a.ms)[c]) : (double)u[c];
+  }
+  if (!done) {
+    const double* const eo = mem(a.eo, a.ms);
+    FsGeo g = a.g;
+    g.topo = mem(g.topo, a.ms);
+    double fc = 0.0, wd = 1.0, rd = 1.0;
+    if (live) {
+      fc = mem(a.f, a.ms)[c];
+      wd = ell_diag_at(g, eo, a.grav, a.dt2, a.th12, c);
+      rd = 1.0 / wd;
+    }
+    int n = a.n, ring = a.rings;
+    if (!a.u && n > 0) {
+      r = (F)(0.0 + div_by(a.w * (fc - 0.0), wd, rd));
+      --n;
+    }
+    if (ring > 0) {
+      int nb[6];
+      EllCoef ell;
+      if (t < cnt[ring - 1]) {
+        int64_t x7[7];
+        cells7(g, c, x7);
+        ell.load(g, eo, a.grav, a.coef, x7);
+        for (int k = 0; k < 3; ++k) {
+          const unsigned p = a.plan.nb[((int64_t)tile * 3 + k) * SW_ROWS + t];
+          nb[2 * k] = min((int)(p & 0xffffu), NT), nb[2 * k + 1] = min((int)(p >> 16), NT);
+        }
+      }
+      if (live) q[t] = r;
+      if (t == 0) v[0][NT] = v[1][NT] = 0.0;
+      __syncthreads();
+      auto Lu = [&]() {
+        double x[7];
+        x[0] = r;
+        for (int k = 0; k < 6; ++k) x[k + 1] = q[nb[k]];
+        return ell.apply(x);
+      };
+      for (; n > 0; --n) {
+        --ring;
+        double* const qn = q == v[0] ? v[1] : v[0];
+        if (t < cnt[ring]) {
+          r = (F)(r + div_by(a.w * (fc - Lu()), wd, rd));
+          qn[t] = r;
+        }
+        q = qn;
+        __syncthreads();
+      }
+      if (res) {
+        double* const qr = q == v[0] ? v[1] : v[0];
+        if (t < own) {
+          const F e = (F)(fc - Lu());
+          res[c] = e;
+          qr[t] = e;
+        }
+        __syncthreads();
+        for (int h = cnt[SW_HALO0] + t; h < cnt[SW_HALO1]; h += nt) res[a.plan.halo[2 * h]] = (F)qr[a.plan.halo[2 * h + 1]];
+      }
+    }
+  }
+  // u and its halo copies
+  if (t < own) {
+    out[c] = (F)r;
+    q[t] = r;
+  }
+  __syncthreads();
+  for (int h = cnt[SW_HALO0] + t; h < cnt[SW_HALO1]; h += nt) out[a.plan.halo[2 * h]] = (F)q[a.plan.halo[2 * h + 1]];
 }
 
 // ===========================================================================
@@ -1013,21 +1152,16 @@ int fs_ready(wtg_ctx* c) {
   WTG_HIPCHK(c, hipMemsetAsync(c->d_count, 0, M * sizeof(unsigned), c->stream));
   if (int rc = wtg_dalloc<double>(c, &c->d_scal, (size_t)SC_NSCAL * M)) return rc;
   WTG_HIPCHK(c, hipMemsetAsync(c->d_scal, 0, SC_NSCAL * M * sizeof(double), c->stream));
-  // (the failed waits of fs_bicg_solve_kernel come back behind the scalars)
-  WTG_HIPCHK(c, hipHostMalloc((void**)&c->h_scal, SC_NSCAL * M * sizeof(double) + M * sizeof(unsigned),
-                              hipHostMallocDefault));
-  c->h_sync = reinterpret_cast<unsigned*>(c->h_scal + SC_NSCAL * M);
+  WTG_HIPCHK(c, hipHostMalloc((void**)&c->h_scal, SC_NSCAL * M * sizeof(double), hipHostMallocDefault));
   std::vector<int> src;
   if (c->red_masters && nblk(c->nmaster) <= BICG_BLOCKS) {
     src.resize(c->info.ncells);
     for (int64_t x = 0; x < c->info.ncells; ++x) src[x] = (int)(c->node_src[x] >= 0 ? c->node_src[x] : x);
     if (int rc = wtg_dalloc<int>(c, &c->d_src, src.size())) return rc;
-    if (int rc = wtg_dalloc<unsigned>(c, &c->d_sync, M)) return rc;
     const std::vector<unsigned long long> empty(6 * BICG_BLOCKS * M, BICG_EMPTY);
     if (int rc = wtg_dalloc<double>(c, &c->d_bpart, empty.size())) return rc;
     WTG_HIPCHK(c, hipMemcpy(c->d_bpart, empty.data(), empty.size() * sizeof(double), hipMemcpyHostToDevice));
     WTG_HIPCHK(c, hipMemcpyAsync(c->d_src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    WTG_HIPCHK(c, hipMemsetAsync(c->d_sync, 0, M * sizeof(unsigned), c->stream));
   }
   WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
@@ -1174,24 +1308,22 @@ int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int 
   const int M = c->nmembers;
   const int64_t ms = c->info.ncells;
   BicgArgs a{c->mg_mdone, c->nmaster, c->d_ncl, c->d_src, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav,
-             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[3], c->d_rw, c->d_scal, c->d_bpart, c->d_sync, ms};
+             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[3], c->d_rw, c->d_scal, c->d_bpart, ms};
   hipLaunchKernelGGL(fs_bicg_solve_kernel, dim3(nblk(c->nmaster), M), dim3(FS_NT), 0, c->stream, a);
   WTG_HIPCHK(c, hipGetLastError());
   WTG_HIPCHK(c, hipMemcpyAsync(c->h_scal, c->d_scal, (size_t)SC_NSCAL * M * sizeof(double), hipMemcpyDeviceToHost,
                                c->stream));
-  WTG_HIPCHK(c, hipMemcpyAsync(c->h_sync, c->d_sync, M * sizeof(unsigned), hipMemcpyDeviceToHost, c->stream));
   WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
   bool failed = false;
-  for (int m = 0; m < M; ++m) failed = failed || c->h_sync[m];
-  if (failed) {  // u is as it was; leave the slots empty and the flags down
+  for (int m = 0; m < M; ++m) failed = failed || c->h_scal[m * SC_NSCAL + SC_FAIL] != 0.0;
+  if (failed) {  // u is as it was; leave the slots empty and no failure behind
     hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(nblk(6 * BICG_BLOCKS), M), dim3(FS_NT), 0, c->stream, 0, c->d_ncl,
-                       W[3], u, c->d_bpart, ms);
+                       W[3], u, c->d_bpart, c->d_scal, ms);
     WTG_HIPCHK(c, hipGetLastError());
-    WTG_HIPCHK(c, hipMemsetAsync(c->d_sync, 0, M * sizeof(unsigned), c->stream));
     return 0;
   }
   hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(std::max(nblk(c->nncl), nblk(6 * BICG_BLOCKS)), M), dim3(FS_NT), 0,
-                     c->stream, c->nncl, c->d_ncl, W[3], u, c->d_bpart, ms);
+                     c->stream, c->nncl, c->d_ncl, W[3], u, c->d_bpart, c->d_scal, ms);
   WTG_HIPCHK(c, hipGetLastError());
   if (sync_end) WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
   // ensembles: the most iterations and the largest residual of the members
@@ -1475,6 +1607,156 @@ struct MgLv {
   double *u, *u_alt, *f, *res, *res_alt, *corr, *corr_alt;
 };
 
+// the tiles of fs_sweeps_kernel on a level (once, when its hierarchy is made)
+int sw_plan(wtg_ctx* c) {
+  if (c->sw_state) return 0;
+  c->sw_state = -1;  // a grid that the tiles do not fit keeps the single sweeps
+  const int S = c->info.S, n = c->info.n, H = (S - n) / 2;
+  const int64_t NC = c->info.ncells, T = (int64_t)S * S;
+  std::vector<int64_t> ncl(2 * (size_t)c->nncl);
+  WTG_HIPCHK(c, hipMemcpyAsync(ncl.data(), c->d_ncl, ncl.size() * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream));
+  std::vector<double> pedf(3 * (size_t)NC);
+  WTG_HIPCHK(c, hipMemcpyAsync(pedf.data(), c->d_pedf, pedf.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
+  const int64_t off[6] = {1, S + 1, S, -1, -S - 1, -S};
+  auto neighbour = [&](int64_t x, int k) { return c->node_src[x + off[k]]; };
+  // tile of every master; a pole joins a neighbour's
+  const int nt1 = n / 16, ntile = (int)(NC / T) * nt1 * nt1;
+  std::vector<int> tile_of(NC, -1);
+  std::vector<std::vector<int>> own(ntile);
+  for (int pass = 0; pass < 2; ++pass)
+    for (int q = 0; q < c->nmaster; ++q) {
+      const int64_t x = ncl[2 * q], rr = x % T;
+      const int j = (int)(rr / S) - H, i = (int)(rr % S) - H;
+      const bool inside = i >= 0 && i < n && j >= 0 && j < n;
+      if (inside != (pass == 0)) continue;
+      int to = -1;
+      if (inside)
+        to = ((int)(x / T) * nt1 + j / 16) * nt1 + i / 16;
+      else
+        for (int k = 0; k < 6 && to < 0; ++k)
+          if (neighbour(x, k) >= 0) to = tile_of[neighbour(x, k)];
+      if (to < 0) return 0;
+      tile_of[x] = to;
+      own[to].push_back((int)x);
+    }
+  std::vector<int> cnt((size_t)ntile * SW_NCNT), cell((size_t)ntile * SW_ROWS, 0), halo;
+  std::vector<unsigned> nb((size_t)ntile * 3 * SW_ROWS, SW_ROWS | (unsigned)SW_ROWS << 16);
+  std::vector<std::vector<std::pair<int, int>>> copies(ntile);
+  std::vector<int> row(NC, -1), ring;
+  for (int h = c->nmaster; h < c->nncl; ++h) {
+    if (tile_of[ncl[2 * h + 1]] < 0) return 0;
+    copies[tile_of[ncl[2 * h + 1]]].push_back({(int)ncl[2 * h], (int)ncl[2 * h + 1]});
+  }
+  for (int r = 0; r <= SW_RINGS; ++r) c->sw_rows[r] = 0;
+  for (int t = 0; t < ntile; ++t) {
+    std::vector<int>& x = own[t];
+    int* const tc = &cnt[(size_t)t * SW_NCNT];
+    for (size_t q = 0; q < x.size(); ++q) row[x[q]] = (int)q;
+    size_t begin = 0;
+    for (int r = 0; r <= SW_RINGS; ++r) {
+      const size_t end = x.size();
+      tc[r] = (int)end;
+      c->sw_rows[r] = std::max(c->sw_rows[r], (int)end);
+      if (r < SW_RINGS)
+        for (size_t q = begin; q < end; ++q)
+          for (int k = 0; k < 6; ++k) {
+            const int64_t y = neighbour(x[q], k);
+            if (y < 0) {  // outside the grid: a flux of zero length
+              const int64_t z = x[q];
+              const double p = k == 0 ? pedf[z] : k == 1 ? pedf[NC + z] : k == 2 ? pedf[2 * NC + z]
+                               : k == 3 ? pedf[z - 1] : k == 4 ? pedf[NC + z - S - 1] : pedf[2 * NC + z - S];
+              if (p != 0.0) return 0;
+            } else if (tile_of[y] < 0) {
+              return 0;
+            } else if (row[y] < 0) {
+              row[y] = (int)x.size();
+              x.push_back((int)y);
+            }
+          }
+      begin = end;
+    }
+    if (x.size() > SW_ROWS) return 0;
+    for (size_t q = 0; q < x.size(); ++q) {
+      cell[(size_t)t * SW_ROWS + q] = x[q];
+      if ((int)q >= tc[SW_RINGS - 1]) continue;  // the last ring is only read
+      for (int k = 0; k < 3; ++k) {
+        const int64_t y0 = neighbour(x[q], 2 * k), y1 = neighbour(x[q], 2 * k + 1);
+        nb[((size_t)t * 3 + k) * SW_ROWS + q] =
+            (unsigned)(y0 < 0 ? SW_ROWS : row[y0]) | (unsigned)(y1 < 0 ? SW_ROWS : row[y1]) << 16;
+      }
+    }
+    tc[SW_HALO0] = (int)halo.size() / 2;
+    for (const auto& h : copies[t]) halo.push_back(h.first), halo.push_back(row[h.second]);
+    tc[SW_HALO1] = (int)halo.size() / 2;
+    for (int y : x) row[y] = -1;
+  }
+  if (int rc = wtg_dalloc<int>(c, &c->d_swcnt, cnt.size())) return rc;
+  if (int rc = wtg_dalloc<int>(c, &c->d_swcell, cell.size())) return rc;
+  if (int rc = wtg_dalloc<unsigned>(c, &c->d_swnb, nb.size())) return rc;
+  if (int rc = wtg_dalloc<int>(c, &c->d_swhalo, halo.size())) return rc;
+  WTG_HIPCHK(c, hipMemcpy(c->d_swcnt, cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice));
+  WTG_HIPCHK(c, hipMemcpy(c->d_swcell, cell.data(), cell.size() * sizeof(int), hipMemcpyHostToDevice));
+  WTG_HIPCHK(c, hipMemcpy(c->d_swnb, nb.data(), nb.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+  WTG_HIPCHK(c, hipMemcpy(c->d_swhalo, halo.data(), halo.size() * sizeof(int), hipMemcpyHostToDevice));
+  c->sw_tiles = ntile;
+  c->sw_state = 1;
+  return 0;
+}
+
+template <class F>
+int launch_sweeps(wtg_ctx* c, const F* u, const F* add, const F* f, double w, int n, int rings, F* out, F* res) {
+  SwArgs<F> a{c->mg_mdone, SwPlan{c->d_swcnt, c->d_swcell, c->d_swnb, c->d_swhalo}, fs_geo(c), u, add, f,
+              c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c), c->fs_dt * c->fs_dt, c->fs_theta1 * c->fs_theta2, w, n,
+              rings, out, res, c->info.ncells};
+  const int nt = (c->sw_rows[rings] + 63) / 64 * 64;
+  const dim3 grid(c->sw_tiles, c->nmembers);
+  if (nt <= SW_SMALL)
+    hipLaunchKernelGGL((fs_sweeps_kernel<F, SW_SMALL>), grid, dim3(nt), 0, c->stream, a);
+  else
+    hipLaunchKernelGGL((fs_sweeps_kernel<F, SW_ROWS>), grid, dim3(nt), 0, c->stream, a);
+  WTG_HIPCHK(c, hipGetLastError());
+  return 0;
+}
+
+template <class F>
+int lv_jacobi(MgLv& v, F*& u, F*& alt, const F* f, double w, int n);
+
+// u := n Jacobi sweeps from u (zero: from 0; add: from u + add), and
+// res := f - L u if asked for
+template <class F>
+int lv_sweeps(MgLv& v, F*& u, F*& alt, bool zero, const F* add, const F* f, double w, int n, F* res) {
+  wtg_ctx* c = v.c;
+  if (zero && n == 0) {
+    RC(mg_fill(c, u, 0.0));
+    zero = false;
+  }
+  if (c->sw_state <= 0) {
+    if (add) {
+      RC(launch_lc(c, 1.0, -1, (const F*)u, 1.0, -1, add, alt));
+      std::swap(u, alt);
+    }
+    if (zero) {
+      RC((launch_jacobi<F, true>(c, u, f, w, alt)));
+      std::swap(u, alt);
+      --n;
+    }
+    RC(lv_jacobi(v, u, alt, f, w, n));
+    return res ? launch_residual(c, (const F*)u, f, res) : 0;
+  }
+  const F* start = zero ? nullptr : u;
+  do {
+    // the rings a launch still has room for: one a sweep (none for the sweep
+    // from 0, which reads no neighbour) and one for the residual
+    const int k = std::min(n, SW_RINGS + (start ? 0 : 1)), rings = k - (start ? 0 : 1);
+    const bool last = k == n && rings + (res ? 1 : 0) <= SW_RINGS;
+    RC(launch_sweeps(c, start, add, f, w, k, rings + (last && res ? 1 : 0), alt, last ? res : (F*)nullptr));
+    std::swap(u, alt);
+    start = u, add = nullptr, n -= k;
+    if (last) return 0;
+  } while (true);
+}
+
 template <class F>
 int lv_jacobi(MgLv& v, F*& u, F*& alt, const F* f, double w, int n) {
   for (int i = 0; i < n; ++i) {
@@ -1484,15 +1766,19 @@ int lv_jacobi(MgLv& v, F*& u, F*& alt, const F* f, double w, int n) {
   return 0;
 }
 
-// ||f - L u|| / nrm_f, read back
-int lv_res_err(MgLv& v, const double* f, const double* u, double nrm_f, double* out) {
-  double* r = v.c->fs[FS_W0];
-  RC(launch_residual(v.c, u, f, r));
+// ||r|| / nrm_f (r = f - L u), read back
+int lv_err(MgLv& v, const double* r, double nrm_f, double* out) {
   RC(launch_dots(v.c, 1, r, r, SC_T0));
   double d;
   RC(read_scalar(v.c, SC_T0, &d));
   *out = std::sqrt(d) / nrm_f;
   return 0;
+}
+
+int lv_res_err(MgLv& v, const double* f, const double* u, double nrm_f, double* out) {
+  double* r = v.c->fs[FS_W0];
+  RC(launch_residual(v.c, u, f, r));
+  return lv_err(v, r, nrm_f, out);
 }
 
 int lv_l2(MgLv& v, const double* a, double* out) {
@@ -1508,15 +1794,6 @@ int lv_l2(MgLv& v, const double* a, double* out) {
 template <class F>
 int lv_prolong0(wtg_mg* m, int l, const F* coarse, F* fine) {
   return mg_inverse<F, true>(m, l, coarse, nullptr, fine);
-}
-
-// n Jacobi sweeps from u = 0 (the first reads no u; n = 0 leaves u = 0)
-template <class F>
-int lv_jacobi0(MgLv& v, F*& u, F*& alt, const F* f, double w, int n) {
-  if (n == 0) return mg_fill(v.c, u, 0.0);
-  RC((launch_jacobi<F, true>(v.c, u, f, w, alt)));
-  std::swap(u, alt);
-  return lv_jacobi(v, u, alt, f, w, n - 1);
 }
 
 std::vector<MgLv> mg_levels(wtg_mg* m) {
@@ -1552,8 +1829,8 @@ int vcycle(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, doubl
   if (!r_in) RC(launch_residual(V[l].c, V[l].u, V[l].f, V[l].res));
   for (int j = l; j >= 1; --j) {
     const double* rhs = j == l && r_in ? r_in : V[j].res;
-    RC(lv_jacobi0(V[j], V[j].corr, V[j].corr_alt, rhs, 1.0, P.down_iter));  // from corr = 0
-    RC(launch_residual(V[j].c, V[j].corr, rhs, V[j].res_alt));  // res := res - L corr
+    // from corr = 0; res := res - L corr
+    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, true, (const double*)nullptr, rhs, 1.0, P.down_iter, V[j].res_alt));
     std::swap(V[j].res, V[j].res_alt);
     RC(mg_forward(m, j, V[j].res, V[j].c->fs[MG_WC], V[j - 1].res));
   }
@@ -1563,15 +1840,13 @@ int vcycle(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, doubl
   for (int j = 1; j <= l; ++j) {
     double* pf = V[j].c->fs[MG_PF];
     RC(lv_prolong0(m, j, (const double*)V[j - 1].corr, pf));
-    RC(launch_lc(V[j].c, 1.0, -1, V[j].corr, 1.0, -1, pf, V[j].corr_alt));
-    std::swap(V[j].corr, V[j].corr_alt);
-    RC(lv_jacobi(V[j], V[j].corr, V[j].corr_alt, V[j].res, 1.0, P.up_iter));
+    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, false, (const double*)pf, (const double*)V[j].res, 1.0, P.up_iter,
+                 (double*)nullptr));
   }
-  RC(launch_lc(V[l].c, 1.0, -1, V[l].u, 1.0, -1, V[l].corr, V[l].u_alt));
-  std::swap(V[l].u, V[l].u_alt);
-  RC(lv_jacobi(V[l], V[l].u, V[l].u_alt, V[l].f, 1.0, P.post_iter));
+  double* r = V[l].c->fs[FS_W0];
+  RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, (const double*)V[l].corr, (const double*)V[l].f, 1.0, P.post_iter, r));
   if (m->M > 1) return 0;  // member-batched cycles test every member's residual in the caller
-  return lv_res_err(V[l], V[l].f, V[l].u, nrm_f, err);
+  return lv_err(V[l], r, nrm_f, err);
 }
 
 // FP32 fields of the correction cycle on every level of the hierarchy
@@ -1613,8 +1888,8 @@ int vcycle32(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, dou
     RC(launch_residual(V[l].c, V[l].u, V[l].f, R));
   for (int j = l; j >= 1; --j) {
     const float* rhs = j == l ? R : res[j];
-    RC(lv_jacobi0(V[j], corr[j], corr_alt[j], rhs, 1.0, P.down_iter));  // from corr = 0
-    RC(launch_residual(V[j].c, corr[j], rhs, res_alt[j]));  // res := rhs - L corr
+    // from corr = 0; res := rhs - L corr
+    RC(lv_sweeps(V[j], corr[j], corr_alt[j], true, (const float*)nullptr, rhs, 1.0, P.down_iter, res_alt[j]));
     std::swap(res[j], res_alt[j]);
     RC(mg_forward(m, j, (const float*)res[j], V[j].c->fs32[M32_WC], res[j - 1]));
   }
@@ -1626,11 +1901,11 @@ int vcycle32(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, dou
   for (int j = 1; j <= l; ++j) {
     float* pf = V[j].c->fs32[M32_PF];
     RC(lv_prolong0(m, j, (const float*)corr[j - 1], pf));
-    RC(launch_lc(V[j].c, 1.0, -1, (const float*)corr[j], 1.0, -1, (const float*)pf, corr_alt[j]));
-    std::swap(corr[j], corr_alt[j]);
-    RC(lv_jacobi(V[j], corr[j], corr_alt[j], (const float*)res[j], 1.0, P.up_iter));
+    RC(lv_sweeps(V[j], corr[j], corr_alt[j], false, (const float*)pf, (const float*)res[j], 1.0, P.up_iter,
+                 (float*)nullptr));
   }
-  RC(lv_jacobi(V[l], corr[l], corr_alt[l], (const float*)R, 1.0, P.post_iter));
+  RC(lv_sweeps(V[l], corr[l], corr_alt[l], false, (const float*)nullptr, (const float*)R, 1.0, P.post_iter,
+               (float*)nullptr));
   RC(launch_lc(V[l].c, 1.0, -1, (const double*)V[l].u, 1.0, -1, (const float*)corr[l], V[l].u_alt));
   std::swap(V[l].u, V[l].u_alt);
   return lv_res_err(V[l], V[l].f, V[l].u, nrm_f, err);
@@ -1652,7 +1927,8 @@ int mg_fmg(wtg_mg* m, const wtg_mg_params& P, int* iters, double* res_out) {
   for (int l = 1; l < nl; ++l) {
     if (nrm1[l] < P.fine_tol) continue;
     RC(lv_prolong0(m, l, (const double*)V[l - 1].u, V[l].u));
-    RC(lv_jacobi(V[l], V[l].u, V[l].u_alt, V[l].f, 1.0, P.pre_iter));
+    RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, (const double*)nullptr, (const double*)V[l].f, 1.0, P.pre_iter,
+                 (double*)nullptr));
     for (int it = 1; it <= P.max_vcycle; ++it) {
       RC(vcycle(m, V, l, P, nrm_f[l], &res_out[l]));
       iters[l] = it;
@@ -1838,8 +2114,7 @@ int mg_cycles_members(wtg_mg* m, const wtg_mg_params& P, bool learned, int* iter
       std::swap(V[l].u, V[l].u_alt);
     }
     double unused;
-    if (int rc = vcycle(m, V, l, P, 1.0, &unused, step ? nullptr : r_top)) return finish(rc);
-    if (int rc = launch_residual(c, V[l].u, V[l].f, c->fs[FS_W0])) return finish(rc);
+    if (int rc = vcycle(m, V, l, P, 1.0, &unused, step ? nullptr : r_top)) return finish(rc);  // r in FS_W0
     if (int rc = test(0)) return finish(rc);
     const std::vector<double> before(h.begin(), h.begin() + M);
     if (int rc = read()) return finish(rc);
@@ -2169,6 +2444,11 @@ int wtg_mg_create(const wtg_grid* const* grids, wtg_ctx* const* levels, int nlev
       g_create_error = levels[l]->err;
       return rc;
     }
+    if (l > 0 || nlevels == 1)
+      if (int rc = sw_plan(levels[l])) {
+        g_create_error = levels[l]->err;
+        return rc;
+      }
     if (hipStreamSynchronize(levels[l]->stream) != hipSuccess)
       return wtg_fail(nullptr, WTG_E_DEVICE, "level %d: stream synchronisation failed", l);
   }
