@@ -1,6 +1,6 @@
-"""BiCGSTAB as one launch (levels of few blocks) against its separate launches,
-which contexts take that replay graphs (needs a GPU): J4 to J6, the last block
-partly filled; solves that converge, that stop at once, at max_iter and never
+"""BiCGSTAB as one launch against its separate launches, which contexts take
+that replay graphs (needs a GPU): J4 to J6, a cell a thread with the last block
+partly filled; J7 and J8, several cells a thread; solves that converge, that stop at once, at max_iter and never
 (a right-hand side of zeros or with a NaN); as the coarse solve of V-cycles;
 and ensembles, whose members converge apart.  The same operations in the same
 order: equal to the last bit.
@@ -29,7 +29,7 @@ def context(level, seed):
     return g, ctx, fields
 
 
-@pytest.mark.parametrize("level", [4, 5, 6])
+@pytest.mark.parametrize("level", [4, 5, 6, 7, 8])
 def test_one_launch_equals_launches(level):
     print(f"BiCGSTAB in one launch, J{level}", flush=True)
     g, ctx, (eo, u0, f) = context(level, 10 * level)

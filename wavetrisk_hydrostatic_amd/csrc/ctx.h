@@ -109,11 +109,13 @@ struct wtg_ctx {
   // launch); larger ones use a final one-block kernel, because the last
   // block's device-scope fence costs L2 write-backs that grow with the grid
   int lastblock_max = 64;
-  // BiCGSTAB in one launch (small levels): owner of every cell and the
-  // blocks' partial sums
+  // BiCGSTAB in one launch: the blocks' partial sums; of a small level the owner
+  // of every cell, of a large one the blocks' neighbour rows and rings
   bool bicg_one = true;
+  int bicg_blocks = 0;
   bool red_masters = false;  // the reduction cells are the masters, in order
-  int* d_src = nullptr;
+  int *d_src = nullptr, *d_blring = nullptr, *d_blnring = nullptr;
+  unsigned* d_blnb = nullptr;
   double* d_bpart = nullptr;
   // several Jacobi sweeps in one launch: 0 not built, 1 built, -1 not for this
   // grid; its tiles, and the most masters of a tile with 0.. rings around it

@@ -632,14 +632,15 @@ __global__ __launch_bounds__(FS_NT) void fs_bicg_res_kernel(
 // invalidated; a block's partial sums go out after its values, and every block
 // then adds all partials in fs_dot_final_kernel's order.  The same operations
 // as the launches of `bicgstab`: same iterates, residuals and counts.
-// A wait is bounded (2 s): if it ends, every block leaves with u untouched and
+// A wait is bounded (20 ms): if it ends, every block leaves with u untouched and
 // the solve is repeated by the launches.
 // Bound by the three device-wide round trips of an iteration.  An iteration by
 // launches (five, replayed from a graph) -> in here: J4 31.1 -> 9.3 us, J5 37.0
-// -> 11.1, J6 (161 blocks) 31.1 -> 12.6; the grids of J7 and finer do not fit.
+// -> 11.1, J6 (161 blocks) 31.1 -> 12.6; finer grids do not fit.
 // ---------------------------------------------------------------------------
 constexpr int BICG_BLOCKS = 256;  // at most one block of a solve per compute unit, so that all are resident
-constexpr unsigned long long BICG_WAIT = 200000000ull;  // ticks of the 100 MHz wall clock
+constexpr int BICG_SLOTS = 512;   // most partial sums of a reduction
+constexpr unsigned long long BICG_WAIT = 2000000ull;  // 20 ms: ticks of the 100 MHz wall clock
 
 __device__ __forceinline__ double load_out(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -655,30 +656,35 @@ constexpr unsigned long long BICG_EMPTY = 0x7ff4b1c657ab0001ull;
 // store_out; false if the wait ran out.  Three sets of slots in turn: a block
 // that leaves a reduction knows that all have read the one before, and empties
 // its slot of that one, which the reduction after the next uses.
+__device__ __forceinline__ double* bicg_slot(double* part, unsigned epoch, int b) {
+  return part + ((epoch % 3) * BICG_SLOTS + b) * 2;
+}
+__device__ __forceinline__ void bicg_post(double* slot, double v) {
+  store_out(slot, v == v ? v : __longlong_as_double(0x7ff8000000000000ll));
+}
+__device__ __forceinline__ void bicg_wait(const double* slot, int* ok, double& v0, double& v1) {
+  const unsigned long long t0 = wall_clock64();
+  while (true) {
+    v0 = load_out(slot), v1 = load_out(slot + 1);
+    if (__double_as_longlong(v0) != (long long)BICG_EMPTY && __double_as_longlong(v1) != (long long)BICG_EMPTY) return;
+    if (wall_clock64() - t0 > BICG_WAIT) {
+      *ok = 0;
+      return;
+    }
+  }
+}
+
 __device__ __forceinline__ bool reduce_out(double s0, double s1, double (*sh)[FS_NT], double* part, unsigned& epoch,
                                            int* ok, double out[2]) {
   const int nb = gridDim.x, tid = threadIdx.x;
-  auto slot = [&](unsigned e, int b) { return part + ((e % 3) * BICG_BLOCKS + b) * 2; };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have left
   double acc[RED_MAX] = {s0, s1, 0.0};
   block_tree(acc, sh);
-  if (tid < 2) {
-    const double v = sh[tid][0];
-    store_out(slot(epoch, blockIdx.x) + tid, v == v ? v : __longlong_as_double(0x7ff8000000000000ll));
-  }
+  if (tid < 2) bicg_post(bicg_slot(part, epoch, blockIdx.x) + tid, sh[tid][0]);
   acc[0] = acc[1] = 0.0;
   if (tid < nb) {  // nb <= BICG_BLOCKS = FS_NT: one block's sums a thread
-    const double* q = slot(epoch, tid);
-    const unsigned long long t0 = wall_clock64();
     double v0, v1;
-    while (true) {
-      v0 = load_out(q), v1 = load_out(q + 1);
-      if (__double_as_longlong(v0) != (long long)BICG_EMPTY && __double_as_longlong(v1) != (long long)BICG_EMPTY) break;
-      if (wall_clock64() - t0 > BICG_WAIT) {
-        *ok = 0;
-        break;
-      }
-    }
+    bicg_wait(bicg_slot(part, epoch, tid), ok, v0, v1);
     acc[0] = acc[0] + v0, acc[1] = acc[1] + v1;
   }
   __syncthreads();  // sh is free again
@@ -687,7 +693,7 @@ __device__ __forceinline__ bool reduce_out(double s0, double s1, double (*sh)[FS
   out[0] = sh[0][0], out[1] = sh[1][0];
   const bool good = *ok;
   __syncthreads();
-  if (tid < 2) store_out(slot(epoch + 2, blockIdx.x) + tid, __longlong_as_double((long long)BICG_EMPTY));
+  if (tid < 2) store_out(bicg_slot(part, epoch + 2, blockIdx.x) + tid, __longlong_as_double((long long)BICG_EMPTY));
   ++epoch;
   return good;
 }
@@ -702,6 +708,7 @@ struct BicgArgs {
   double grav, coef, tol;
   int zero_u, maxit;
   double *res, *Ap;    // the published vectors
+  double* cs;          // squared wave speed of every cell (fs_bicg_large_kernel)
   double* out;         // the solution's masters
   const double* rw;    // reduction weight of every master
   double *scal, *part;
@@ -717,7 +724,7 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
   const double *u = mem(a.u, a.ms), *f = mem(a.f, a.ms), *eo = mem(a.eo, a.ms);
   double *const res = mem(a.res, a.ms), *const Apv = mem(a.Ap, a.ms), *const out = mem(a.out, a.ms);
   double* const scal = mem(a.scal, SC_NSCAL);
-  double* const part = mem(a.part, (int64_t)6 * BICG_BLOCKS);
+  double* const part = mem(a.part, (int64_t)6 * BICG_SLOTS);
   const int t = blockIdx.x * FS_NT + threadIdx.x;
   const bool live = t < a.n;
   const int64_t c = a.ncl[2 * (live ? t : 0) + 1];
@@ -809,6 +816,275 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// fs_bicg_large_kernel: the same for the levels above, up to BL_K * 512 blocks of
+// the launches' reductions (J7 and J8), with one block of 512 threads to every
+// compute unit.  A block owns the masters that two neighbouring blocks of the
+// launches' reductions sum (2 x 256 masters in a row, and on every 512 x 256
+// from there), so the sums are theirs to the last bit.  The owned vectors live
+// in registers, the operand of the stencil in LDS, and so do the residual, Ap and
+// direction of the masters around the owned ones (the ring), which are read
+// once after their reduction; the operator comes from memory (L2 and the
+// memory-side cache) in each apply.
+// Bound by the operator's planes from there (8 planes, two passes an iteration:
+// 21 of 50 us at J8 at the rate of a large copy) and the three reductions.  An
+// iteration by launches -> in here: J7 52.8 -> 27.6 us, J8 99.8 -> 50.5.  All of
+// a row's loads go out before the row ahead of it is computed; left to the
+// compiler, which waits for each, J8 took 78 us.
+// ---------------------------------------------------------------------------
+// a plane read at one byte offset per lane plus a scalar one: a stencil's
+// addresses then cost no vector instruction
+using Plane = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ Plane plane_of(const double* p) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00027000);
+}
+__device__ __forceinline__ double ldb(Plane p, uint32_t lane, uint32_t off) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(p, lane, off, 0));
+}
+
+constexpr int BL_NT = 512, BL_K = 6, BL_OWN = BL_K * BL_NT, BL_RING = 2816;
+constexpr int BL_RK = (BL_RING + BL_NT - 1) / BL_NT;
+constexpr int BL_ZERO = BL_OWN + BL_RING;  // row of a neighbour outside the grid
+
+struct BlPlan {
+  const unsigned* nb;  // [block][3][BL_OWN]: rows of the six neighbours, two a word
+  const int* ring;     // [block][BL_RING]: cells
+  const int* nring;    // [block]
+};
+
+// reduce_out over two halves of a block, each a block of the launches' reductions
+__device__ __forceinline__ bool reduce_large(double s0, double s1, int nb, double (*sh)[2][FS_NT], double* part,
+                                             unsigned& epoch, int* ok, double out[2]) {
+  const int tid = threadIdx.x, half = tid / FS_NT, t = tid % FS_NT;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have left
+  auto tree = [&](int h, bool mine) {  // block_tree's order
+    for (int s = FS_NT / 2; s >= 64; s >>= 1) {
+      if (mine && t < s)
+        for (int k = 0; k < 2; ++k) sh[h][k][t] = sh[h][k][t] + sh[h][k][t + s];
+      __syncthreads();
+    }
+    if (mine && t < 64) {
+      double v[2] = {sh[h][0][t], sh[h][1][t]};
+      for (int s = 32; s > 0; s >>= 1)
+        for (int k = 0; k < 2; ++k) v[k] = v[k] + __shfl_down(v[k], s, 64);
+      if (t == 0) sh[h][0][0] = v[0], sh[h][1][0] = v[1];
+    }
+    __syncthreads();
+  };
+  sh[half][0][t] = s0, sh[half][1][t] = s1;
+  __syncthreads();
+  tree(half, true);
+  const int me = 2 * xcd_block() + half;
+  if (t < 2 && me < nb) bicg_post(bicg_slot(part, epoch, me) + t, sh[half][t][0]);
+  double v0 = 0.0, v1 = 0.0;
+  if (tid < nb) bicg_wait(bicg_slot(part, epoch, tid), ok, v0, v1);
+  __syncthreads();  // sh is free again
+  sh[half][0][t] = v0, sh[half][1][t] = v1;
+  __syncthreads();
+  if (half == 0) {
+    for (int k = 0; k < 2; ++k) {
+      double acc = 0.0 + sh[0][k][t];
+      if (t + FS_NT < nb) acc = acc + sh[1][k][t];
+      sh[0][k][t] = acc;
+    }
+  }
+  __syncthreads();
+  tree(0, half == 0);
+  out[0] = sh[0][0][0], out[1] = sh[0][1][0];
+  const bool good = *ok;
+  __syncthreads();
+  if (t < 2 && me < nb)
+    store_out(bicg_slot(part, epoch + 2, me) + t, __longlong_as_double((long long)BICG_EMPTY));
+  ++epoch;
+  return good;
+}
+
+__global__ __launch_bounds__(BL_NT, 2) void fs_bicg_large_kernel(BicgArgs a, BlPlan plan, int nb) {
+  __shared__ double sh[2][2][FS_NT];
+  __shared__ double x[BL_ZERO + 1], rp[BL_RING], rr[BL_RING], rA[BL_RING], r0[BL_OWN];
+  __shared__ int ok;
+  const int tid = threadIdx.x, B = xcd_block();
+  if (tid == 0) {
+    ok = 1;
+    x[BL_ZERO] = 0.0;
+  }
+  const FsGeo g = a.g;
+  const int nring = plan.nring[B];
+  // the operator's planes, from the south-west neighbour of their first cell on
+  const Plane cs = plane_of(a.cs - (g.S + 1)), hv = plane_of(g.hinv - (g.S + 1)), l0 = plane_of(g.lenf - (g.S + 1)),
+              l1 = plane_of(g.lenf + g.NC - (g.S + 1)), l2 = plane_of(g.lenf + 2 * g.NC - (g.S + 1)),
+              e0 = plane_of(g.pedf - (g.S + 1)), e1 = plane_of(g.pedf + g.NC - (g.S + 1)),
+              e2 = plane_of(g.pedf + 2 * g.NC - (g.S + 1));
+  int rc[BL_RK];
+  for (int m = 0; m < BL_RK; ++m) rc[m] = plan.ring[(int64_t)B * BL_RING + min(tid + m * BL_NT, nring - 1)];
+  // rows in use: the launches' block `me` sums the masters me * 256 + t, + nb * 256, ...
+  const int me = 2 * B + tid / FS_NT, i0 = me * FS_NT + tid % FS_NT;
+  int c[BL_K], nbr[BL_K][3];
+  double w[BL_K], p[BL_K], r[BL_K], Ap[BL_K], As[BL_K];
+  bool live[BL_K];
+  int nk = 0;  // uniform over the block
+  for (int k = 0; k < BL_K; ++k) nk += (2 * B + nb * k) * FS_NT < a.n;
+#define EACH_ROW                                                                                                      \
+  _Pragma("unroll") for (int k = 0; k < BL_K; ++k) if (k < nk)
+#pragma unroll
+  for (int k = 0; k < BL_K; ++k) {
+    const int i = i0 + nb * k * FS_NT;
+    live[k] = me < nb && i < a.n;
+    c[k] = (int)a.ncl[2 * (int64_t)(live[k] ? i : 0) + 1];
+    w[k] = live[k] ? a.rw[i] : 0.0;
+    for (int q = 0; q < 3; ++q) nbr[k][q] = (int)plan.nb[((int64_t)B * 3 + q) * BL_OWN + k * BL_NT + tid];
+  }
+  // the operator at a row (all its loads at once) and its application
+  struct Row {
+    double cs[7], len[6], ped[6], hv;
+  };
+  const uint32_t at = (g.S + 1) * 8;
+  auto load = [&](int k) {
+    const uint32_t y = (uint32_t)c[k] * 8;
+    return Row{{ldb(cs, y, at), ldb(cs, y, at + 8), ldb(cs, y, at - 8), ldb(cs, y, 0), ldb(cs, y, 2 * at),
+                ldb(cs, y, 2 * at - 8), ldb(cs, y, 8)},
+               {ldb(l0, y, at), ldb(l0, y, at - 8), ldb(l1, y, 0), ldb(l1, y, at), ldb(l2, y, at), ldb(l2, y, 8)},
+               {ldb(e0, y, at), ldb(e0, y, at - 8), ldb(e1, y, 0), ldb(e1, y, at), ldb(e2, y, at), ldb(e2, y, 8)},
+               ldb(hv, y, at)};
+  };
+  auto apply = [&](int k, const Row& o) {
+    double q[7];
+    q[0] = x[k * BL_NT + tid];
+    for (int j = 0; j < 3; ++j) q[2 * j + 1] = x[nbr[k][j] & 0xffff], q[2 * j + 2] = x[(unsigned)nbr[k][j] >> 16];
+    auto flux = [&](int e, double d) { return interp(o.cs[0], o.cs[e + 1]) * d / o.len[e] * o.ped[e]; };
+    const double dv = (flux(0, q[1] - q[0]) - flux(1, q[0] - q[4]) + flux(2, q[5] - q[0]) - flux(3, q[0] - q[2]) +
+                       flux(4, q[3] - q[0]) - flux(5, q[0] - q[6])) *
+                      o.hv;
+    return a.coef * dv - q[0];
+  };
+  // v = L x: each row's loads are under way while the row before is computed
+  auto apply_all = [&](double v[BL_K], Row o) {
+#pragma unroll
+    for (int k = 0; k < BL_K; ++k)
+      if (k < nk) {
+        const Row next = load(k + 1 < BL_K ? k + 1 : k);
+        __builtin_amdgcn_sched_barrier(0);
+        v[k] = apply(k, o);
+        o = next;
+      }
+  };
+  unsigned epoch = 0;
+  double sum[2];
+  bool good = true;
+  auto sums = [&](double s0, double s1) {
+    return reduce_large(s0, s1, nb, sh, a.part, epoch, &ok, sum);
+  };
+  // res = f - L u; nrm_f = l2(f); rho = dp(res0, res)
+  double s0 = 0.0, s1 = 0.0;
+  EACH_ROW {
+    if (live[k]) {
+      const double fc = a.f[c[k]];
+      a.out[c[k]] = a.zero_u ? 0.0 : a.u[c[k]];
+      r[k] = a.zero_u ? fc - 0.0 : fc - ell_apply_at(g, a.u, a.eo, a.grav, a.coef, (int64_t)c[k]);
+      store_out(a.res + c[k], r[k]);
+      s0 = s0 + w[k] * (fc * fc);
+      s1 = s1 + w[k] * (r[k] * r[k]);
+    } else {
+      r[k] = 0.0;
+    }
+    p[k] = r0[k * BL_NT + tid] = r[k];
+  }
+  good = sums(s0, s1);
+  const double nf = sqrt(sum[0]), nrmf = nf == 0.0 ? 1.0 : nf;
+  double rho = sum[1], err = 0.0;
+  double rv[BL_RK];  // a reduction's ring values: all loads, then their use
+  auto gather = [&](const double* v) {
+#pragma unroll
+    for (int m = 0; m < BL_RK; ++m)
+      if (m * BL_NT < nring) rv[m] = load_out(v + rc[m]);
+  };
+#define EACH_RING                                                                                                     \
+  _Pragma("unroll") for (int m = 0; m < BL_RK; ++m) if (const int q = tid + m * BL_NT; q < nring)
+  gather(a.res);
+  EACH_RING rr[q] = rp[q] = x[BL_OWN + q] = rv[m];
+  EACH_ROW x[k * BL_NT + tid] = p[k];
+  __syncthreads();
+  apply_all(Ap, load(0));
+  int iter = 1;
+  bool done = false;
+  for (; good && iter <= a.maxit; ++iter) {
+    s0 = 0.0;
+    EACH_ROW if (live[k]) {
+      store_out(a.Ap + c[k], Ap[k]);
+      s0 = s0 + w[k] * (Ap[k] * r0[k * BL_NT + tid]);
+    }
+    good = sums(s0, 0.0);
+    const double alph = rho / sum[0], ma = -1.0 * alph;
+    gather(a.Ap);
+    EACH_RING {
+      rA[q] = rv[m];
+      x[BL_OWN + q] = 1.0 * rr[q] + ma * rv[m];
+    }
+    EACH_ROW x[k * BL_NT + tid] = 1.0 * r[k] + ma * Ap[k];
+    __syncthreads();
+    s0 = s1 = 0.0;
+    apply_all(As, load(0));
+    EACH_ROW {
+      if (live[k]) {
+        s0 = s0 + w[k] * (As[k] * x[k * BL_NT + tid]);
+        s1 = s1 + w[k] * (As[k] * As[k]);
+      }
+    }
+    good = good && sums(s0, s1);
+    const double omga = sum[0] / sum[1], mo = -1.0 * omga;
+    s0 = s1 = 0.0;
+    EACH_ROW {
+      const double sc = x[k * BL_NT + tid], corr = (1.0 * alph) * p[k] + (1.0 * omga) * sc;
+      r[k] = 1.0 * sc + mo * As[k];
+      if (live[k]) {
+        a.out[c[k]] = 1.0 * a.out[c[k]] + 1.0 * corr;
+        store_out(a.res + c[k], r[k]);
+        s0 = s0 + w[k] * (r[k] * r[k]);
+        s1 = s1 + w[k] * (r0[k * BL_NT + tid] * r[k]);
+      }
+    }
+    good = good && sums(s0, s1);
+    err = sqrt(sum[0]) / nrmf;
+    if (err <= a.tol) {
+      done = true;
+      break;
+    }
+    const double rho_old = rho;
+    rho = sum[1];
+    const double b = (alph / omga) * (rho / rho_old), bb = 1.0 * b;
+    gather(a.res);
+    EACH_RING {
+      const double cr = 1.0 * rp[q] + mo * rA[q], pn = 1.0 * rv[m] + bb * cr;
+      rr[q] = rv[m], rp[q] = pn, x[BL_OWN + q] = pn;
+    }
+    EACH_ROW {
+      const double cr = 1.0 * p[k] + mo * Ap[k];
+      p[k] = 1.0 * r[k] + bb * cr;
+      x[k * BL_NT + tid] = p[k];
+    }
+    __syncthreads();
+    apply_all(Ap, load(0));
+  }
+  if (!good) {
+    if (tid == 0) a.scal[SC_FAIL] = 1.0;
+    return;
+  }
+#undef EACH_ROW
+#undef EACH_RING
+  if (B == 0 && tid == 0) {
+    a.scal[SC_NRMF] = nrmf;
+    a.scal[SC_ERR] = err;
+    a.scal[SC_ITER] = (double)(done ? iter : a.maxit);
+    a.scal[SC_DONE] = done ? 1.0 : 0.0;
+  }
+}
+
+__global__ void fs_speed_kernel(int64_t n, const double* __restrict__ topo, const double* __restrict__ eo, double grav,
+                                double* __restrict__ cs) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) cs[t] = grav * (fabs(topo[t]) * 1.0 + eo[t]);
+}
+
 // u = the solution of fs_bicg_solve_kernel, masters and halo copies; its
 // slots empty for the next launch
 __global__ void fs_bicg_out_kernel(int n, const int64_t* __restrict__ ncl, const double* __restrict__ out,
@@ -816,7 +1092,7 @@ __global__ void fs_bicg_out_kernel(int n, const int64_t* __restrict__ ncl, const
                                    int64_t ms) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t == 0) mem(scal, SC_NSCAL)[SC_FAIL] = 0.0;
-  if (t < 6 * BICG_BLOCKS) mem(part, (int64_t)6 * BICG_BLOCKS)[t] = __longlong_as_double((long long)BICG_EMPTY);
+  if (t < 6 * BICG_SLOTS) mem(part, (int64_t)6 * BICG_SLOTS)[t] = __longlong_as_double((long long)BICG_EMPTY);
   if (t >= n) return;
   mem(u, ms)[ncl[2 * t]] = mem(out, ms)[ncl[2 * t + 1]];
 }
@@ -1135,6 +1411,80 @@ FsGeo fs_geo(const wtg_ctx* c) {
   return FsGeo{c->d_lenf, c->d_pedf, c->d_hinv, c->d_topo, c->info.ncells, c->info.S};
 }
 
+// what the one-launch BiCGSTAB of a level needs, for levels that have one
+int bicg_plan(wtg_ctx* c) {
+  const int nchunk = (int)nblk(c->nmaster), nb = std::min(RED_BLOCKS, nchunk);
+  const int64_t NC = c->info.ncells, S = c->info.S;
+  int dev = 0, ncu = 0;
+  WTG_HIPCHK(c, hipGetDevice(&dev));
+  WTG_HIPCHK(c, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
+  // blocks that must run together: one to a compute unit
+  c->bicg_blocks = std::min(BICG_BLOCKS, ncu);
+  const bool large = nchunk > BICG_BLOCKS;
+  if (!c->red_masters || nchunk > BL_K * RED_BLOCKS || (large ? (nb + 1) / 2 : nchunk) > ncu) return 0;
+  std::vector<int> src(NC), ring, nring, row;
+  std::vector<unsigned> nbr;
+  for (int64_t x = 0; x < NC; ++x) src[x] = (int)(c->node_src[x] >= 0 ? c->node_src[x] : x);
+  if (large) {
+    const int64_t off[6] = {1, S + 1, S, -1, -S - 1, -S};
+    std::vector<int64_t> ncl(2 * (size_t)c->nmaster);
+    WTG_HIPCHK(c, hipMemcpy(ncl.data(), c->d_ncl, ncl.size() * sizeof(int64_t), hipMemcpyDeviceToHost));
+    const int nblocks = (nb + 1) / 2;
+    ring.assign((size_t)nblocks * BL_RING, 0);
+    nring.assign(nblocks, 0);
+    row.assign(NC, -1);
+    nbr.assign((size_t)nblocks * 3 * BL_OWN, BL_ZERO | (unsigned)BL_ZERO << 16);
+    for (int B = 0; B < nblocks; ++B) {
+      std::vector<std::pair<int, int>> own;  // (row, cell)
+      for (int k = 0; k < BL_K; ++k)
+        for (int t = 0; t < BL_NT; ++t) {
+          const int me = 2 * B + t / FS_NT, i = (me + nb * k) * FS_NT + t % FS_NT;
+          if (me < nb && i < c->nmaster) own.push_back({k * BL_NT + t, (int)ncl[2 * (size_t)i]});
+        }
+      for (const auto& o : own) row[o.second] = o.first;
+      int* const rc = &ring[(size_t)B * BL_RING];
+      int n = 0;
+      for (const auto& o : own)
+        for (int k = 0; k < 6; ++k) {
+          const int64_t y = c->node_src[o.second + off[k]];
+          if (y < 0 || row[y] >= 0) continue;
+          if (n == BL_RING) return 0;  // not for this grid
+          rc[n] = (int)y;
+          row[y] = BL_OWN + n++;
+        }
+      std::sort(rc, rc + n);
+      for (int q = 0; q < n; ++q) row[rc[q]] = BL_OWN + q;
+      for (const auto& o : own)
+        for (int k = 0; k < 6; ++k) {
+          const int64_t y = c->node_src[o.second + off[k]];
+          const unsigned id = y < 0 ? BL_ZERO : row[y];
+          unsigned& word = nbr[((size_t)B * 3 + k / 2) * BL_OWN + o.first];
+          word = k % 2 ? (word & 0xffffu) | id << 16 : (word & 0xffff0000u) | id;
+        }
+      nring[B] = n;
+      for (const auto& o : own) row[o.second] = -1;
+      for (int q = 0; q < n; ++q) row[rc[q]] = -1;
+    }
+    auto up = [&](auto** d, const auto& h) -> int {
+      using T = std::remove_const_t<std::remove_reference_t<decltype(h[0])>>;
+      if (int rc = wtg_dalloc<T>(c, d, h.size())) return rc;
+      WTG_HIPCHK(c, hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+      return 0;
+    };
+    if (int rc = up(&c->d_blnb, nbr)) return rc;
+    if (int rc = up(&c->d_blring, ring)) return rc;
+    if (int rc = up(&c->d_blnring, nring)) return rc;
+  } else {
+    if (int rc = wtg_dalloc<int>(c, &c->d_src, src.size())) return rc;
+    WTG_HIPCHK(c, hipMemcpy(c->d_src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
+  const std::vector<unsigned long long> empty((size_t)6 * BICG_SLOTS * c->nmembers, BICG_EMPTY);
+  if (int rc = wtg_dalloc<double>(c, &c->d_bpart, empty.size())) return rc;
+  WTG_HIPCHK(c, hipMemcpy(c->d_bpart, empty.data(), empty.size() * sizeof(double), hipMemcpyHostToDevice));
+  return 0;
+}
+
 int fs_ready(wtg_ctx* c) {
   if (!c) return WTG_E_ARG;
   if (!c->topo_set) return wtg_fail(c, WTG_E_STATE, "wtg_set_topography must be called first");
@@ -1152,18 +1502,7 @@ int fs_ready(wtg_ctx* c) {
   if (int rc = wtg_dalloc<double>(c, &c->d_scal, (size_t)SC_NSCAL * M)) return rc;
   WTG_HIPCHK(c, hipMemsetAsync(c->d_scal, 0, SC_NSCAL * M * sizeof(double), c->stream));
   WTG_HIPCHK(c, hipHostMalloc((void**)&c->h_scal, SC_NSCAL * M * sizeof(double), hipHostMallocDefault));
-  std::vector<int> src;
-  if (c->red_masters && nblk(c->nmaster) <= BICG_BLOCKS) {
-    src.resize(c->info.ncells);
-    for (int64_t x = 0; x < c->info.ncells; ++x) src[x] = (int)(c->node_src[x] >= 0 ? c->node_src[x] : x);
-    if (int rc = wtg_dalloc<int>(c, &c->d_src, src.size())) return rc;
-    const std::vector<unsigned long long> empty(6 * BICG_BLOCKS * M, BICG_EMPTY);
-    if (int rc = wtg_dalloc<double>(c, &c->d_bpart, empty.size())) return rc;
-    WTG_HIPCHK(c, hipMemcpy(c->d_bpart, empty.data(), empty.size() * sizeof(double), hipMemcpyHostToDevice));
-    WTG_HIPCHK(c, hipMemcpyAsync(c->d_src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-  }
-  WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
-  return 0;
+  return bicg_plan(c);
 }
 
 int fs_field(wtg_ctx* c, int f, int nuser = FS_NUSER) {
@@ -1291,14 +1630,14 @@ int read_scalar(wtg_ctx* c, int i, double* out) {
 // masters in place and its halo copies refreshed after the loop.
 constexpr int BICG_CHUNK = 8;
 
-// whether a solve on this level is one launch of fs_bicg_solve_kernel: one
-// block per 256 masters of every member, all resident at once with room for a
-// second such solve on another stream (a compute unit holds two blocks).  It is
-// the faster one wherever it fits; a context that replays graphs has asked for
-// the launches.
+// whether a solve on this level is one launch: fs_bicg_solve_kernel with a block
+// per 256 masters of every member, all resident at once with room for a second
+// such solve on another stream (a compute unit holds two blocks), or one
+// member's fs_bicg_large_kernel.  It is the faster one wherever it fits; a
+// context that replays graphs has asked for the launches.
 bool bicg_one_launch(const wtg_ctx* c, int maxit) {
-  return c->bicg_one && c->d_src && !c->fs_graph && maxit > 0 &&
-         (int64_t)nblk(c->nmaster) * c->nmembers <= BICG_BLOCKS;
+  return c->bicg_one && c->d_bpart && !c->fs_graph && maxit > 0 &&
+         (c->d_src ? (int64_t)nblk(c->nmaster) * c->nmembers <= c->bicg_blocks : c->nmembers == 1 && !c->mg_mdone);
 }
 
 int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int* iters, double* err_out,
@@ -1307,8 +1646,17 @@ int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int 
   const int M = c->nmembers;
   const int64_t ms = c->info.ncells;
   BicgArgs a{c->mg_mdone, c->nmaster, c->d_ncl, c->d_src, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav,
-             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[3], c->d_rw, c->d_scal, c->d_bpart, ms};
-  hipLaunchKernelGGL(fs_bicg_solve_kernel, dim3(nblk(c->nmaster), M), dim3(FS_NT), 0, c->stream, a);
+             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[5], W[3], c->d_rw, c->d_scal, c->d_bpart, ms};
+  if (c->d_src) {
+    hipLaunchKernelGGL(fs_bicg_solve_kernel, dim3(nblk(c->nmaster), M), dim3(FS_NT), 0, c->stream, a);
+  } else {
+    const int nb = std::min(RED_BLOCKS, (int)nblk(c->nmaster));
+    hipLaunchKernelGGL(fs_speed_kernel, dim3((unsigned)((ms + FS_NT - 1) / FS_NT)), dim3(FS_NT), 0, c->stream, ms,
+                       c->d_topo, c->fs[FS_ETA_OLD], c->params.grav, W[5]);
+    WTG_HIPCHK(c, hipGetLastError());
+    hipLaunchKernelGGL(fs_bicg_large_kernel, dim3((nb + 1) / 2), dim3(BL_NT), 0, c->stream, a,
+                       BlPlan{c->d_blnb, c->d_blring, c->d_blnring}, nb);
+  }
   WTG_HIPCHK(c, hipGetLastError());
   WTG_HIPCHK(c, hipMemcpyAsync(c->h_scal, c->d_scal, (size_t)SC_NSCAL * M * sizeof(double), hipMemcpyDeviceToHost,
                                c->stream));
@@ -1316,12 +1664,12 @@ int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int 
   bool failed = false;
   for (int m = 0; m < M; ++m) failed = failed || c->h_scal[m * SC_NSCAL + SC_FAIL] != 0.0;
   if (failed) {  // u is as it was; leave the slots empty and no failure behind
-    hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(nblk(6 * BICG_BLOCKS), M), dim3(FS_NT), 0, c->stream, 0, c->d_ncl,
+    hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(nblk(6 * BICG_SLOTS), M), dim3(FS_NT), 0, c->stream, 0, c->d_ncl,
                        W[3], u, c->d_bpart, c->d_scal, ms);
     WTG_HIPCHK(c, hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(std::max(nblk(c->nncl), nblk(6 * BICG_BLOCKS)), M), dim3(FS_NT), 0,
+  hipLaunchKernelGGL(fs_bicg_out_kernel, dim3(std::max(nblk(c->nncl), nblk(6 * BICG_SLOTS)), M), dim3(FS_NT), 0,
                      c->stream, c->nncl, c->d_ncl, W[3], u, c->d_bpart, c->d_scal, ms);
   WTG_HIPCHK(c, hipGetLastError());
   if (sync_end) WTG_HIPCHK(c, hipStreamSynchronize(c->stream));
