@@ -1108,10 +1108,11 @@ __global__ void fs_bicg_out_kernel(int n, const int64_t* __restrict__ ncl, const
 // Bound by the loads of the operator (15 doubles a master) and the rings' share
 // of them: 1.6 times the tile's masters for two rings, 2.6 times for five.
 // A V-cycle's smoothing (2 sweeps down and up, 4 after) as single sweeps -> in
-// here: cycles on levels J5-J7 249 -> 176 us, J5-J8 513 -> 302 us, of which the
+// here: cycles on levels J5-J7 249 -> 163 us, J5-J8 513 -> 286 us, of which the
 // coarse solve takes about 110.  Four sweeps with the residual take 20 us at J7
 // (11 each before).  The tiles of an XCD in a row instead of dealt out: 3 to
-// 6 % of a cycle.
+// 6 % of a cycle; the prolongation evaluated where its values are added instead
+// of in two launches: 6 to 8 %.
 // ---------------------------------------------------------------------------
 constexpr int SW_RINGS = 5;     // most rings of a launch
 constexpr int SW_ROWS = 768;    // most masters of a block and its rings
@@ -1130,7 +1131,9 @@ struct SwArgs {
   const double* mdone;
   SwPlan plan;
   FsGeo g;
-  const F *u, *add, *f;  // the sweeps start from u (null: 0), or u + add
+  const F *u, *add, *f;  // the sweeps start from u (null: 0), or u + add,
+  const F* coarse;       // or u + the prolongation of coarse (mg_prolong0)
+  MgGeo mg;
   const double* eo;
   double grav, coef, dt2, th12, w;
   int n, rings;          // sweeps; rings they and the residual need
@@ -1152,7 +1155,11 @@ __global__ __launch_bounds__(NT, NT > SW_SMALL ? 3 : 4) void fs_sweeps_kernel(Sw
   double r = 0.0;
   if (live && a.u) {
     const F* const u = mem(a.u, a.ms);
-    r = a.add && !done ? (double)(F)(1.0 * u[c] + 1.0 * mem(a.add, a.ms)[c]) : (double)u[c];
+    r = (double)u[c];
+    if (!done && (a.add || a.coarse)) {
+      const F e = a.add ? mem(a.add, a.ms)[c] : mg_prolong0(a.mg, mem(a.coarse, a.mg.NCc), c);
+      r = (double)(F)(1.0 * r + 1.0 * e);
+    }
   }
   if (!done) {
     const double* const eo = mem(a.eo, a.ms);
@@ -1954,6 +1961,13 @@ struct MgLv {
   double *u, *u_alt, *f, *res, *res_alt, *corr, *corr_alt;
 };
 
+// zero-wavelet prolongation (prolong / prol_fun, lin_solve.f90:244-269) of
+// level l - 1's coarse field into level l
+template <class F>
+int lv_prolong0(wtg_mg* m, int l, const F* coarse, F* fine) {
+  return mg_inverse<F, true>(m, l, coarse, nullptr, fine);
+}
+
 // the tiles of fs_sweeps_kernel on a level (once, when its hierarchy is made)
 int sw_plan(wtg_ctx* c) {
   if (c->sw_state) return 0;
@@ -2051,9 +2065,21 @@ int sw_plan(wtg_ctx* c) {
   return 0;
 }
 
+// a level's correction from the coarser one
 template <class F>
-int launch_sweeps(wtg_ctx* c, const F* u, const F* add, const F* f, double w, int n, int rings, F* out, F* res) {
-  SwArgs<F> a{c->mg_mdone, SwPlan{c->d_swcnt, c->d_swcell, c->d_swnb, c->d_swhalo}, fs_geo(c), u, add, f,
+struct MgAdd {
+  const F* field = nullptr;   // on the level, or
+  wtg_mg* m = nullptr;        // of level l - 1, prolonged to l with zero wavelets
+  int l = 0;
+  const F* coarse = nullptr;
+  F* fine = nullptr;          // where the prolongation goes if it is not done in passing
+};
+
+template <class F>
+int launch_sweeps(wtg_ctx* c, const F* u, const MgAdd<F>& add, const F* f, double w, int n, int rings, F* out,
+                  F* res) {
+  SwArgs<F> a{c->mg_mdone, SwPlan{c->d_swcnt, c->d_swcell, c->d_swnb, c->d_swhalo}, fs_geo(c), u, add.field, f,
+              add.coarse, add.coarse ? mg_geo(add.m, add.l) : MgGeo{},
               c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c), c->fs_dt * c->fs_dt, c->fs_theta1 * c->fs_theta2, w, n,
               rings, out, res, c->info.ncells};
   const int nt = (c->sw_rows[rings] + 63) / 64 * 64;
@@ -2069,18 +2095,22 @@ int launch_sweeps(wtg_ctx* c, const F* u, const F* add, const F* f, double w, in
 template <class F>
 int lv_jacobi(MgLv& v, F*& u, F*& alt, const F* f, double w, int n);
 
-// u := n Jacobi sweeps from u (zero: from 0; add: from u + add), and
+// u := n Jacobi sweeps from u (zero: from 0; else from u + add), and
 // res := f - L u if asked for
 template <class F>
-int lv_sweeps(MgLv& v, F*& u, F*& alt, bool zero, const F* add, const F* f, double w, int n, F* res) {
+int lv_sweeps(MgLv& v, F*& u, F*& alt, bool zero, MgAdd<F> add, const F* f, double w, int n, F* res) {
   wtg_ctx* c = v.c;
   if (zero && n == 0) {
     RC(mg_fill(c, u, 0.0));
     zero = false;
   }
   if (c->sw_state <= 0) {
-    if (add) {
-      RC(launch_lc(c, 1.0, -1, (const F*)u, 1.0, -1, add, alt));
+    if (add.coarse) {
+      RC(lv_prolong0(add.m, add.l, add.coarse, add.fine));
+      add.field = add.fine;
+    }
+    if (add.field) {
+      RC(launch_lc(c, 1.0, -1, (const F*)u, 1.0, -1, add.field, alt));
       std::swap(u, alt);
     }
     if (zero) {
@@ -2099,7 +2129,7 @@ int lv_sweeps(MgLv& v, F*& u, F*& alt, bool zero, const F* add, const F* f, doub
     const bool last = k == n && rings + (res ? 1 : 0) <= SW_RINGS;
     RC(launch_sweeps(c, start, add, f, w, k, rings + (last && res ? 1 : 0), alt, last ? res : (F*)nullptr));
     std::swap(u, alt);
-    start = u, add = nullptr, n -= k;
+    start = u, add = {}, n -= k;
     if (last) return 0;
   } while (true);
 }
@@ -2136,13 +2166,6 @@ int lv_l2(MgLv& v, const double* a, double* out) {
   return 0;
 }
 
-// zero-wavelet prolongation (prolong / prol_fun, lin_solve.f90:244-269) of
-// level l - 1's coarse field into level l
-template <class F>
-int lv_prolong0(wtg_mg* m, int l, const F* coarse, F* fine) {
-  return mg_inverse<F, true>(m, l, coarse, nullptr, fine);
-}
-
 std::vector<MgLv> mg_levels(wtg_mg* m) {
   std::vector<MgLv> V(m->nl);
   for (int l = 0; l < m->nl; ++l) {
@@ -2177,7 +2200,7 @@ int vcycle(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, doubl
   for (int j = l; j >= 1; --j) {
     const double* rhs = j == l && r_in ? r_in : V[j].res;
     // from corr = 0; res := res - L corr
-    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, true, (const double*)nullptr, rhs, 1.0, P.down_iter, V[j].res_alt));
+    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, true, {}, rhs, 1.0, P.down_iter, V[j].res_alt));
     std::swap(V[j].res, V[j].res_alt);
     RC(mg_forward(m, j, V[j].res, V[j].c->fs[MG_WC], V[j - 1].res));
   }
@@ -2185,13 +2208,12 @@ int vcycle(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, doubl
   double cerr;
   RC(bicgstab(V[0].c, V[0].corr, V[0].res, P.coarse_tol, P.coarse_iter, &cit, &cerr, true, false));
   for (int j = 1; j <= l; ++j) {
-    double* pf = V[j].c->fs[MG_PF];
-    RC(lv_prolong0(m, j, (const double*)V[j - 1].corr, pf));
-    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, false, (const double*)pf, (const double*)V[j].res, 1.0, P.up_iter,
+    const MgAdd<double> up{nullptr, m, j, V[j - 1].corr, V[j].c->fs[MG_PF]};
+    RC(lv_sweeps(V[j], V[j].corr, V[j].corr_alt, false, up, (const double*)V[j].res, 1.0, P.up_iter,
                  (double*)nullptr));
   }
   double* r = V[l].c->fs[FS_W0];
-  RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, (const double*)V[l].corr, (const double*)V[l].f, 1.0, P.post_iter, r));
+  RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, MgAdd<double>{V[l].corr}, (const double*)V[l].f, 1.0, P.post_iter, r));
   if (m->M > 1) return 0;  // member-batched cycles test every member's residual in the caller
   return lv_err(V[l], r, nrm_f, err);
 }
@@ -2236,7 +2258,7 @@ int vcycle32(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, dou
   for (int j = l; j >= 1; --j) {
     const float* rhs = j == l ? R : res[j];
     // from corr = 0; res := rhs - L corr
-    RC(lv_sweeps(V[j], corr[j], corr_alt[j], true, (const float*)nullptr, rhs, 1.0, P.down_iter, res_alt[j]));
+    RC(lv_sweeps(V[j], corr[j], corr_alt[j], true, {}, rhs, 1.0, P.down_iter, res_alt[j]));
     std::swap(res[j], res_alt[j]);
     RC(mg_forward(m, j, (const float*)res[j], V[j].c->fs32[M32_WC], res[j - 1]));
   }
@@ -2246,12 +2268,10 @@ int vcycle32(wtg_mg* m, std::vector<MgLv>& V, int l, const wtg_mg_params& P, dou
   RC(bicgstab(V[0].c, V[0].corr, V[0].res, P.coarse_tol, P.coarse_iter, &cit, &cerr, true, false));
   RC(launch_copy(V[0].c, (const double*)V[0].corr, corr[0]));
   for (int j = 1; j <= l; ++j) {
-    float* pf = V[j].c->fs32[M32_PF];
-    RC(lv_prolong0(m, j, (const float*)corr[j - 1], pf));
-    RC(lv_sweeps(V[j], corr[j], corr_alt[j], false, (const float*)pf, (const float*)res[j], 1.0, P.up_iter,
-                 (float*)nullptr));
+    const MgAdd<float> up{nullptr, m, j, corr[j - 1], V[j].c->fs32[M32_PF]};
+    RC(lv_sweeps(V[j], corr[j], corr_alt[j], false, up, (const float*)res[j], 1.0, P.up_iter, (float*)nullptr));
   }
-  RC(lv_sweeps(V[l], corr[l], corr_alt[l], false, (const float*)nullptr, (const float*)R, 1.0, P.post_iter,
+  RC(lv_sweeps(V[l], corr[l], corr_alt[l], false, {}, (const float*)R, 1.0, P.post_iter,
                (float*)nullptr));
   RC(launch_lc(V[l].c, 1.0, -1, (const double*)V[l].u, 1.0, -1, (const float*)corr[l], V[l].u_alt));
   std::swap(V[l].u, V[l].u_alt);
@@ -2274,7 +2294,7 @@ int mg_fmg(wtg_mg* m, const wtg_mg_params& P, int* iters, double* res_out) {
   for (int l = 1; l < nl; ++l) {
     if (nrm1[l] < P.fine_tol) continue;
     RC(lv_prolong0(m, l, (const double*)V[l - 1].u, V[l].u));
-    RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, (const double*)nullptr, (const double*)V[l].f, 1.0, P.pre_iter,
+    RC(lv_sweeps(V[l], V[l].u, V[l].u_alt, false, {}, (const double*)V[l].f, 1.0, P.pre_iter,
                  (double*)nullptr));
     for (int it = 1; it <= P.max_vcycle; ++it) {
       RC(vcycle(m, V, l, P, nrm_f[l], &res_out[l]));

@@ -44,6 +44,23 @@ __device__ __forceinline__ double mg_interp(const MgGeo& g, const F* __restrict_
          g.hinv_f[x];
 }
 
+// value at fine cell x of the inverse transform of coarse field s with all
+// wavelets zero (prol_fun): the parent's at a coincident cell, else mg_interp of
+// the four parents'
+template <class F>
+__device__ __forceinline__ F mg_prolong0(const MgGeo& g, const F* __restrict__ s, int64_t x) {
+  int lz, i, j;
+  mg_ij(x, g.Sf, lz, i, j);
+  const F* const sl = s + (int64_t)lz * g.Sc * g.Sc + 2 * g.Sc + 2;
+  auto at = [&](int di, int dj) { return sl[(int64_t)((j + dj) / 2) * g.Sc + (i + di) / 2]; };
+  if (!((i | j) & 1)) return at(0, 0);
+  const bool rt = !(j & 1), up = !(i & 1);
+  const int64_t NC = g.NCf;
+  const double s1 = rt ? at(-1, 0) : up ? at(0, -1) : at(1, 1), s2 = rt ? at(1, 0) : up ? at(0, 1) : at(-1, -1),
+               s3 = rt ? at(1, 2) : up ? at(-2, -1) : at(1, -1), s4 = rt ? at(-1, -2) : up ? at(2, 1) : at(-1, 1);
+  return (F)((g.ovl[x] * s1 + g.ovl[NC + x] * s2 + g.ovl[2 * NC + x] * s3 + g.ovl[3 * NC + x] * s4) * g.hinv_f[x]);
+}
+
 // lifting around fine coincident cell c (Restrict_scalar wavelet.f90:542-567,
 // twelve terms; Prolong_scalar 586-611 omits id2NE)
 template <class F>
