@@ -111,7 +111,7 @@ __device__ __forceinline__ double ell_diag_at(const FsGeo& g, const double* __re
 __global__ void fs_apply_kernel(const double* __restrict__ gate, int n, const int64_t* __restrict__ ncl, FsGeo g,
                                 const double* __restrict__ q, const double* __restrict__ eo, double grav, double coef,
                                 double* __restrict__ out, double* __restrict__ out2, int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), q = mem(q, ms), eo = mem(eo, ms), out = mem(out, ms), out2 = mem(out2, ms);
@@ -126,7 +126,7 @@ __global__ void fs_bicg_init_kernel(int n, const int64_t* __restrict__ ncl, FsGe
                                     const double* __restrict__ f, const double* __restrict__ eo, double grav,
                                     double coef, int zero_u, double* __restrict__ res, double* __restrict__ res0,
                                     double* __restrict__ p, double* __restrict__ s, int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms);
   res = mem(res, ms), res0 = mem(res0, ms), p = mem(p, ms), s = mem(s, ms);
@@ -155,7 +155,7 @@ __global__ void fs_jacobi_kernel(const double* __restrict__ mdone, int n, const 
                                  const F* __restrict__ u, const F* __restrict__ f, const double* __restrict__ eo,
                                  double grav, double coef, double dt2, double th12, double w, F* __restrict__ out,
                                  int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms), out = mem(out, ms);
   const int64_t c = ncl[2 * t + 1];
@@ -178,7 +178,7 @@ __global__ void fs_residual_kernel(const double* __restrict__ mdone, int n, cons
                                    const Fu* __restrict__ u, const Ff* __restrict__ f,
                                    const double* __restrict__ eo, double grav, double coef, Fo* __restrict__ out,
                                    int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms), out = mem(out, ms);
   const int64_t c = ncl[2 * t + 1];
@@ -249,7 +249,7 @@ __global__ void fs_edge_flux_kernel(int nlz, FsGeo g, int L, const double* __res
                                     const double* __restrict__ u, double* __restrict__ F0, double* __restrict__ F1,
                                     double* __restrict__ F2) {
   const int w = nlz + 2;  // cells per row and rows per lozenge in the pass
-  const int64_t t = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)list_block() * blockDim.x + threadIdx.x;
   if (t >= (int64_t)10 * w * w) return;
   const int lz = (int)(t / ((int64_t)w * w)), r = (int)(t % ((int64_t)w * w));
   const int i = r % w - 1, j = r / w - 1;
@@ -262,7 +262,7 @@ __global__ void fs_edge_flux_kernel(int nlz, FsGeo g, int L, const double* __res
 __global__ void fs_div_kernel(int n, const int64_t* __restrict__ ncl, FsGeo g, const double* __restrict__ F0,
                               const double* __restrict__ F1, const double* __restrict__ F2,
                               double* __restrict__ out) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t c = ncl[2 * t + 1];
   const int64_t cW = c - 1, cSW = c - g.S - 1, cS = c - g.S;
@@ -542,7 +542,7 @@ __global__ void fs_bicg_s_apply_kernel(const double* __restrict__ gate, int n, c
                                        const double* __restrict__ eo, double grav, double coef,
                                        const double* __restrict__ scal, double* __restrict__ s_out,
                                        double* __restrict__ As_out, int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), res = mem(res, ms), Ap = mem(Ap, ms), eo = mem(eo, ms);
@@ -563,7 +563,7 @@ __global__ void fs_bicg_p_apply_kernel(const double* __restrict__ gate, int n, c
                                        const double* __restrict__ Ap, const double* __restrict__ eo, double grav,
                                        double coef, const double* __restrict__ scal, double* __restrict__ pn_out,
                                        double* __restrict__ Apn_out, int64_t ms) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), res = mem(res, ms), p = mem(p, ms), Ap = mem(Ap, ms), eo = mem(eo, ms);
@@ -1238,7 +1238,7 @@ __global__ __launch_bounds__(NT, NT > SW_SMALL ? 3 : 4) void fs_sweeps_kernel(Sw
 template <class F>
 __global__ void mg_wavelet_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl, MgGeo g,
                                   const F* __restrict__ s, F* __restrict__ wc) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   s = mem(s, g.NCf), wc = mem(wc, g.NCf);
   const int64_t x = ncl[2 * t + 1];
@@ -1282,7 +1282,7 @@ template <class F, bool ZeroW = false>
 __global__ void mg_prolong_even_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl,
                                        MgGeo g, const F* __restrict__ sc, const F* __restrict__ wc,
                                        F* __restrict__ sf) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   sc = mem(sc, g.NCc), wc = mem(wc, g.NCf), sf = mem(sf, g.NCf);
   const int64_t x = ncl[2 * t + 1];
@@ -1305,7 +1305,7 @@ __global__ void mg_prolong_even_kernel(const double* __restrict__ mdone, int n, 
 template <class F, bool ZeroW = false>
 __global__ void mg_prolong_odd_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl,
                                       MgGeo g, const F* __restrict__ wc, F* __restrict__ sf) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   wc = mem(wc, g.NCf), sf = mem(sf, g.NCf);
   const int64_t x = ncl[2 * t + 1];

@@ -101,7 +101,7 @@ constexpr int ML_KCV = 1;
 __global__ void ml_scalar_wavelet_kernel(int n, const int64_t* __restrict__ ncl, MgGeo g, int L,
                                          const double* __restrict__ sm, const double* __restrict__ st,
                                          double* __restrict__ wc) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -118,7 +118,7 @@ __global__ void ml_restrict_scalar_kernel(int n, const int64_t* __restrict__ ncl
                                           const double* __restrict__ fm, const double* __restrict__ ft,
                                           const double* __restrict__ wc, double* __restrict__ cm,
                                           double* __restrict__ ct, int64_t NCc) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t p = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -140,7 +140,7 @@ __global__ void ml_prolong_even_kernel(int n, const int64_t* __restrict__ ncl, M
                                        const double* __restrict__ cm, const double* __restrict__ ct, int64_t NCc,
                                        const double* __restrict__ wc, double* __restrict__ fm,
                                        double* __restrict__ ft) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -162,7 +162,7 @@ __global__ void ml_prolong_even_kernel(int n, const int64_t* __restrict__ ncl, M
 __global__ void ml_prolong_odd_kernel(int n, const int64_t* __restrict__ ncl, MgGeo g, int L,
                                       const double* __restrict__ wc, double* __restrict__ fm,
                                       double* __restrict__ ft) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -248,7 +248,7 @@ __device__ __forceinline__ void interp_inner(const PairGeo& g, const double* __r
 
 __device__ __forceinline__ bool parent_of(const PairGeo& g, int& lz, int& ip, int& jp, int& k, int L) {
   const int64_t per = (int64_t)10 * g.nc * g.nc;
-  const int64_t t = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)list_block() * blockDim.x + threadIdx.x;
   if (t >= per) return false;
   k = blockIdx.y;
   lz = (int)(t / ((int64_t)g.nc * g.nc));
@@ -716,7 +716,7 @@ __global__ void ml_coarse_scalar_kernel(int n, int nmaster, const int64_t* __res
                                         double* __restrict__ dsl, const double* __restrict__ qm,
                                         const double* __restrict__ qt, double* __restrict__ om,
                                         double* __restrict__ ot, double h, int trend_only, int plus_div) {
-  const int t = xcd_block() * blockDim.x + threadIdx.x;
+  const int t = list_block() * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int y = blockIdx.y, k = y % L;
   const double* hf = hcl + (int64_t)y * 3 * NC;

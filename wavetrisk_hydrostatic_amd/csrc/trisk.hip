@@ -808,7 +808,7 @@ __global__ __launch_bounds__(THREADS2, 2) void trisk_stage_kernel2(StageArgs a_i
 // (two layers in lock step in one 768-thread block, the geometry in LDS)
 // took 1034 us, and 15.5 -> 13.7 us at J5 L1, 224 -> 156 us at J7 L20.  The
 // column sum of the stage before saves reading mass and temp twice (0.44 GB),
-// the split-explicit form no longer spills (2070 -> 720 us).
+// the split-explicit form no longer spills (2070 -> 727 us).
 // ---------------------------------------------------------------------------
 constexpr int GROUP = 384;
 constexpr int THREADS3 = 2 * GROUP;
