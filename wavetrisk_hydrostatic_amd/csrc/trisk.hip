@@ -2783,9 +2783,10 @@ int wtg_split_steps(wtg_ctx* c, int slot, int nsteps, wtg_fs_solver solve, void*
                              c->stream));
     for (int st = 0; st < nstages; ++st) {
       const auto &in = c->slots[ins[st]], &tr = c->slots[trs[st]], &out = c->slots[outs[st]];
-      double* const csum = c->d_csum[0];
+      double* const csum = f32 ? nullptr : c->d_csum[0];  // the FP32-bulk stage takes its own
       for (size_t i = 0; i < V.size(); ++i)
-        if (int rc = baro_correction(V[i], V[i]->slots[ins[st]], csum + (int64_t)i * NC)) return view_err(V[i], rc);
+        if (int rc = baro_correction(V[i], V[i]->slots[ins[st]], csum ? csum + (int64_t)i * NC : nullptr))
+          return view_err(V[i], rc);
       if (int rc = launch_ghost_fill(c, in, csum)) return rc;
       if (fused && ins[st] != outs[st]) {  // trend and u_star / scalar_star in one launch
         if (int rc = launch_stage(c, in, sol, out, coef[st], 0, nullptr, c->fs[FS_ETA], csum)) return rc;
