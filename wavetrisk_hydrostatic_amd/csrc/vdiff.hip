@@ -367,7 +367,7 @@ __global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) 
 // with dUdZ^2, N^2, one length or pivot and the right-hand side per level kept
 // between them.  Same operations as turbulent_column, to which a system that
 // dgtsv would pivot is left (vd_tke_left_kernel).  Bound by the latency of its divisions and square roots at
-// one or two waves per SIMD.  J8 L30: 1.79 -> 0.88 ms
+// one or two waves per SIMD.  J8 L30: 1.79 -> 1.07 ms
 // (one wave per SIMD); the whole call 3.48 -> 1.85 ms, at J7 L20 0.69 -> 0.30 ms.
 template <int LM>
 __global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
