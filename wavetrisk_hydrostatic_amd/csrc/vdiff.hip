@@ -366,7 +366,8 @@ __global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) 
 //   up    the new length from the bottom and the coefficients,
 // with dUdZ^2, N^2, one length or pivot and the right-hand side per level kept
 // between them.  Same operations as turbulent_column, to which a system that
-// dgtsv would pivot is left (vd_tke_left_kernel).  Bound by the latency of its divisions and square roots at
+// dgtsv would pivot is left (vd_tke_left_kernel), and one with an infinity or
+// NaN (a massless layer).  Bound by the latency of its divisions and square roots at
 // one or two waves per SIMD.  J8 L30: 1.79 -> 1.07 ms
 // (one wave per SIMD); the whole call 3.48 -> 1.85 ms, at J7 L20 0.69 -> 0.30 ms.
 template <int LM>
@@ -389,6 +390,7 @@ __global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
   const int64_t W = c - 1, SW = c - a.S - 1, Sx = c - a.S;
   // dUdZ^2 and N^2 at the interfaces 1 .. L - 1
   double dU2[LM], Nsq[LM], A[LM + 1], X[LM];
+  bool fast = true;
   {
     const double l0 = a.len[c], l1 = a.len[NC + c], l2 = a.len[2 * NC + c], p0 = a.ped[c], p1 = a.ped[NC + c];
     const double p2 = a.ped[2 * NC + c], lS = a.len[2 * NC + Sx], pS = a.ped[2 * NC + Sx], lSW = a.len[NC + SW];
@@ -427,6 +429,8 @@ __global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
             const double dzm = 0.5 * (dzp + dz), rz = 1.0 / dzm, q = div_by(um - umag, dzm, rz);
             dU2[k - 1] = q * q;
             Nsq[k - 1] = div_by(a.grav * (b - bp), dzm, rz);
+            // div_by gives NaN where a division gives an infinity
+            if (k < L) fast = fast && fabs(dU2[k - 1]) < INFINITY && fabs(Nsq[k - 1]) < INFINITY;
           }
           umag = um;
           dzp = dz;
@@ -449,7 +453,6 @@ __global__ __launch_bounds__(VT, LM > 24 ? 1 : 2) void vd_tke_kernel(VdArgs a) {
         A[l] = prev;
       }
   }
-  bool fast = true;
   double di = 0.0, xi = 0.0, ui = 0.0;
   {
     double dn = p.l_0, dzc = DZ(1), Kvp = 0.0, Kvc = kv[NC];
