@@ -32,6 +32,7 @@
 
 #include "ctx.h"
 #include "exact_div.h"
+#include "planes.h"
 
 namespace {
 
@@ -840,7 +841,8 @@ __device__ __forceinline__ void weights_lds(const TileS& s, int y, int offs, dou
 
 // Planes read and written through buffer descriptors: a uniform base, a
 // uniform 32-bit byte offset of the plane and the cell's 32-bit byte offset,
-// so that an address costs no vector register or instruction of its own.
+// so that an address costs no vector register or instruction of its own.  At
+// most three planes from one base (plane_at).
 using Plane = __amdgpu_buffer_rsrc_t;
 __device__ __forceinline__ Plane plane(const double* p) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, -1, 0x00027000);
@@ -876,7 +878,10 @@ __device__ __forceinline__ void tile_geometry(TileCell& c, const StageArgs& a) {
 
 // planes of the geometry that neighbours read, of one region cell
 __device__ __forceinline__ void tile_areas(double v[7], const StageArgs& a, uint32_t xb) {
-  for (int p = 0; p < 6; ++p) v[p] = ldp(plane(a.g.area), xb, p * (uint32_t)a.NC * 8u);
+  for (int p = 0; p < 6; ++p) {
+    const wtg::PlaneAt at = wtg::plane_at(p, a.NC);
+    v[p] = ldp(plane(a.g.area + at.first), xb, at.byte);
+  }
   v[6] = ldp(plane(a.g.hinv), xb);
 }
 
