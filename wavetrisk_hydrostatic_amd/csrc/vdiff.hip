@@ -347,14 +347,26 @@ __global__ __launch_bounds__(VT) void vd_turbulent_kernel(VdArgs a) {
   turbulent_column(a, blockIdx.y, column(a, tid, pole));
 }
 
-// the columns that vd_tke_kernel left (a thread looks at a block's word)
-__global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) {
-  const int id = blockIdx.x * VT + threadIdx.x;
-  if (id >= nblocks) return;
-  for (unsigned long long w = a.left[(int64_t)blockIdx.y * nblocks + id]; w; w &= w - 1) {
-    bool pole;
-    turbulent_column(a, blockIdx.y, column(a, (int64_t)id * VT + __builtin_ctzll(w), pole));
+// What the register kernels left, a lane a system: a wave looks at LEFT words
+// together and takes those that are not empty one after another, so that a
+// grid whose systems are all left still has VT times its words in flight.
+constexpr int LEFT = 8;
+template <class F>
+__device__ __forceinline__ void each_left(const unsigned long long* left, int nwords, const F& take) {
+  const int lane = threadIdx.x, first = blockIdx.x * LEFT;
+  const unsigned long long mine = lane < LEFT && first + lane < nwords ? left[first + lane] : 0;
+  for (unsigned long long some = __ballot(mine != 0); some; some &= some - 1) {
+    const int k = __builtin_ctzll(some);
+    if (__shfl(mine, k) >> lane & 1) take(first + k);
   }
+}
+
+// the columns that vd_tke_kernel left
+__global__ __launch_bounds__(VT) void vd_tke_left_kernel(VdArgs a, int nblocks) {
+  each_left(a.left + (int64_t)blockIdx.y * nblocks, nblocks, [&](int word) {
+    bool pole;
+    turbulent_column(a, blockIdx.y, column(a, (int64_t)word * VT + threadIdx.x, pole));
+  });
 }
 
 // The TKE closure for at most LM layers (and istep > 1, whose coefficients are
@@ -695,19 +707,22 @@ __global__ __launch_bounds__(VT) void vd_solve_kernel(VdArgs a) {
 // The same for at most LM layers, a lane one system: the elimination's
 // diagonal, super-diagonal and right-hand side stay in registers (the loops
 // over layers are unrolled), so that the state's own bytes are what moves.
-// Rows without a solar flux; a system that dgtsv would pivot, one with a solar
-// flux and a column with a thickness that is not positive are left to
-// vd_solve_left_kernel (a call from here would cost the arrays their registers).
+// A system that dgtsv would pivot and a column with a thickness that is not
+// positive are left to vd_solve_left_kernel (a call from here would cost the
+// arrays their registers).  Grid x: count systems of every column block, the
+// first being `first`.  SOLAR: the buoyancy rows with a solar flux, whose two
+// exponentials an interface cost the other systems no registers this way.
 // Bound by memory latency at two waves per SIMD (three arrays of 32 doubles are
 // 192 // 192 registers).  J8 L30: 1.63 -> 0.70 ms; with the arrays in LDS (three waves
 // per compute unit) 1.6 ms.
-template <int LM>
-__global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArgs a, int ncb) {
+template <int LM, bool SOLAR>
+__global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArgs a, int ncb, int first, int count) {
   const int L = a.L;
   // consecutive blocks lie on different XCDs: an XCD takes a run of column
-  // blocks, the four systems of one after another
-  const int per = ncb / 8, id = blockIdx.x, e = (id / 8) % 4 - 1, cb = (id % 8) * per + id / 32;
-  const bool edge = e >= 0;
+  // blocks, the systems of one after another
+  const int per = ncb / 8, id = blockIdx.x, e = SOLAR ? -1 : first + id / 8 % count;
+  const int cb = id % 8 * per + id / 8 / count;
+  const bool edge = !SOLAR && e >= 0;
   const int64_t nown = (int64_t)10 * a.n * a.n, tid = (int64_t)cb * VT + threadIdx.x;
   const bool live = tid < (edge ? nown : nown + 2);  // the poles carry no edges of their own
   bool pole;
@@ -724,7 +739,7 @@ __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArg
   // thickness, coefficient at the upper interface and value of every layer;
   // they become the elimination's super-diagonal, diagonal and right-hand side
   double U[LM], D[LM], X[LM];
-  double least = INFINITY;
+  double least = INFINITY, depth = 0.0;
   constexpr int CH = 4;
 #pragma unroll
   for (int k0 = 0; k0 < LM; k0 += CH) {
@@ -743,12 +758,20 @@ __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArg
         const double z = div_by(0.0 + m0[j], rho, rrho);
         U[k0 + j] = edge ? 0.5 * (z + div_by(0.0 + m1[j], rho, rrho)) : z;
         least = U[k0 + j] > 0.0 ? least : -1.0;
+        if (SOLAR && k0 + j < L) depth = depth + z;
         if (!edge) X[k0 + j] = X[k0 + j] / (0.0 + m0[j]);
       }
     }
   }
-  bool fast = least > 0.0 && (edge || p.Q_sr == 0.0);
+  bool fast = least > 0.0;
   if (fast) {
+    // the irradiance at the layer's lower interface, of height z0
+    double z0 = 0.0, eta = 0.0, below = 0.0;
+    if (SOLAR) {
+      z0 = a.topo[mb * NC + c];
+      eta = a.eta ? a.eta[mb * NC + c] : depth + z0;
+      below = irradiance(p, eta - z0);
+    }
     const double bot = edge ? 0.0 : f[0], top = edge ? f[(3 + e) * NC] : f[NC];
     double di = 0.0, xi = 0.0, ui = 0.0, Kp = 0.0, dzp = 0.0;
 #pragma unroll
@@ -763,7 +786,15 @@ __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArg
           if (k == 0) dg = dg + dt * p.bottom_friction / dz;
           if (last) r = r + dt * top / dz;
         } else {
-          if (k == 0) r = r + dt * (-bot + 0.0) / dz;
+          if (SOLAR && !last) {
+            z0 = z0 + dz;
+            const double above = irradiance(p, eta - z0);
+            const double solar = p.Q_sr * (above - below) / (a.rho0 * p.c_p);
+            below = above;
+            r = r + dt * (k == 0 ? -bot + solar : solar) / dz;
+          } else if (k == 0) {
+            r = r + dt * (-bot + 0.0) / dz;
+          }
           if (last) {
             // the reference's top row takes the row below's super-diagonal entry
             dg = 1.0 - (-(dt * Kp / (0.5 * (dzp + dz) * dzp)));
@@ -805,22 +836,34 @@ __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArg
     }
   }
   const unsigned long long left = __ballot(!fast && live);
-  if (threadIdx.x == 0) a.left[mb * gridDim.x + id] = left;
+  if (threadIdx.x == 0) a.left[(mb * 4 + e + 1) * ncb + cb] = left;
 }
 
-// the systems that vd_solve_reg_kernel left (a thread looks at a block's word)
+// the systems that vd_solve_reg_kernel left
 __global__ __launch_bounds__(VT) void vd_solve_left_kernel(VdArgs a, int ncb) {
-  const int id = blockIdx.x * VT + threadIdx.x;
-  if (id >= 4 * ncb) return;
   const int64_t mb = blockIdx.y, NC = a.NC;
-  const int per = ncb / 8, e = (id / 8) % 4 - 1, cb = (id % 8) * per + id / 32;
-  for (unsigned long long w = a.left[mb * 4 * ncb + id]; w; w &= w - 1) {
+  each_left(a.left + mb * 4 * ncb, 4 * ncb, [&](int word) {
     bool pole;
-    const int64_t c = column(a, (int64_t)cb * VT + __builtin_ctzll(w), pole);
+    const int64_t c = column(a, (int64_t)(word % ncb) * VT + threadIdx.x, pole);
+    const int e = word / ncb - 1;
     const double zs = a.topo[mb * NC + c];
     const double eta = e >= 0 ? 0.0 : a.eta ? a.eta[mb * NC + c] : free_surface(a, a.m + mb * a.L * NC, zs, c);
     solve_column(a, mb, c, e, eta);
-  }
+  });
+}
+
+// With a solar flux the buoyancy rows are a launch of their own: the call at J8
+// L30 takes 1.87 ms (3.48 with every system in private arrays), J6 L20 141 us
+// (310), 8 us more than without the flux.
+template <int LM>
+void launch_solve_reg(const VdArgs& a, int ncb, unsigned members, hipStream_t stream) {
+  const bool solar = a.p.Q_sr != 0.0;
+  if (solar)
+    hipLaunchKernelGGL((vd_solve_reg_kernel<LM, true>), dim3((unsigned)ncb, members), dim3(VT), 0, stream, a, ncb, -1,
+                       1);
+  const int first = solar ? 0 : -1, count = solar ? 3 : 4;
+  hipLaunchKernelGGL((vd_solve_reg_kernel<LM, false>), dim3((unsigned)(count * ncb), members), dim3(VT), 0, stream, a,
+                     ncb, first, count);
 }
 
 }  // namespace
@@ -942,7 +985,6 @@ extern "C" int wtg_vertical_diffusion(wtg_ctx* c, int slot, double dt, int istep
   const dim3 grid((unsigned)((cols + VT - 1) / VT), (unsigned)M);
   // the register kernels hold up to 32 layers; above, the private arrays
   const int nblk = (int)grid.x, ncb = (nblk + 7) / 8 * 8;
-  const dim3 systems((unsigned)(4 * ncb), (unsigned)M);
   if (!c->vd.tke_closure || istep == 1 || L > 32) {
     hipLaunchKernelGGL(vd_turbulent_kernel, grid, dim3(VT), 0, c->stream, a);
   } else {
@@ -953,21 +995,21 @@ extern "C" int wtg_vertical_diffusion(wtg_ctx* c, int slot, double dt, int istep
     else
       hipLaunchKernelGGL(vd_tke_kernel<32>, grid, dim3(VT), 0, c->stream, a);
     WTG_HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(vd_tke_left_kernel, dim3((unsigned)((nblk + VT - 1) / VT), (unsigned)M), dim3(VT), 0, c->stream,
-                       a, nblk);
+    hipLaunchKernelGGL(vd_tke_left_kernel, dim3((unsigned)((nblk + LEFT - 1) / LEFT), (unsigned)M), dim3(VT), 0,
+                       c->stream, a, nblk);
   }
   WTG_HIPCHK(c, hipGetLastError());
   if (L > 32) {
     hipLaunchKernelGGL(vd_solve_kernel, grid, dim3(VT), 0, c->stream, a);
   } else {
     if (L <= 16)
-      hipLaunchKernelGGL(vd_solve_reg_kernel<16>, systems, dim3(VT), 0, c->stream, a, ncb);
+      launch_solve_reg<16>(a, ncb, (unsigned)M, c->stream);
     else if (L <= 24)
-      hipLaunchKernelGGL(vd_solve_reg_kernel<24>, systems, dim3(VT), 0, c->stream, a, ncb);
+      launch_solve_reg<24>(a, ncb, (unsigned)M, c->stream);
     else
-      hipLaunchKernelGGL(vd_solve_reg_kernel<32>, systems, dim3(VT), 0, c->stream, a, ncb);
+      launch_solve_reg<32>(a, ncb, (unsigned)M, c->stream);
     WTG_HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(vd_solve_left_kernel, dim3((unsigned)((4 * ncb + VT - 1) / VT), (unsigned)M), dim3(VT), 0,
+    hipLaunchKernelGGL(vd_solve_left_kernel, dim3((unsigned)((4 * ncb + LEFT - 1) / LEFT), (unsigned)M), dim3(VT), 0,
                        c->stream, a, ncb);
   }
   WTG_HIPCHK(c, hipGetLastError());
