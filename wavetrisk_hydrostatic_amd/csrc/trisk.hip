@@ -411,10 +411,13 @@ __global__ __launch_bounds__(THREADS) void trisk_stage_kernel(StageArgs a_in) {
 // circulation and mass, and two qe values per corner are overwritten.
 // `which` = 0..3 for the SW, SE, NW, NE corner; region cell (1,1), (T+1,1),
 // (1,T+1), (T+1,T+1).  U(e, i, j) and M(i, j) give the region's velocities
-// and masses; out = the corner's two values of qe.
-template <class UF, class MF>
+// and masses; put(k, e, i, j, v) takes the corner's two values k of qe, of edge
+// e at region cell (i, j).  Everything but `which` is known when it is compiled:
+// values gathered in an array and stored at the end cost the FP32-bulk stage,
+// which calls this in its layer loop, 3 to 4 registers and up to 11 spills.
+template <class UF, class MF, class PF>
 __device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF& M, const Geo& g, int64_t NC,
-                                                int64_t base, int S, double out[2]) {
+                                                int64_t base, int S, const PF& put) {
   auto gcell = [&](int ri, int rj) -> int64_t { return base + (int64_t)rj * S + ri; };
   auto P = [&](int e, int i, int j) { return U(e, i, j) * g.len[(int64_t)e * NC + gcell(i, j)]; };
   auto AR = [&](int p, int i, int j) { return g.area[(int64_t)(p - 1) * NC + gcell(i, j)]; };
@@ -431,8 +434,8 @@ __device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF
     double pvWL = (COR(0, i - 1, j) + cW_L) / m1;
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m2;
     double pvSU = (COR(1, i, j - 1) + cS_U) / m3;
-    out[0] = interp(pvWL, pvSWL);
-    out[1] = interp(pvSU, pvSWL);
+    put(0, 0, i - 1, j, interp(pvWL, pvSWL));
+    put(1, 2, i, j - 1, interp(pvSU, pvSWL));
   } else if (which == 1) {  // IPLUSJMINUS
     const int i = T + 1, j = 1;
     double cSW_L = -P(0, i, j) + P(0, i - 1, j - 1) + P(1, i - 1, j - 1);
@@ -446,8 +449,8 @@ __device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m1;
     double pvL = (COR(0, i, j) + cL) / m2;
     double pvSWU = (COR(1, i - 1, j - 1) + cSW_U) / m3;
-    out[0] = interp(pvSWL, pvL);
-    out[1] = interp(pvSWL, pvSWU);
+    put(0, 0, i, j, interp(pvSWL, pvL));
+    put(1, 1, i - 1, j - 1, interp(pvSWL, pvSWU));
   } else if (which == 2) {  // IMINUSJPLUS
     const int i = 1, j = T + 1;
     double cSW_U = P(2, i, j) - P(1, i - 1, j - 1) - P(2, i - 1, j - 1);
@@ -461,8 +464,8 @@ __device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF
     double pvSWU = (COR(1, i - 1, j - 1) + cSW_U) / m1;
     double pvU = (COR(1, i, j) + cU) / m2;
     double pvSWL = (COR(0, i - 1, j - 1) + cSW_L) / m3;
-    out[0] = interp(pvSWU, pvU);
-    out[1] = interp(pvSWL, pvSWU);
+    put(0, 2, i, j, interp(pvSWU, pvU));
+    put(1, 1, i - 1, j - 1, interp(pvSWL, pvSWU));
   } else {  // IJPLUS
     const int i = T + 1, j = T + 1;
     double cL = P(0, i, j) - P(0, i, j + 1) - P(2, i, j);
@@ -474,8 +477,8 @@ __device__ __forceinline__ void pentagon_values(int which, const UF& U, const MF
     double pvL = (COR(0, i, j) + cL) / m1;
     double pvWL = (COR(0, i - 1, j) + cW_L) / m2;
     double pvSU = (COR(1, i, j - 1) + cS_U) / m3;
-    out[0] = interp(pvL, pvSU);
-    out[1] = interp(pvL, pvWL);
+    put(0, 0, i, j, interp(pvL, pvSU));
+    put(1, 2, i, j, interp(pvL, pvWL));
   }
 }
 
@@ -486,13 +489,11 @@ __device__ void pentagon_fixup(int which, const F* __restrict__ u0p, const F* __
                                const F* __restrict__ u2p, const F* __restrict__ mp, F* qe0, F* qe1, F* qe2,
                                const Geo& g, int64_t NC, int64_t base, int S) {
   const F* up[3] = {u0p, u1p, u2p};
-  double v[2];
+  F* const qe[3] = {qe0, qe1, qe2};
   pentagon_values(
       which, [&](int e, int i, int j) { return (double)up[e][j * R + i]; },
-      [&](int i, int j) { return (double)mp[j * R + i]; }, g, NC, base, S, v);
-  const int at[4][2] = {{R, 1}, {R + T + 1, T}, {(T + 1) * R + 1, T * R}, {(T + 1) * R + T + 1, (T + 1) * R + T + 1}};
-  (which == 2 ? qe2 : qe0)[at[which][0]] = (F)v[0];
-  (which == 1 || which == 2 ? qe1 : qe2)[at[which][1]] = (F)v[1];
+      [&](int i, int j) { return (double)mp[j * R + i]; }, g, NC, base, S,
+      [&](int, int e, int i, int j, double v) { qe[e][j * R + i] = (F)v; });
 }
 
 // Loads and stores at a uniform base pointer plus a 32-bit byte offset, so the
@@ -1088,12 +1089,10 @@ __global__ __launch_bounds__(THREADS, 2) void trisk_stage_tile_kernel(StageArgs 
       const int wh = i & 3, k = k0 + (i >> 2);
       if (wh == 0 ? cSW : wh == 1 ? cSE : wh == 2 ? cNW : cNE) {
         const int64_t ks = (int64_t)k * NC;
-        double v[2];
         pentagon_values(
             wh, [&](int e, int i, int j) { return a.yu[3 * ks + e * NC + gcell(i, j)]; },
-            [&](int i, int j) { return a.ym[ks + gcell(i, j)]; }, g, NC, base, S, v);
-        fixes[((int64_t)wh * a.L + k) * 2] = v[0];
-        fixes[((int64_t)wh * a.L + k) * 2 + 1] = v[1];
+            [&](int i, int j) { return a.ym[ks + gcell(i, j)]; }, g, NC, base, S,
+            [&](int q, int, int, int, double v) { fixes[((int64_t)wh * a.L + k) * 2 + q] = v; });
       }
     }
     __threadfence_block();
