@@ -140,7 +140,7 @@ __global__ void ml_prolong_even_kernel(int n, const int64_t* __restrict__ ncl, M
                                        const double* __restrict__ cm, const double* __restrict__ ct, int64_t NCc,
                                        const double* __restrict__ wc, double* __restrict__ fm,
                                        double* __restrict__ ft) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;

@@ -17,4 +17,6 @@ __device__ __forceinline__ unsigned xcd_block() {
 // prolongation at J7 L20 33 -> 27, an apply at J7 for three members 15.8 ->
 // 15.5; below, an eighth is a few blocks and the halo copies at the list's end
 // fall to one XCD: the applies at J6 for four members 8.3 -> 9.2 and 9.0 -> 10.3.
+// Not for the multi-level even prolongation, which reads several planes of two
+// levels and loses at J8 (153 -> 206 us on the levels of J5 to J8 with L30).
 __device__ __forceinline__ unsigned list_block() { return gridDim.x < 512 ? blockIdx.x : xcd_block(); }
