@@ -367,6 +367,15 @@ int wtg_elliptic_solve(wtg_ctx* ctx, int method, double rel_tol, int max_iter, i
  * are those of the eager launches.  0 (default): eager launches.  No
  * counterpart in the reference. */
 int wtg_fs_set_graph(wtg_ctx* ctx, int enable);
+/* BiCGSTAB is one launch on grids whose blocks can all run at once (up to J8),
+ * with the launches' results to the last bit.  Its blocks wait for each other
+ * at most `ms` milliseconds (default 20, range [0, 1000]); where that runs
+ * out, for instance beside another solve that holds part of the GPU, the
+ * launches repeat the solve, and take the next 16 (then 32, up to 1024) too
+ * before one launch is tried again.  No counterpart in the reference. */
+int wtg_fs_set_wait(wtg_ctx* ctx, double ms);
+/* solves of the context tried in one launch, and those of them given up */
+int wtg_fs_one_launch(const wtg_ctx* ctx, long long* solves, long long* given_up);
 
 /* dt_step_split => RK4_split (time_integr.f90:360-382, main.f90:209): nsteps
  * split-explicit steps of size dt (wtg_fs_set_params) on state slot `slot`

@@ -103,6 +103,8 @@ SIGNATURES = {
     "wtg_grid_shard_halo": (C.c_int, [_P, C.c_int, C.POINTER(C.c_int64)]),
     "wtg_ghost_fill_split_timed": (C.c_int, [_P, C.c_int, C.c_int, C.c_int, _D, _D]),
     "wtg_fs_set_graph": (C.c_int, [_P, C.c_int]),
+    "wtg_fs_set_wait": (C.c_int, [_P, C.c_double]),
+    "wtg_fs_one_launch": (C.c_int, [_P, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]),
     "wtg_get_stage_shape": (C.c_int, [_P, C.POINTER(C.c_int), C.POINTER(C.c_float)]),
     "wtg_state_device_ptrs": (C.c_int, [_P, C.c_int, C.POINTER(_P), C.POINTER(_P), C.POINTER(_P)]),
     "wtg_synchronize": (C.c_int, [_P]),
@@ -373,6 +375,17 @@ class Context:
     def fs_set_graph(self, enable: bool):
         """BiCGSTAB chunks replayed from a captured HIP graph (default off)."""
         _check(_lib.wtg_fs_set_graph(self._h, int(bool(enable))), self._h, "wtg_fs_set_graph")
+
+    def fs_set_wait(self, ms: float):
+        """How long the blocks of a one-launch BiCGSTAB wait for each other
+        before the separate launches repeat the solve (default 20 ms)."""
+        _check(_lib.wtg_fs_set_wait(self._h, float(ms)), self._h, "wtg_fs_set_wait")
+
+    def fs_one_launch(self):
+        """(solves tried in one launch, those of them given up)."""
+        n, failed = C.c_longlong(), C.c_longlong()
+        _check(_lib.wtg_fs_one_launch(self._h, C.byref(n), C.byref(failed)), self._h, "wtg_fs_one_launch")
+        return n.value, failed.value
 
     def set_graph(self, enable: bool):
         """rk4 replays its steps from a captured HIP graph (identical results)."""

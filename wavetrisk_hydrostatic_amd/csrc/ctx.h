@@ -111,7 +111,9 @@ struct wtg_ctx {
   int lastblock_max = 64;
   // BiCGSTAB in one launch: the blocks' partial sums; of a small level the owner
   // of every cell, of a large one the blocks' neighbour rows and rings
-  bool bicg_one = true;
+  unsigned long long bicg_wait = 2000000;   // bound of its blocks' waits: 20 ms in ticks of the 100 MHz wall clock
+  int bicg_rest = 0, bicg_rests = 0;         // solves left to the launches after a wait ran out; the last such number
+  long long bicg_solves = 0, bicg_given_up = 0;  // solves in one launch; of these given up and repeated
   int bicg_blocks = 0;
   bool red_masters = false;  // the reduction cells are the masters, in order
   int *d_src = nullptr, *d_blring = nullptr, *d_blnring = nullptr;

@@ -632,15 +632,17 @@ __global__ __launch_bounds__(FS_NT) void fs_bicg_res_kernel(
 // invalidated; a block's partial sums go out after its values, and every block
 // then adds all partials in fs_dot_final_kernel's order.  The same operations
 // as the launches of `bicgstab`: same iterates, residuals and counts.
-// A wait is bounded (20 ms): if it ends, every block leaves with u untouched and
-// the solve is repeated by the launches.
+// A wait is bounded (wtg_fs_set_wait): if it runs out, every block leaves with u
+// untouched and the solve is repeated by the launches.
+// That a block's values are out before its sums rests on the machine (a store
+// past the L2s that s_waitcnt has seen off is seen by every later such load on
+// gfx950), not on the memory model, whose release would write the L2 back.
 // Bound by the three device-wide round trips of an iteration.  An iteration by
 // launches (five, replayed from a graph) -> in here: J4 31.1 -> 9.3 us, J5 37.0
 // -> 11.1, J6 (161 blocks) 31.1 -> 12.6; finer grids do not fit.
 // ---------------------------------------------------------------------------
 constexpr int BICG_BLOCKS = 256;  // at most one block of a solve per compute unit, so that all are resident
 constexpr int BICG_SLOTS = 512;   // most partial sums of a reduction
-constexpr unsigned long long BICG_WAIT = 2000000ull;  // 20 ms: ticks of the 100 MHz wall clock
 
 __device__ __forceinline__ double load_out(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -662,12 +664,13 @@ __device__ __forceinline__ double* bicg_slot(double* part, unsigned epoch, int b
 __device__ __forceinline__ void bicg_post(double* slot, double v) {
   store_out(slot, v == v ? v : __longlong_as_double(0x7ff8000000000000ll));
 }
-__device__ __forceinline__ void bicg_wait(const double* slot, int* ok, double& v0, double& v1) {
+__device__ __forceinline__ void bicg_wait(const double* slot, unsigned long long most, int* ok, double& v0,
+                                          double& v1) {
   const unsigned long long t0 = wall_clock64();
   while (true) {
     v0 = load_out(slot), v1 = load_out(slot + 1);
     if (__double_as_longlong(v0) != (long long)BICG_EMPTY && __double_as_longlong(v1) != (long long)BICG_EMPTY) return;
-    if (wall_clock64() - t0 > BICG_WAIT) {
+    if (wall_clock64() - t0 >= most) {
       *ok = 0;
       return;
     }
@@ -675,7 +678,7 @@ __device__ __forceinline__ void bicg_wait(const double* slot, int* ok, double& v
 }
 
 __device__ __forceinline__ bool reduce_out(double s0, double s1, double (*sh)[FS_NT], double* part, unsigned& epoch,
-                                           int* ok, double out[2]) {
+                                           unsigned long long wait, int* ok, double out[2]) {
   const int nb = gridDim.x, tid = threadIdx.x;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have left
   double acc[RED_MAX] = {s0, s1, 0.0};
@@ -684,7 +687,7 @@ __device__ __forceinline__ bool reduce_out(double s0, double s1, double (*sh)[FS
   acc[0] = acc[1] = 0.0;
   if (tid < nb) {  // nb <= BICG_BLOCKS = FS_NT: one block's sums a thread
     double v0, v1;
-    bicg_wait(bicg_slot(part, epoch, tid), ok, v0, v1);
+    bicg_wait(bicg_slot(part, epoch, tid), wait, ok, v0, v1);
     acc[0] = acc[0] + v0, acc[1] = acc[1] + v1;
   }
   __syncthreads();  // sh is free again
@@ -713,6 +716,7 @@ struct BicgArgs {
   const double* rw;    // reduction weight of every master
   double *scal, *part;
   int64_t ms;
+  unsigned long long wait;  // bound of a wait, in ticks
 };
 
 __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
@@ -747,7 +751,7 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
   unsigned epoch = 0;
   double sum[2];
   auto sums = [&](double s0, double s1) {
-    return reduce_out(live ? w * s0 : 0.0, live ? w * s1 : 0.0, sh, part, epoch, &ok, sum);
+    return reduce_out(live ? w * s0 : 0.0, live ? w * s1 : 0.0, sh, part, epoch, a.wait, &ok, sum);
   };
   // res = f - L u; nrm_f = l2(f); rho = dp(res0, res)
   const double fc = f[c];
@@ -854,7 +858,7 @@ struct BlPlan {
 
 // reduce_out over two halves of a block, each a block of the launches' reductions
 __device__ __forceinline__ bool reduce_large(double s0, double s1, int nb, double (*sh)[2][FS_NT], double* part,
-                                             unsigned& epoch, int* ok, double out[2]) {
+                                             unsigned& epoch, unsigned long long wait, int* ok, double out[2]) {
   const int tid = threadIdx.x, half = tid / FS_NT, t = tid % FS_NT;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have left
   auto tree = [&](int h, bool mine) {  // block_tree's order
@@ -877,7 +881,7 @@ __device__ __forceinline__ bool reduce_large(double s0, double s1, int nb, doubl
   const int me = 2 * xcd_block() + half;
   if (t < 2 && me < nb) bicg_post(bicg_slot(part, epoch, me) + t, sh[half][t][0]);
   double v0 = 0.0, v1 = 0.0;
-  if (tid < nb) bicg_wait(bicg_slot(part, epoch, tid), ok, v0, v1);
+  if (tid < nb) bicg_wait(bicg_slot(part, epoch, tid), wait, ok, v0, v1);
   __syncthreads();  // sh is free again
   sh[half][0][t] = v0, sh[half][1][t] = v1;
   __syncthreads();
@@ -972,7 +976,7 @@ __global__ __launch_bounds__(BL_NT, 2) void fs_bicg_large_kernel(BicgArgs a, BlP
   double sum[2];
   bool good = true;
   auto sums = [&](double s0, double s1) {
-    return reduce_large(s0, s1, nb, sh, a.part, epoch, &ok, sum);
+    return reduce_large(s0, s1, nb, sh, a.part, epoch, a.wait, &ok, sum);
   };
   // res = f - L u; nrm_f = l2(f); rho = dp(res0, res)
   double s0 = 0.0, s1 = 0.0;
@@ -1641,10 +1645,19 @@ constexpr int BICG_CHUNK = 8;
 // per 256 masters of every member, all resident at once with room for a second
 // such solve on another stream (a compute unit holds two blocks), or one
 // member's fs_bicg_large_kernel.  It is the faster one wherever it fits; a
-// context that replays graphs has asked for the launches.
-bool bicg_one_launch(const wtg_ctx* c, int maxit) {
-  return c->bicg_one && c->d_bpart && !c->fs_graph && maxit > 0 &&
-         (c->d_src ? (int64_t)nblk(c->nmaster) * c->nmembers <= c->bicg_blocks : c->nmembers == 1 && !c->mg_mdone);
+// context that replays graphs has asked for the launches.  After a wait has run
+// out (two large solves at once, each on part of the chip) the next 16 solves
+// are launches, after every further one in a row twice as many, up to 1024: what
+// the waits cost stays small and a passing neighbour does not slow the run down
+// for good.
+constexpr int BICG_REST = 16, BICG_REST_MAX = 1024;
+bool bicg_one_launch(wtg_ctx* c, int maxit) {
+  if (!(c->d_bpart && !c->fs_graph && maxit > 0 &&
+        (c->d_src ? (int64_t)nblk(c->nmaster) * c->nmembers <= c->bicg_blocks : c->nmembers == 1 && !c->mg_mdone)))
+    return false;
+  if (c->bicg_rest == 0) return true;
+  --c->bicg_rest;
+  return false;
 }
 
 int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int* iters, double* err_out,
@@ -1653,7 +1666,8 @@ int bicgstab_one_launch(wtg_ctx* c, double* u, const double* f, double tol, int 
   const int M = c->nmembers;
   const int64_t ms = c->info.ncells;
   BicgArgs a{c->mg_mdone, c->nmaster, c->d_ncl, c->d_src, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav,
-             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[5], W[3], c->d_rw, c->d_scal, c->d_bpart, ms};
+             fs_coef(c), tol, zero_u ? 1 : 0, maxit, W[0], W[4], W[5], W[3], c->d_rw, c->d_scal, c->d_bpart, ms,
+             c->bicg_wait};
   if (c->d_src) {
     hipLaunchKernelGGL(fs_bicg_solve_kernel, dim3(nblk(c->nmaster), M), dim3(FS_NT), 0, c->stream, a);
   } else {
@@ -1704,8 +1718,14 @@ int bicgstab(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int*
   if (bicg_one_launch(c, maxit)) {
     bool solved = false;
     RC(bicgstab_one_launch(c, u, f, tol, maxit, iters, err_out, zero_u, sync_end, &solved));
-    if (solved) return 0;
-    c->bicg_one = false;  // its blocks did not run together; u is as it was
+    ++c->bicg_solves;
+    if (solved) {
+      c->bicg_rests = 0;
+      return 0;
+    }
+    // its blocks did not run together; u is as it was
+    ++c->bicg_given_up;
+    c->bicg_rest = c->bicg_rests = c->bicg_rests ? std::min(2 * c->bicg_rests, BICG_REST_MAX) : BICG_REST;
   }
   double** W = c->fs + FS_W0;
   double *res = W[0], *res0 = W[1], *p = W[2], *s = W[3], *Ap = W[4], *As = W[5], *p_alt = W[6];
@@ -1872,6 +1892,21 @@ int wtg_fs_ready(wtg_ctx* c) { return fs_ready(c); }
 int wtg_fs_set_graph(wtg_ctx* c, int enable) {
   if (!c) return WTG_E_ARG;
   c->fs_graph = enable != 0;
+  return 0;
+}
+
+int wtg_fs_set_wait(wtg_ctx* c, double ms) {
+  if (!c) return WTG_E_ARG;
+  if (!(ms >= 0.0 && ms <= 1000.0)) return wtg_fail(c, WTG_E_ARG, "wait of %g ms out of range [0,1000]", ms);
+  c->bicg_wait = (unsigned long long)(ms * 1e5);
+  c->bicg_rest = c->bicg_rests = 0;
+  return 0;
+}
+
+int wtg_fs_one_launch(const wtg_ctx* c, long long* solves, long long* given_up) {
+  if (!c || !solves || !given_up) return WTG_E_ARG;
+  *solves = c->bicg_solves;
+  *given_up = c->bicg_given_up;
   return 0;
 }
 
