@@ -826,7 +826,8 @@ __global__ __launch_bounds__(FS_NT, 2) void fs_bicg_solve_kernel(BicgArgs a) {
 // compute unit.  A block owns the masters that two neighbouring blocks of the
 // launches' reductions sum (2 x 256 masters in a row, and on every 512 x 256
 // from there), so the sums are theirs to the last bit.  The owned vectors live
-// in registers, the operand of the stencil in LDS, and so do the residual, Ap and
+// in registers (56 of them spilled: 220 bytes of scratch a lane), the operand of
+// the stencil in LDS, and so do the residual, Ap and
 // direction of the masters around the owned ones (the ring), which are read
 // once after their reduction; the operator comes from memory (L2 and the
 // memory-side cache) in each apply.

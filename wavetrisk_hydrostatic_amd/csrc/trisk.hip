@@ -810,7 +810,10 @@ __global__ __launch_bounds__(THREADS2, 2) void trisk_stage_kernel2(StageArgs a_i
 // (two layers in lock step in one 768-thread block, the geometry in LDS)
 // took 1034 us, and 15.5 -> 13.7 us at J5 L1, 224 -> 156 us at J7 L20.  The
 // column sum of the stage before saves reading mass and temp twice (0.44 GB),
-// the split-explicit form no longer spills (2070 -> 727 us).
+// the split-explicit form no longer spills (2070 -> 727 us).  The forms with
+// diffusion hooks spill 12 values (8 with the split update); the one that keeps
+// its fluxes for coarser levels is bound by their stores (1585 us at J8 L30,
+// the earlier kernel 1529; 142 and 161 at J7 L20).
 // ---------------------------------------------------------------------------
 constexpr int GROUP = 384;
 constexpr int THREADS3 = 2 * GROUP;

@@ -630,29 +630,6 @@ struct Rows {
 
 // One system of a column in private arrays: the buoyancy (e = -1) or the
 // velocity of the RT, DG or UP edge (0..2)
-__device__ void solve_column(const VdArgs& a, int64_t mb, int64_t c, int e, double eta, SolveWork& w) {
-  const int L = a.L;
-  const int64_t NC = a.NC;
-  const double* m = a.m + mb * L * NC;
-  double* t = a.t + mb * L * NC;
-  double* u = a.u + mb * 3 * L * NC;
-  const double* f = a.force + mb * 6 * NC;
-  const double zs = a.topo[mb * NC + c];
-  const bool edge = e >= 0;
-  const int64_t nb = e == 0 ? c + 1 : e == 1 ? c + a.S + 1 : e == 2 ? c + a.S : c;
-  Rows rows{a, m, t, u, (edge ? a.kv : a.kt) + mb * (L + 1) * NC, f, c, nb, e, eta, a.dt};
-  solve_rows(L, rows, zs, w);
-  for (int k = 1; k <= L; ++k) {
-    const int64_t x = (int64_t)(k - 1) * NC + c;
-    if (edge)
-      u[((int64_t)(k - 1) * 3 + e) * NC + c] = w.X[k];
-    else
-      t[x] = (0.0 + m[x]) * w.X[k];
-  }
-}
-
-// One system of a column in private arrays: the buoyancy (e = -1) or the
-// velocity of the RT, DG or UP edge (0..2)
 __device__ void solve_column(const VdArgs& a, int64_t mb, int64_t c, int e, double eta) {
   const int L = a.L;
   const int64_t NC = a.NC;
@@ -713,7 +690,7 @@ __global__ __launch_bounds__(VT) void vd_solve_kernel(VdArgs a) {
 // first being `first`.  SOLAR: the buoyancy rows with a solar flux, whose two
 // exponentials an interface cost the other systems no registers this way.
 // Bound by memory latency at two waves per SIMD (three arrays of 32 doubles are
-// 192 // 192 registers).  J8 L30: 1.63 -> 0.70 ms; with the arrays in LDS (three waves
+// 192 registers).  J8 L30: 1.63 -> 0.70 ms; with the arrays in LDS (three waves
 // per compute unit) 1.6 ms.
 template <int LM, bool SOLAR>
 __global__ __launch_bounds__(VT, LM > 16 ? 2 : 3) void vd_solve_reg_kernel(VdArgs a, int ncb, int first, int count) {
