@@ -211,8 +211,8 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
-            "traffic": measured_traffic(J, L),
-            "kernel": "trisk_stage_kernel",
+            "traffic": measured_traffic(J, L, "trisk_stage", "trisk_stage_tile_kernel"),
+            "kernel": "trisk_stage_tile_kernel",
             "kernel_ms": kernel_ms,
             "algorithmic_bytes_per_launch": alg_bytes,
         },
@@ -228,14 +228,17 @@ def main():
     print(json.dumps(out))
 
 
-def measured_traffic(J: int, L: int, kernel: str = "trisk_stage"):
-    """HBM bytes per launch of the stage kernel from the committed rocprofv3
-    counter summary of this workload (FETCH_SIZE + WRITE_SIZE per dispatch,
-    scaled by a plain copy's readings), or None if it is absent."""
-    path = os.path.join(ROOT, "profiles", f"{kernel}_J{J}_L{L}_hbm.txt")
+def measured_traffic(J: int, L: int, summary: str, kernel: str):
+    """HBM bytes per launch of `kernel` from the committed rocprofv3 counter
+    summary of this workload (FETCH_SIZE + WRITE_SIZE per dispatch, scaled by
+    a plain copy's readings), or None if it is absent or of another kernel."""
+    path = os.path.join(ROOT, "profiles", f"{summary}_J{J}_L{L}_hbm.txt")
     if not os.path.exists(path):
         return None
-    for line in open(path):
+    text = open(path).read()
+    if kernel not in text:
+        return None
+    for line in text.splitlines():
         if line.startswith("traffic_bytes_per_launch:"):
             return float(line.split(":", 1)[1])
     return None
@@ -280,7 +283,7 @@ def fp32_bulk(grid, topo, mass, temp, velo, L, dt, warmup, steps, m64, u64, dof_
             "stage_kernel_ms": kernel_ms,
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": achieved / HBM_PEAK_GBS,
-                         "traffic": measured_traffic(lay.level, L, "trisk_stage_mixed"),
+                         "traffic": measured_traffic(lay.level, L, "trisk_stage_mixed", "trisk_stage_mixed_kernel"),
                          "kernel": "trisk_stage_mixed_kernel", "algorithmic_bytes_per_launch": alg},
             "stage_shape": shape,
             "drift_vs_fp64": {"steps": warmup + steps,

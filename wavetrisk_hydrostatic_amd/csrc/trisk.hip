@@ -803,8 +803,8 @@ __global__ __launch_bounds__(THREADS2, 2) void trisk_stage_kernel2(StageArgs a_i
 //      since A).
 // A block spans the layers [k0, k0 + kchunk): the column scan takes the
 // layers below it first, with a single sweep's operations in the same order.
-// What bounds it at J8 L30: HBM latency and bandwidth together, 2.5 GB a
-// launch at 3.7 TB/s (a large copy reaches 4.7), and the registers: one
+// What bounds it at J8 L30: HBM latency and bandwidth together, 2.7 GB a
+// launch at 3.9 TB/s (a large copy reaches 4.7), and the registers: one
 // spilled value in the loop waits for the next layer's loads (677 -> 727 us).
 // Two independent blocks overlap each other's barriers; the earlier kernel
 // (two layers in lock step in one 768-thread block, the geometry in LDS)
