@@ -110,8 +110,8 @@ __device__ __forceinline__ double ell_diag_at(const FsGeo& g, const double* __re
 
 __global__ void fs_apply_kernel(const double* __restrict__ gate, int n, const int64_t* __restrict__ ncl, FsGeo g,
                                 const double* __restrict__ q, const double* __restrict__ eo, double grav, double coef,
-                                double* __restrict__ out, double* __restrict__ out2, int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                double* __restrict__ out, double* __restrict__ out2, int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), q = mem(q, ms), eo = mem(eo, ms), out = mem(out, ms), out2 = mem(out2, ms);
@@ -125,8 +125,8 @@ __global__ void fs_apply_kernel(const double* __restrict__ gate, int n, const in
 __global__ void fs_bicg_init_kernel(int n, const int64_t* __restrict__ ncl, FsGeo g, double* __restrict__ u,
                                     const double* __restrict__ f, const double* __restrict__ eo, double grav,
                                     double coef, int zero_u, double* __restrict__ res, double* __restrict__ res0,
-                                    double* __restrict__ p, double* __restrict__ s, int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                    double* __restrict__ p, double* __restrict__ s, int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms);
   res = mem(res, ms), res0 = mem(res0, ms), p = mem(p, ms), s = mem(s, ms);
@@ -154,8 +154,8 @@ template <class F, bool Zero = false>
 __global__ void fs_jacobi_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl, FsGeo g,
                                  const F* __restrict__ u, const F* __restrict__ f, const double* __restrict__ eo,
                                  double grav, double coef, double dt2, double th12, double w, F* __restrict__ out,
-                                 int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                 int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms), out = mem(out, ms);
   const int64_t c = ncl[2 * t + 1];
@@ -177,8 +177,8 @@ template <class Fu, class Ff, class Fo>
 __global__ void fs_residual_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl, FsGeo g,
                                    const Fu* __restrict__ u, const Ff* __restrict__ f,
                                    const double* __restrict__ eo, double grav, double coef, Fo* __restrict__ out,
-                                   int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                   int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   g.topo = mem(g.topo, ms), u = mem(u, ms), f = mem(f, ms), eo = mem(eo, ms), out = mem(out, ms);
   const int64_t c = ncl[2 * t + 1];
@@ -247,9 +247,9 @@ __device__ __forceinline__ double vflux(const FsGeo& g, int L, const double* __r
 // in the order of div (ops.f90:1325-1343).
 __global__ void fs_edge_flux_kernel(int nlz, FsGeo g, int L, const double* __restrict__ m,
                                     const double* __restrict__ u, double* __restrict__ F0, double* __restrict__ F1,
-                                    double* __restrict__ F2) {
+                                    double* __restrict__ F2, int per) {
   const int w = nlz + 2;  // cells per row and rows per lozenge in the pass
-  const int64_t t = (int64_t)list_block() * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)list_block(per) * blockDim.x + threadIdx.x;
   if (t >= (int64_t)10 * w * w) return;
   const int lz = (int)(t / ((int64_t)w * w)), r = (int)(t % ((int64_t)w * w));
   const int i = r % w - 1, j = r / w - 1;
@@ -261,8 +261,8 @@ __global__ void fs_edge_flux_kernel(int nlz, FsGeo g, int L, const double* __res
 
 __global__ void fs_div_kernel(int n, const int64_t* __restrict__ ncl, FsGeo g, const double* __restrict__ F0,
                               const double* __restrict__ F1, const double* __restrict__ F2,
-                              double* __restrict__ out) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                              double* __restrict__ out, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t c = ncl[2 * t + 1];
   const int64_t cW = c - 1, cSW = c - g.S - 1, cS = c - g.S;
@@ -541,8 +541,8 @@ __global__ void fs_bicg_s_apply_kernel(const double* __restrict__ gate, int n, c
                                        FsGeo g, const double* __restrict__ res, const double* __restrict__ Ap,
                                        const double* __restrict__ eo, double grav, double coef,
                                        const double* __restrict__ scal, double* __restrict__ s_out,
-                                       double* __restrict__ As_out, int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                       double* __restrict__ As_out, int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), res = mem(res, ms), Ap = mem(Ap, ms), eo = mem(eo, ms);
@@ -562,8 +562,8 @@ __global__ void fs_bicg_p_apply_kernel(const double* __restrict__ gate, int n, c
                                        FsGeo g, const double* __restrict__ res, const double* __restrict__ p,
                                        const double* __restrict__ Ap, const double* __restrict__ eo, double grav,
                                        double coef, const double* __restrict__ scal, double* __restrict__ pn_out,
-                                       double* __restrict__ Apn_out, int64_t ms) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                       double* __restrict__ Apn_out, int64_t ms, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   gate = mem(gate, SC_NSCAL);
   if (t >= n || gated(gate)) return;
   g.topo = mem(g.topo, ms), res = mem(res, ms), p = mem(p, ms), Ap = mem(Ap, ms), eo = mem(eo, ms);
@@ -1242,8 +1242,8 @@ __global__ __launch_bounds__(NT, NT > SW_SMALL ? 3 : 4) void fs_sweeps_kernel(Sw
 // wc = s - Interp_node at midpoints, 0 at coincident nodes
 template <class F>
 __global__ void mg_wavelet_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl, MgGeo g,
-                                  const F* __restrict__ s, F* __restrict__ wc) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                  const F* __restrict__ s, F* __restrict__ wc, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   s = mem(s, g.NCf), wc = mem(wc, g.NCf);
   const int64_t x = ncl[2 * t + 1];
@@ -1286,8 +1286,8 @@ __global__ void mg_restrict_ss_kernel(int n, const int64_t* __restrict__ ncl, Mg
 template <class F, bool ZeroW = false>
 __global__ void mg_prolong_even_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl,
                                        MgGeo g, const F* __restrict__ sc, const F* __restrict__ wc,
-                                       F* __restrict__ sf) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                       F* __restrict__ sf, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   sc = mem(sc, g.NCc), wc = mem(wc, g.NCf), sf = mem(sf, g.NCf);
   const int64_t x = ncl[2 * t + 1];
@@ -1309,8 +1309,8 @@ __global__ void mg_prolong_even_kernel(const double* __restrict__ mdone, int n, 
 // cells and writes only midpoints, so it runs in place after the even pass.
 template <class F, bool ZeroW = false>
 __global__ void mg_prolong_odd_kernel(const double* __restrict__ mdone, int n, const int64_t* __restrict__ ncl,
-                                      MgGeo g, const F* __restrict__ wc, F* __restrict__ sf) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                      MgGeo g, const F* __restrict__ wc, F* __restrict__ sf, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n || mdone_of(mdone)) return;
   wc = mem(wc, g.NCf), sf = mem(sf, g.NCf);
   const int64_t x = ncl[2 * t + 1];
@@ -1539,7 +1539,7 @@ double fs_coef(const wtg_ctx* c) { return c->fs_theta1 * c->fs_theta2 * (c->fs_d
 int launch_apply(wtg_ctx* c, const double* q, double* out, bool gate = false, double* out2 = nullptr) {
   hipLaunchKernelGGL(fs_apply_kernel, dim3(nblk(c->nncl), c->nmembers), dim3(FS_NT), 0, c->stream,
                      gate ? c->d_scal : nullptr, c->nncl, c->d_ncl, fs_geo(c), q, c->fs[FS_ETA_OLD], c->params.grav,
-                     fs_coef(c), out, out2, c->info.ncells);
+                     fs_coef(c), out, out2, c->info.ncells, xcd_rows(nblk(c->nncl), c->nmembers));
   WTG_HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -1548,7 +1548,7 @@ template <class Fu, class Ff, class Fo>
 int launch_residual(wtg_ctx* c, const Fu* u, const Ff* f, Fo* out) {
   hipLaunchKernelGGL((fs_residual_kernel<Fu, Ff, Fo>), dim3(nblk(c->nncl), c->nmembers), dim3(FS_NT), 0, c->stream,
                      c->mg_mdone, c->nncl, c->d_ncl, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c),
-                     out, c->info.ncells);
+                     out, c->info.ncells, xcd_rows(nblk(c->nncl), c->nmembers));
   WTG_HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -1557,7 +1557,8 @@ template <class F, bool Zero = false>
 int launch_jacobi(wtg_ctx* c, const F* u, const F* f, double w, F* out) {
   hipLaunchKernelGGL((fs_jacobi_kernel<F, Zero>), dim3(nblk(c->nncl), c->nmembers), dim3(FS_NT), 0, c->stream,
                      c->mg_mdone, c->nncl, c->d_ncl, fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c),
-                     c->fs_dt * c->fs_dt, c->fs_theta1 * c->fs_theta2, w, out, c->info.ncells);
+                     c->fs_dt * c->fs_dt, c->fs_theta1 * c->fs_theta2, w, out, c->info.ncells,
+                     xcd_rows(nblk(c->nncl), c->nmembers));
   WTG_HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -1735,7 +1736,7 @@ int bicgstab(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int*
   const int64_t ms = c->info.ncells;
   hipLaunchKernelGGL(fs_bicg_init_kernel, dim3(nblk(c->nncl), M), dim3(FS_NT), 0, c->stream, c->nncl, c->d_ncl,
                      fs_geo(c), u, f, c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c), zero_u ? 1 : 0, res, res0, p,
-                     s, ms);
+                     s, ms, xcd_rows(nblk(c->nncl), M));
   WTG_HIPCHK(c, hipGetLastError());
   RC(launch_apply(c, p, Ap, false, As));  // Ap = As = L p
   RC(launch_dots(c, 1, res0, res, SC_RHO));
@@ -1756,7 +1757,7 @@ int bicgstab(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int*
       RC(launch_dots_g(c, true, OP_ALPH, 1, Ap, res0, SC_T0));
       hipLaunchKernelGGL(fs_bicg_s_apply_kernel, dim3(nblk(c->nncl), M), dim3(FS_NT), 0, c->stream, c->d_scal,
                          c->nncl, c->d_ncl, fs_geo(c), res, Ap, c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c),
-                         c->d_scal, s, As, ms);  // s = res - alph Ap; As = L s
+                         c->d_scal, s, As, ms, xcd_rows(nblk(c->nncl), M));  // s = res - alph Ap; As = L s
       WTG_HIPCHK(c, hipGetLastError());
       RC(launch_dots_g(c, true, OP_OMGA, 2, As, s, SC_T1, As, As, SC_T2));
       const bool last = nbred <= c->lastblock_max && M == 1;
@@ -1772,7 +1773,8 @@ int bicgstab(wtg_ctx* c, double* u, const double* f, double tol, int maxit, int*
       }
       hipLaunchKernelGGL(fs_bicg_p_apply_kernel, dim3(nblk(c->nncl), M), dim3(FS_NT), 0, c->stream, c->d_scal,
                          c->nncl, c->d_ncl, fs_geo(c), res, p, Ap, c->fs[FS_ETA_OLD], c->params.grav, fs_coef(c),
-                         c->d_scal, p_alt, Ap_alt, ms);  // p = res + b (p - omga Ap); Ap = L p
+                         c->d_scal, p_alt, Ap_alt, ms,
+                         xcd_rows(nblk(c->nncl), M));  // p = res + b (p - omga Ap); Ap = L p
       WTG_HIPCHK(c, hipGetLastError());
       std::swap(p, p_alt);
       std::swap(Ap, Ap_alt);
@@ -1966,7 +1968,7 @@ int mg_forward(wtg_mg* m, int l, const F* s, F* wc, F* s_c) {
   wtg_ctx *f = m->lv[l], *c = m->lv[l - 1];
   const MgGeo g = mg_geo(m, l);
   hipLaunchKernelGGL(mg_wavelet_kernel<F>, dim3(nblk(f->nncl), f->nmembers), dim3(FS_NT), 0, f->stream, f->mg_mdone,
-                     f->nncl, f->d_ncl, g, s, wc);
+                     f->nncl, f->d_ncl, g, s, wc, xcd_rows(nblk(f->nncl), f->nmembers));
   WTG_HIPCHK(f, hipGetLastError());
   hipLaunchKernelGGL(mg_restrict_kernel<F>, dim3(nblk(c->nncl), f->nmembers), dim3(FS_NT), 0, f->stream, f->mg_mdone,
                      c->nncl, c->d_ncl, g, s, wc, s_c);
@@ -1981,10 +1983,10 @@ int mg_inverse(wtg_mg* m, int l, const F* s_c, const F* wc, F* s_f) {
   wtg_ctx* f = m->lv[l];
   const MgGeo g = mg_geo(m, l);
   hipLaunchKernelGGL((mg_prolong_even_kernel<F, ZeroW>), dim3(nblk(f->nncl), f->nmembers), dim3(FS_NT), 0, f->stream,
-                     f->mg_mdone, f->nncl, f->d_ncl, g, s_c, wc, s_f);
+                     f->mg_mdone, f->nncl, f->d_ncl, g, s_c, wc, s_f, xcd_rows(nblk(f->nncl), f->nmembers));
   WTG_HIPCHK(f, hipGetLastError());
   hipLaunchKernelGGL((mg_prolong_odd_kernel<F, ZeroW>), dim3(nblk(f->nncl), f->nmembers), dim3(FS_NT), 0, f->stream,
-                     f->mg_mdone, f->nncl, f->d_ncl, g, wc, s_f);
+                     f->mg_mdone, f->nncl, f->d_ncl, g, wc, s_f, xcd_rows(nblk(f->nncl), f->nmembers));
   WTG_HIPCHK(f, hipGetLastError());
   return 0;
 }
@@ -2584,10 +2586,11 @@ int wtg_fs_flux_div_async(wtg_ctx* c, int slot) {
   double *F0 = c->fs[FS_W0], *F1 = c->fs[FS_W0 + 1], *F2 = c->fs[FS_W0 + 2];
   const int64_t ne = (int64_t)10 * (c->info.n + 2) * (c->info.n + 2);
   hipLaunchKernelGGL(fs_edge_flux_kernel, dim3((unsigned)((ne + FS_NT - 1) / FS_NT)), dim3(FS_NT), 0, c->stream,
-                     c->info.n, fs_geo(c), c->params.nlayers, s.m, s.u, F0, F1, F2);
+                     c->info.n, fs_geo(c), c->params.nlayers, s.m, s.u, F0, F1, F2,
+                     xcd_rows((unsigned)((ne + FS_NT - 1) / FS_NT), c->params.nlayers));
   WTG_HIPCHK(c, hipGetLastError());
   hipLaunchKernelGGL(fs_div_kernel, dim3(nblk(c->nncl)), dim3(FS_NT), 0, c->stream, c->nncl, c->d_ncl, fs_geo(c), F0,
-                     F1, F2, c->fs[FS_DIVF]);
+                     F1, F2, c->fs[FS_DIVF], xcd_rows(nblk(c->nncl), 1));
   WTG_HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -2608,10 +2611,11 @@ int wtg_fs_flux_div_into(wtg_ctx* c, int slot, double* flux3, double* divf) {
   const int64_t NC = c->info.ncells;
   const int64_t ne = (int64_t)10 * (c->info.n + 2) * (c->info.n + 2);
   hipLaunchKernelGGL(fs_edge_flux_kernel, dim3((unsigned)((ne + FS_NT - 1) / FS_NT)), dim3(FS_NT), 0, c->stream,
-                     c->info.n, fs_geo(c), c->params.nlayers, s.m, s.u, flux3, flux3 + NC, flux3 + 2 * NC);
+                     c->info.n, fs_geo(c), c->params.nlayers, s.m, s.u, flux3, flux3 + NC, flux3 + 2 * NC,
+                     xcd_rows((unsigned)((ne + FS_NT - 1) / FS_NT), c->params.nlayers));
   WTG_HIPCHK(c, hipGetLastError());
   hipLaunchKernelGGL(fs_div_kernel, dim3(nblk(c->nncl)), dim3(FS_NT), 0, c->stream, c->nncl, c->d_ncl, fs_geo(c), flux3,
-                     flux3 + NC, flux3 + 2 * NC, divf);
+                     flux3 + NC, flux3 + 2 * NC, divf, xcd_rows(nblk(c->nncl), 1));
   WTG_HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -2628,7 +2632,8 @@ int wtg_mg_eta_transform(wtg_mg* m) {
     wtg_ctx* f = m->lv[l];
     const MgGeo g = mg_geo(m, l);
     hipLaunchKernelGGL(mg_wavelet_kernel<double>, dim3(nblk(f->nncl), f->nmembers), dim3(FS_NT), 0, f->stream,
-                       (const double*)nullptr, f->nncl, f->d_ncl, g, (const double*)f->fs[FS_ETA], f->fs[MG_WC]);
+                       (const double*)nullptr, f->nncl, f->d_ncl, g, (const double*)f->fs[FS_ETA], f->fs[MG_WC],
+                       xcd_rows(nblk(f->nncl), f->nmembers));
     WTG_HIPCHK(f, hipGetLastError());
   }
   for (int l = 1; l < m->nl; ++l)

@@ -77,6 +77,7 @@ struct PairGeo {
   const double* rf;             // [24][NCc]
   const int64_t* wide;          // fine level's lattice map, frame [-WH, nf+WH)
   int WH;
+  int per;  // list_block's rows over the parents
 };
 
 __device__ __forceinline__ int64_t cellc(const PairGeo& g, int lz, int i, int j) {
@@ -100,8 +101,8 @@ constexpr int ML_KCV = 1;
 
 __global__ void ml_scalar_wavelet_kernel(int n, const int64_t* __restrict__ ncl, MgGeo g, int L,
                                          const double* __restrict__ sm, const double* __restrict__ st,
-                                         double* __restrict__ wc) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                         double* __restrict__ wc, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -117,8 +118,8 @@ __global__ void ml_scalar_wavelet_kernel(int n, const int64_t* __restrict__ ncl,
 __global__ void ml_restrict_scalar_kernel(int n, const int64_t* __restrict__ ncl, MgGeo g, int L,
                                           const double* __restrict__ fm, const double* __restrict__ ft,
                                           const double* __restrict__ wc, double* __restrict__ cm,
-                                          double* __restrict__ ct, int64_t NCc) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                          double* __restrict__ ct, int64_t NCc, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t p = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -161,8 +162,8 @@ __global__ void ml_prolong_even_kernel(int n, const int64_t* __restrict__ ncl, M
 
 __global__ void ml_prolong_odd_kernel(int n, const int64_t* __restrict__ ncl, MgGeo g, int L,
                                       const double* __restrict__ wc, double* __restrict__ fm,
-                                      double* __restrict__ ft) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                      double* __restrict__ ft, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int64_t x = ncl[2 * t + 1], dst = ncl[2 * t];
   int lz, i, j;
@@ -248,7 +249,7 @@ __device__ __forceinline__ void interp_inner(const PairGeo& g, const double* __r
 
 __device__ __forceinline__ bool parent_of(const PairGeo& g, int& lz, int& ip, int& jp, int& k, int L) {
   const int64_t per = (int64_t)10 * g.nc * g.nc;
-  const int64_t t = (int64_t)list_block() * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)list_block(g.per) * blockDim.x + threadIdx.x;
   if (t >= per) return false;
   k = blockIdx.y;
   lz = (int)(t / ((int64_t)g.nc * g.nc));
@@ -715,8 +716,8 @@ __global__ void ml_coarse_scalar_kernel(int n, int nmaster, const int64_t* __res
                                         const double* __restrict__ hinv, const double* __restrict__ hcl,
                                         double* __restrict__ dsl, const double* __restrict__ qm,
                                         const double* __restrict__ qt, double* __restrict__ om,
-                                        double* __restrict__ ot, double h, int trend_only, int plus_div) {
-  const int t = list_block() * blockDim.x + threadIdx.x;
+                                        double* __restrict__ ot, double h, int trend_only, int plus_div, int per) {
+  const int t = list_block(per) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const int y = blockIdx.y, k = y % L;
   const double* hf = hcl + (int64_t)y * 3 * NC;
@@ -844,6 +845,7 @@ PairGeo pgeo(const wtg_ml* m, int l) {
   g.rf = m->rf[l - 1];
   g.wide = m->wide[l];
   g.WH = m->WH;
+  g.per = xcd_rows(nblk((int64_t)10 * g.nc * g.nc), 2 * m->L);
   return g;
 }
 
@@ -868,7 +870,7 @@ int wavelets(wtg_ml* m, int l, const wtg_ctx::Slot& fine, const wtg_ctx::Slot& c
   const int L = m->L;
   const MgGeo g = mgeo(m, l);
   hipLaunchKernelGGL(ml_scalar_wavelet_kernel, dim3(nblk(f->nncl), ml_chunks(2 * L)), dim3(NT), 0, mstream(m), f->nncl, f->d_ncl,
-                     g, L, fine.m, fine.t, m->wcs[l]);
+                     g, L, fine.m, fine.t, m->wcs[l], xcd_rows(nblk(f->nncl), 2 * L));
   MLCHK(m, hipGetLastError());
   const PairGeo pg = pgeo(m, l);
   hipLaunchKernelGGL(ml_velo_wavelet_kernel, velo_grid(pg.nc, L), dim3(NT), 0,
@@ -889,7 +891,7 @@ int inverse(wtg_ml* m, int l, const wtg_ctx::Slot& fine, const wtg_ctx::Slot& co
                      L, coarse.m, coarse.t, c->info.ncells, m->wcs[l], fine.m, fine.t);
   MLCHK(m, hipGetLastError());
   hipLaunchKernelGGL(ml_prolong_odd_kernel, dim3(nblk(f->nncl), ml_chunks(2 * L)), dim3(NT), 0, mstream(m), f->nncl, f->d_ncl, g,
-                     L, m->wcs[l], fine.m, fine.t);
+                     L, m->wcs[l], fine.m, fine.t, xcd_rows(nblk(f->nncl), 2 * L));
   MLCHK(m, hipGetLastError());
   const PairGeo pg = pgeo(m, l);
   const dim3 pgrid = velo_grid(pg.nc, L);
@@ -949,7 +951,7 @@ int stage(wtg_ml* m, const std::vector<const wtg_ctx::Slot*>& y, const std::vect
     const int64_t NC = c->info.ncells;
     hipLaunchKernelGGL(ml_coarse_scalar_kernel, dim3(nblk(c->nncl), 2 * L), dim3(NT), 0, mstream(m), c->nncl,
                        c->nmaster, c->d_ncl, c->info.S, NC, L, c->d_hinv, m->hflux[l], m->dsc[l], q[l]->m, q[l]->t,
-                       out[l]->m, out[l]->t, h, trend_only, 0);
+                       out[l]->m, out[l]->t, h, trend_only, 0, xcd_rows(nblk(c->nncl), 2 * L));
     MLCHK(m, hipGetLastError());
     hipLaunchKernelGGL(ml_coarse_velo_kernel, dim3(nblk((int64_t)10 * pg.nc * pg.nc), L), dim3(NT), 0, mstream(m), pg, L,
                        1 << (top - l), ft->info.S, NT_, m->bern, m->exn, m->src[l + 1], m->src[l], y[l]->m, y[l]->t,
@@ -1086,10 +1088,11 @@ int wtg_ml_forward(wtg_ml* m, int slot) {
     if (int rc = wtg_ghost_fill_layers(f, L, s[l]->m, s[l]->t, nullptr)) return rc;
     const MgGeo g = mgeo(m, l);
     hipLaunchKernelGGL(ml_scalar_wavelet_kernel, dim3(nblk(f->nncl), ml_chunks(2 * L)), dim3(NT), 0, mstream(m), f->nncl,
-                       f->d_ncl, g, L, s[l]->m, s[l]->t, m->wcs[l]);
+                       f->d_ncl, g, L, s[l]->m, s[l]->t, m->wcs[l], xcd_rows(nblk(f->nncl), 2 * L));
     MLCHK(m, hipGetLastError());
     hipLaunchKernelGGL(ml_restrict_scalar_kernel, dim3(nblk(c->nncl), ml_chunks(2 * L)), dim3(NT), 0, mstream(m), c->nncl,
-                       c->d_ncl, g, L, s[l]->m, s[l]->t, m->wcs[l], s[l - 1]->m, s[l - 1]->t, c->info.ncells);
+                       c->d_ncl, g, L, s[l]->m, s[l]->t, m->wcs[l], s[l - 1]->m, s[l - 1]->t, c->info.ncells,
+                       xcd_rows(nblk(c->nncl), 2 * L));
     MLCHK(m, hipGetLastError());
     if (int rc = wtg_restrict_velo(f, slot, c, slot)) return rc;
   }
@@ -1195,7 +1198,8 @@ int flux_divergence_ml(wtg_ml* m, int slot, int out) {
     if (int rc = wtg_ghost_fill_layers(c, 1, nullptr, nullptr, m->hflux[l])) return rc;
     hipLaunchKernelGGL(ml_coarse_scalar_kernel, dim3(nblk(c->nncl), 1), dim3(NT), 0, mstream(m), c->nncl, c->nmaster,
                        c->d_ncl, c->info.S, c->info.ncells, 1, c->d_hinv, m->hflux[l], c->fs[out],
-                       (const double*)nullptr, (const double*)nullptr, (double*)nullptr, (double*)nullptr, 0.0, 1, 1);
+                       (const double*)nullptr, (const double*)nullptr, (double*)nullptr, (double*)nullptr, 0.0, 1, 1,
+                       xcd_rows(nblk(c->nncl), 1));
     MLCHK(m, hipGetLastError());
   }
   return 0;
