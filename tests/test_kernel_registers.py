@@ -45,7 +45,8 @@ def registers(tmp_path_factory):
     return out
 
 
-# the counts of the code whose times are noted beside the kernels: (HasD, output, edge tasks) of the layer-pair forms, (HasD, output) of the one-layer form
+# the counts of the code whose times are noted beside the kernels:
+# (HasD, output, edge tasks) of the layer-pair forms, (HasD, output) of the one-layer form
 @pytest.mark.parametrize("kernel,args,vgprs,spills", [
     ("trisk_stage_mixed_kernel", ("0", "f", "0"), 115, 0), ("trisk_stage_mixed_kernel", ("1", "f", "0"), 124, 0),
     ("trisk_stage_mixed_kernel", ("1", "d", "0"), 143, 0), ("trisk_stage_mixed_kernel", ("0", "f", "1"), 126, 0),
